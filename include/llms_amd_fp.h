@@ -63,7 +63,8 @@ const char* fp_status_string(int status);
 
 /* ABI version of this library: (major << 16) | minor. Minor 5 adds
  * fp_rmsnorm_qkv_bf16_noalloc and FP_ERR_SCRATCH, and sizes
- * fp_rmsnorm_workspace_bytes for the normalised rows of every call. */
+ * fp_rmsnorm_workspace_bytes for the normalised rows of every call. Minor 6
+ * adds fp_attention_bf16. */
 int fp_abi_version(void);
 
 /*
@@ -278,6 +279,48 @@ int fp_rmsnorm_qkv_bf16_noalloc(const void* x, int64_t ldx, const void* gamma, f
                                 void* y, int64_t ldy,
                                 int64_t M, int64_t n_q, int64_t n_k, int64_t K,
                                 void* stream);
+
+/*
+ * The attention layer between its two projections (reference:
+ * src/kernels/fused_qkv.py:242-282): RMS-norm of every q and k head, rotate-half
+ * RoPE, the write of k and v into the layer's cache at positions pos .. pos+T-1
+ * and causal softmax attention (scale D^-0.5, key position <= query position)
+ * of the T tokens over the cache, grouped-query heads sharing their kv head.
+ *   q, k, v    rows m = b*T + t of n_heads / n_kv_heads heads of head_dim, bf16
+ *   q_gamma, k_gamma  [head_dim] bf16, both NULL: q and k are normalised already
+ *   cos, sin   [T, head_dim] bf16 (the two halves share frequencies)
+ *   cache_k/v  element (b, head, position, d) at b*s_b + head*s_h + position*s_p + d
+ *   y          [B*T, n_heads*head_dim] bf16, contiguous
+ * pos_dev, when not NULL, is one int64 on the device that replaces pos (a call
+ * captured in a HIP graph replays at any position); positions outside the cache
+ * are then neither written nor attended (with pos, FP_ERR_SHAPE).
+ * Rounding: bf16 where the unfused torch path rounds (norm, norm weight, RoPE
+ * products and sum, output); scores, softmax and p.V in fp32.
+ * head_dim is 64 or 128; n_heads a multiple of n_kv_heads. q, k, v and the gammas
+ * are 8-byte aligned with row strides that are multiples of 4, the caches
+ * 16-byte aligned with strides that are multiples of 8, one head's cache (64
+ * positions more than cache_len) under 2^31 bytes. workspace: at least
+ * fp_attention_workspace_bytes(..., keys) with keys = pos + T, or cache_len with
+ * pos_dev; 16-byte aligned; written in full before it is read.
+ */
+typedef struct fp_attention_args {
+  const void *q, *k, *v;
+  int64_t ldq, ldk, ldv;
+  const void *q_gamma, *k_gamma;
+  const void *cos, *sin;
+  int64_t ld_cos, ld_sin;
+  void *cache_k, *cache_v;
+  int64_t k_s_b, k_s_h, k_s_p, v_s_b, v_s_h, v_s_p;
+  void* y;
+  int64_t B, T, n_heads, n_kv_heads, head_dim, cache_len, pos;
+  const int64_t* pos_dev;
+  float q_eps, k_eps;
+} fp_attention_args;
+
+int64_t fp_attention_workspace_bytes(int64_t B, int64_t T, int64_t n_heads, int64_t n_kv_heads,
+                                     int64_t head_dim, int64_t keys);
+int fp_attention_bf16(const fp_attention_args* args, void* workspace, int64_t workspace_bytes,
+                      void* stream);
 
 /*
  * Per-output-channel symmetric int8 quantisation on the device (the packing

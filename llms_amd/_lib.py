@@ -55,6 +55,8 @@ CAPI_SIGNATURES: dict[str, list] = {
     "fp_rmsnorm_qkv_w8": [_P, _I64, _P, _F, _P, _I64, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _I64, _P],
     "fp_rmsnorm_gate_up_silu_w8": [_P, _I64, _P, _F, _P, _I64, _P, _P, _I64, _P, _P, _I64, _I64, _I64,
                                    _I64, _P, _I64, _P],
+    "fp_attention_workspace_bytes": [_I64, _I64, _I64, _I64, _I64, _I64],
+    "fp_attention_bf16": [_P, _P, _I64, _P],
     "fp_rmsnorm_qkv_bf16_noalloc": [_P, _I64, _P, _F, _P, _I64, _P, _I64, _I64, _I64, _I64, _I64, _P],
 }
 
@@ -95,7 +97,8 @@ def capi() -> ctypes.CDLL:
                 fn.restype = {"fp_status_string": ctypes.c_char_p,
                               "fp_workspace_bytes": ctypes.c_int64,
                               "fp_workspace_bytes_w8": ctypes.c_int64,
-                              "fp_rmsnorm_workspace_bytes": ctypes.c_int64}.get(name, ctypes.c_int)
+                              "fp_rmsnorm_workspace_bytes": ctypes.c_int64,
+                              "fp_attention_workspace_bytes": ctypes.c_int64}.get(name, ctypes.c_int)
             _capi = lib
         return _capi
 

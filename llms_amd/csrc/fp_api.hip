@@ -139,6 +139,17 @@ int check_common(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy) {
   return FP_OK;
 }
 
+// B, T, heads and head size of an attention call: sizes that keep every grid
+// dimension and row index within 32 bits.
+int check_attention(int64_t B, int64_t T, int64_t Hq, int64_t Hk, int64_t D) {
+  if (B < 1 || T < 1 || Hk < 1 || Hq < Hk || Hq % Hk != 0 || (D != 64 && D != 128))
+    return FP_ERR_SHAPE;
+  if (B > 65535 || Hq > 65535 || B * Hk > 65535 || T > (int64_t)1 << 24 ||
+      T * (Hq / Hk) > (int64_t)1 << 30 || B * T * (Hq + 2 * Hk) > (int64_t)1 << 31)
+    return FP_ERR_SHAPE;
+  return FP_OK;
+}
+
 }  // namespace
 
 int rmsnorm_qkv_args(const void* x, int64_t ldx, const void* gamma, float eps, const void* w,
@@ -173,7 +184,7 @@ const char* fp_status_string(int status) {
   }
 }
 
-int fp_abi_version(void) { return (1 << 16) | 5; }
+int fp_abi_version(void) { return (1 << 16) | 6; }
 
 int64_t fp_workspace_bytes(int64_t M, int64_t N, int64_t K, int gate_up) {
   if (M < 1 || N < 1 || K < 1) return 0;
@@ -385,6 +396,58 @@ int fp_rmsnorm_gate_up_silu_w8(const void* x, int64_t ldx, const void* gamma, fl
   const bool xal = K % 16 == 0 && ldx % 8 == 0 && fp::al16(x);
   const bool wal = ldqg % 16 == 0 && ldqu % 16 == 0 && fp::al16(qg) && fp::al16(qu);
   return fp::run_norm<true, true>(a, xal, wal, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int64_t fp_attention_workspace_bytes(int64_t B, int64_t T, int64_t n_heads, int64_t n_kv_heads,
+                                     int64_t head_dim, int64_t keys) {
+  if (fp::check_attention(B, T, n_heads, n_kv_heads, head_dim) || keys < 1) return 0;
+  return fp::attn_workspace_bytes(B, T, n_heads, n_kv_heads, head_dim, keys);
+}
+
+int fp_attention_bf16(const fp_attention_args* g, void* workspace, int64_t workspace_bytes,
+                      void* stream) {
+  if (!g) return FP_ERR_NULL;
+  const int64_t D = g->head_dim, S = g->cache_len, T = g->T;
+  int st = fp::check_attention(g->B, T, g->n_heads, g->n_kv_heads, D);
+  if (st) return st;
+  if (S < 1 || S > (int64_t)1 << 30) return FP_ERR_SHAPE;
+  if (!g->pos_dev && (g->pos < 0 || g->pos + T > S)) return FP_ERR_SHAPE;
+  if (!(g->q_eps >= 0.f) || !(g->k_eps >= 0.f)) return FP_ERR_SHAPE;
+  if (g->ldq < g->n_heads * D || g->ldk < g->n_kv_heads * D || g->ldv < g->n_kv_heads * D ||
+      g->ld_cos < D || g->ld_sin < D || g->k_s_p < D || g->v_s_p < D || g->k_s_b < 0 ||
+      g->k_s_h < 0 || g->v_s_b < 0 || g->v_s_h < 0)
+    return FP_ERR_STRIDE;
+  const int64_t any4 = g->ldq | g->ldk | g->ldv;
+  const int64_t any8 = g->k_s_b | g->k_s_h | g->k_s_p | g->v_s_b | g->v_s_h | g->v_s_p;
+  if ((any4 & 3) || (any8 & 7)) return FP_ERR_STRIDE;
+  constexpr int64_t kLim = (int64_t)1 << 31;
+  if ((S + 64) * g->k_s_p * 2 >= kLim || (S + 64) * g->v_s_p * 2 >= kLim) return FP_ERR_SHAPE;
+  if (!g->q || !g->k || !g->v || !g->cos || !g->sin || !g->cache_k || !g->cache_v || !g->y)
+    return FP_ERR_NULL;
+  if (!g->q_gamma != !g->k_gamma) return FP_ERR_NULL;
+  const auto al8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0; };
+  if (!al8(g->q) || !al8(g->k) || !al8(g->v) || !al8(g->q_gamma) || !al8(g->k_gamma) ||
+      !al8(g->y) || !fp::al16(g->cache_k) || !fp::al16(g->cache_v))
+    return FP_ERR_STRIDE;
+  const int64_t keys = g->pos_dev ? S : g->pos + T;
+  if (!workspace || !fp::al16(workspace) ||
+      workspace_bytes < fp::attn_workspace_bytes(g->B, T, g->n_heads, g->n_kv_heads, D, keys))
+    return FP_ERR_WORKSPACE;
+  fp::AttnArgs a{};
+  a.q = (const uint16_t*)g->q, a.k = (const uint16_t*)g->k, a.v = (const uint16_t*)g->v;
+  a.ldq = g->ldq, a.ldk = g->ldk, a.ldv = g->ldv;
+  a.gq = (const uint16_t*)g->q_gamma, a.gk = (const uint16_t*)g->k_gamma;
+  a.epsq = g->q_eps, a.epsk = g->k_eps;
+  a.cos = (const uint16_t*)g->cos, a.sin = (const uint16_t*)g->sin;
+  a.ldc = g->ld_cos, a.lds = g->ld_sin;
+  a.ck = (uint16_t*)g->cache_k, a.cv = (uint16_t*)g->cache_v;
+  a.ckb = g->k_s_b, a.ckh = g->k_s_h, a.cks = g->k_s_p;
+  a.cvb = g->v_s_b, a.cvh = g->v_s_h, a.cvs = g->v_s_p;
+  a.y = (uint16_t*)g->y;
+  a.B = (int)g->B, a.T = (int)T, a.Hq = (int)g->n_heads, a.Hk = (int)g->n_kv_heads, a.S = (int)S;
+  a.pos = g->pos;
+  a.pos_dev = g->pos_dev;
+  return fp::launch_status(fp::launch_attention(a, D, keys, workspace, (hipStream_t)stream));
 }
 
 int fp_quantize_w8_per_row(const void* w, int64_t ldw, int8_t* q, int64_t ldq, float* scale,

@@ -166,6 +166,33 @@ bool use_gemm_split(const StreamArgs& a, bool aligned, bool gateup, GemmSplit* p
 template <bool GATEUP, bool W8>
 int launch_gemm_split(const StreamArgs& a, const GemmSplit& p, hipStream_t s);
 
+// What follows the QKV projection up to the o projection (fp_attn.hip). q, k, v
+// rows m = b T + t (Hq, Hk, Hk heads of D, row strides ld*), gq/gk the QK-norm
+// weights or NULL, cos/sin rows t, the layer's cache [b][head][position][D] by
+// strides (elements), y [B T][Hq D]. The tokens are at pos + t, or *pos_dev + t.
+struct AttnArgs {
+  const uint16_t *q, *k, *v;
+  int64_t ldq, ldk, ldv;
+  const uint16_t *gq, *gk;
+  float epsq, epsk;
+  const uint16_t *cos, *sin;
+  int64_t ldc, lds;
+  uint16_t *ck, *cv;
+  int64_t ckb, ckh, cks, cvb, cvh, cvs;
+  uint16_t* y;
+  int B, T, Hq, Hk, S;  // S: positions in the cache
+  int64_t pos;
+  const int64_t* pos_dev;
+  // workspace: normalised and rotated q [B T][Hq][D]; a split's partial sums
+  // [nsplit][B Hk][rows][D] and their {max, sum}
+  uint16_t* qn;
+  float *part, *stat;
+  int nsplit;
+};
+// keys: the keys the call may see (pos + T; with pos_dev the whole cache).
+int64_t attn_workspace_bytes(int64_t B, int64_t T, int64_t Hq, int64_t Hk, int64_t D, int64_t keys);
+int launch_attention(AttnArgs a, int64_t D, int64_t keys, void* ws, hipStream_t s);
+
 // Device-side per-row int8 quantisation.
 int launch_quantize_w8(const uint16_t* w, int64_t ldw, int8_t* q, int64_t ldq,
                        float* scale, int64_t N, int64_t K, hipStream_t s);

@@ -280,6 +280,92 @@ at::Tensor rmsnorm_gate_up_silu_w8(const at::Tensor& x, const at::Tensor& gamma,
   return y;
 }
 
+// ---- the attention layer between its projections ----
+
+// q [B, T, n] as rows b*T + t of a row stride the kernels take; -1 if not.
+int64_t token_rows(const at::Tensor& t, int64_t B, int64_t T, int64_t n) {
+  if (t.dim() != 3 || t.size(0) != B || t.size(1) != T || t.size(2) != n || t.stride(2) != 1)
+    return -1;
+  const int64_t ld = T > 1 ? t.stride(1) : B > 1 ? t.stride(0) : n;
+  if (B > 1 && t.stride(0) != T * ld) return -1;
+  return ld >= n && ld % 4 == 0 && (uintptr_t)t.data_ptr() % 8 == 0 ? ld : -1;
+}
+
+// q, k, v: the projection's flat outputs. q_gamma, k_gamma: the QK-norm
+// weights, or absent where q and k are normalised already. Returns the
+// attention output [B, T, n_heads * D], or an empty 1-D tensor, with nothing
+// launched and nothing written, where the kernels do not take the call (types,
+// devices, sizes, strides): the caller then runs the torch form, which also
+// raises the errors of invalid calls.
+at::Tensor attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                     const c10::optional<at::Tensor>& q_gamma,
+                     const c10::optional<at::Tensor>& k_gamma, double q_eps, double k_eps,
+                     const at::Tensor& cos, const at::Tensor& sin, at::Tensor cache_k,
+                     at::Tensor cache_v, int64_t n_heads, int64_t start_pos,
+                     const c10::optional<at::Tensor>& pos) {
+  const auto none = [&] { return at::empty({0}, q.options()); };
+  const auto bf16_here = [&](const at::Tensor& t) {
+    return t.scalar_type() == at::kBFloat16 && t.device() == q.device() &&
+           t.layout() == at::kStrided && !t.is_neg();
+  };
+  for (const at::Tensor* t : {&q, &k, &v, &cos, &sin, (const at::Tensor*)&cache_k,
+                              (const at::Tensor*)&cache_v})
+    if (!bf16_here(*t)) return none();
+  if (!q.is_cuda() || q.dim() != 3 || cache_k.dim() != 4 || cache_v.dim() != 4) return none();
+  const int64_t B = q.size(0), T = q.size(1), Hk = cache_k.size(1), S = cache_k.size(2);
+  const int64_t D = cache_k.size(3);
+  if (B < 1 || T < 1 || Hk < 1 || n_heads < 1 || n_heads % Hk != 0) return none();
+  if (cache_v.sizes() != cache_k.sizes() || cache_k.size(0) < B || cache_k.stride(3) != 1 ||
+      cache_v.stride(3) != 1)
+    return none();
+  fp_attention_args a{};
+  a.ldq = token_rows(q, B, T, n_heads * D);
+  a.ldk = token_rows(k, B, T, Hk * D);
+  a.ldv = token_rows(v, B, T, Hk * D);
+  if (a.ldq < 0 || a.ldk < 0 || a.ldv < 0) return none();
+  for (const at::Tensor* t : {&cos, &sin})
+    if (t->dim() != 2 || t->size(0) != T || t->size(1) != D || t->stride(1) != 1) return none();
+  if (q_gamma.has_value() != k_gamma.has_value()) return none();
+  if (q_gamma.has_value()) {
+    for (const at::Tensor* t : {&*q_gamma, &*k_gamma})
+      if (!bf16_here(*t) || t->dim() != 1 || t->size(0) != D || t->stride(0) != 1) return none();
+    a.q_gamma = q_gamma->data_ptr(), a.k_gamma = k_gamma->data_ptr();
+  }
+  int64_t keys = S;
+  if (pos.has_value()) {
+    if (pos->dim() != 0 || pos->scalar_type() != at::kLong || pos->device() != q.device())
+      return none();
+    a.pos_dev = pos->data_ptr<int64_t>();
+  } else {
+    if (start_pos < 0 || start_pos + T > S) return none();
+    a.pos = start_pos;
+    keys = start_pos + T;
+  }
+  a.q = q.data_ptr(), a.k = k.data_ptr(), a.v = v.data_ptr();
+  a.cos = cos.data_ptr(), a.sin = sin.data_ptr();
+  a.ld_cos = T > 1 ? cos.stride(0) : D, a.ld_sin = T > 1 ? sin.stride(0) : D;
+  a.cache_k = cache_k.data_ptr(), a.cache_v = cache_v.data_ptr();
+  // a dimension of one element may carry any stride
+  const auto sd = [](const at::Tensor& t, int64_t i) { return t.size(i) > 1 ? t.stride(i) : 0; };
+  a.k_s_b = sd(cache_k, 0), a.k_s_h = sd(cache_k, 1), a.k_s_p = S > 1 ? cache_k.stride(2) : D;
+  a.v_s_b = sd(cache_v, 0), a.v_s_h = sd(cache_v, 1), a.v_s_p = S > 1 ? cache_v.stride(2) : D;
+  a.B = B, a.T = T, a.n_heads = n_heads, a.n_kv_heads = Hk, a.head_dim = D, a.cache_len = S;
+  a.q_eps = (float)q_eps, a.k_eps = (float)k_eps;
+  const c10::DeviceGuard guard(q.device());
+  const int64_t bytes = fp_attention_workspace_bytes(B, T, n_heads, Hk, D, keys);
+  if (bytes <= 0) return none();
+  at::Tensor y = at::empty({B, T, n_heads * D}, q.options());
+  at::Tensor ws = at::empty({bytes}, q.options().dtype(at::kByte));
+  a.y = y.data_ptr();
+  const int st = fp_attention_bf16(&a, ws.data_ptr(), bytes, cur_stream(q));
+  // sizes, strides and alignments that the kernels do not take: nothing ran
+  if (st == FP_ERR_SHAPE || st == FP_ERR_STRIDE) return none();
+  check_status(st, "fp_attention_bf16");
+  for (at::Tensor* t : {&cache_k, &cache_v})
+    if (!t->is_inference()) t->unsafeGetTensorImpl()->bump_version();
+  return y;
+}
+
 std::tuple<at::Tensor, at::Tensor> quantize_w8(const at::Tensor& w) {
   check_2d(w, "W", at::kBFloat16);
   const c10::DeviceGuard guard(w.device());
@@ -307,6 +393,9 @@ TORCH_LIBRARY(llms_amd, m) {
         "int n_k) -> Tensor");
   m.def("rmsnorm_gate_up_silu_w8(Tensor x, Tensor gamma, float eps, Tensor qg, Tensor sg, "
         "Tensor qu, Tensor su) -> Tensor");
+  m.def("attention(Tensor q, Tensor k, Tensor v, Tensor? q_gamma, Tensor? k_gamma, float q_eps, "
+        "float k_eps, Tensor cos, Tensor sin, Tensor(a!) cache_k, Tensor(b!) cache_v, "
+        "int n_heads, int start_pos, Tensor? pos) -> Tensor");
   m.def("quantize_w8(Tensor w) -> (Tensor, Tensor)");
 }
 
@@ -321,5 +410,6 @@ TORCH_LIBRARY_IMPL(llms_amd, CUDA, m) {
   m.impl("rmsnorm_gate_up_silu", rmsnorm_gate_up_silu);
   m.impl("rmsnorm_qkv_w8", rmsnorm_qkv_w8);
   m.impl("rmsnorm_gate_up_silu_w8", rmsnorm_gate_up_silu_w8);
+  m.impl("attention", attention);
   m.impl("quantize_w8", quantize_w8);
 }

@@ -17,6 +17,7 @@ from torch import nn
 from .. import _lib
 from ._checks import inner_contiguous, require_bf16_hip, require_device
 from ._eager import RMSNorm, apply_rope, attend, write_kv
+from .fused_attention import attention_core
 
 
 def triton_fused_qkv(
@@ -126,10 +127,11 @@ def fused_qkv_w8(
 class TritonAttention(nn.Module):
     """Drop-in for the reference's ``TritonAttention``
     (``src/kernels/fused_qkv.py:152-282``): stores one stacked ``W_qkv``
-    instead of ``q``/``k``/``v`` Linears and runs the fused HIP projection;
-    QK-norm, RoPE, the KV-cache write, attention and ``o`` stay eager (the
-    attention core is :func:`attend`, fp32 softmax attention with the
-    reference's causal semantics).
+    instead of ``q``/``k``/``v`` Linears and runs the fused HIP projection.
+    QK-norm, RoPE, the KV-cache write and attention run on HIP kernels too
+    (:func:`~llms_amd.kernels.fused_attention.attention_core`) in bf16
+    inference, else eagerly (:func:`attend`, fp32 softmax attention with the
+    reference's causal semantics); ``o`` is the module's own Linear.
 
     With ``from_eager(..., int8=True)`` the stacked weight is kept as
     per-row int8 (``q_qkv``, ``s_qkv`` buffers) and the int8 kernel runs.
@@ -220,11 +222,18 @@ class TritonAttention(nn.Module):
         start_pos: int,
     ) -> torch.Tensor:
         # The reference forward (src/kernels/fused_qkv.py:242-282) with the
-        # fused HIP projection in place of the Triton call and attend() in
-        # place of its three SDPA branches. start_pos may be a 0-dim device
-        # tensor (a step captured in a HIP graph, replayed at any position).
+        # fused HIP projection in place of the Triton call. start_pos may be a
+        # 0-dim device tensor (a step captured in a HIP graph, replayed at any
+        # position). Between the projections the HIP attention kernels run,
+        # or, where they do not take the call, the torch form with attend() in
+        # place of the reference's three SDPA branches.
         B, T, _ = x.shape
         q_flat, k_flat, v_flat = self.project(x)
+        attn = attention_core(q_flat, k_flat, v_flat, q_norm=self.q_norm, k_norm=self.k_norm,
+                              num_heads=self.num_heads, cache_k=kv_cache.k[layer_idx],
+                              cache_v=kv_cache.v[layer_idx], cos=cos, sin=sin, start_pos=start_pos)
+        if attn is not None:
+            return self.o(attn)
         q = q_flat.view(B, T, self.num_heads, self.head_dim)
         k = k_flat.view(B, T, self.num_kv_heads, self.head_dim)
         v = v_flat.view(B, T, self.num_kv_heads, self.head_dim)

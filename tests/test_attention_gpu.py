@@ -1,0 +1,185 @@
+"""The HIP attention layer core (``kernels/fused_attention.py``) against the torch
+form it stands in for (``kernels/_eager.py``).
+
+QK-norm, RoPE and the cache rows are the same bf16 roundings of the same
+values: the only freedom is the fp32 sum of squares, whose order may move the
+scale by an ulp of fp32 and so flip a bf16 rounding (an ulp, 2^-8 of the value)
+now and then. The attention output is rounded once from fp32, so against the
+fp64 softmax over the kernel's own cache rows it is within half a bf16 ulp plus
+fp32 evaluation error: |y - t| <= 2^-8 |t| + 1e-5 max|v|, the bound of
+``test_attend_cpu.py``.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from llms_amd.kernels import _eager
+from llms_amd.kernels.fused_attention import attention_core
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+def _inputs(seed, B, T, Hq, Hk, D, S, pos, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV)  # noqa: E731
+    n = (Hq + 2 * Hk) * D
+    y = (r(B, T, n) * scale).bfloat16()
+    q, k, v = y.split([Hq * D, Hk * D, Hk * D], dim=-1)
+    qn, kn = _eager.RMSNorm(D).to(DEV, torch.bfloat16), _eager.RMSNorm(D).to(DEV, torch.bfloat16)
+    with torch.no_grad():
+        qn.weight.copy_(1 + 0.1 * r(D))
+        kn.weight.copy_(1 + 0.1 * r(D))
+    cos, sin = (t.to(DEV, torch.bfloat16) for t in _eager.build_rope_tables(D, S, 1e4))
+    ck, cv = (r(B + 1, Hk, S, D).bfloat16() for _ in range(2))
+    ck[:, :, pos:] = float("nan")  # slots not written yet may hold anything
+    cv[:, :, pos:] = float("nan")
+    return dict(q=q, k=k, v=v, q_norm=qn, k_norm=kn, num_heads=Hq, cache_k=ck, cache_v=cv,
+                cos=cos[pos:pos + T], sin=sin[pos:pos + T], start_pos=pos)
+
+
+def _eager_rows(c, B, T, Hq, Hk, D):
+    """q, k, v [B, H, T, D] as the torch form rotates and normalises them."""
+    q = c["q_norm"](c["q"].view(B, T, Hq, D)).transpose(1, 2)
+    k = c["k_norm"](c["k"].view(B, T, Hk, D)).transpose(1, 2)
+    q, k = _eager.apply_rope(q, k, c["cos"], c["sin"])
+    return q, k, c["v"].view(B, T, Hk, D).transpose(1, 2)
+
+
+def _near_bf16(a, b, share=0.01):
+    """Equal in all but `share` of the elements. Where a flipped rounding of a
+    normalised value (its own and its weight product's, 2^-8 of it each) is
+    carried through RoPE's two products and their sum (2^-8 each), the element
+    moves by at most 2^-6 of the size of its rotate-half pair, also where the
+    two products cancel."""
+    d = (a.float() - b.float()).abs()
+    h = b.shape[-1] // 2
+    pair = torch.hypot(b[..., :h].float(), b[..., h:].float())
+    assert bool((d <= 2.0 ** -6 * torch.cat([pair, pair], dim=-1)).all())
+    assert (d > 0).float().mean().item() <= share
+
+
+def _check(c, B, T, Hq, Hk, D, y):
+    """y, and the cache after the call, against the torch form's values."""
+    pos, end = c["start_pos"], c["start_pos"] + T
+    q, k, v = _eager_rows(c, B, T, Hq, Hk, D)
+    _near_bf16(c["cache_k"][:B, :, pos:end], k)
+    assert torch.equal(c["cache_v"][:B, :, pos:end], v)
+    full_k, full_v = (t[:B, :, :end].double().repeat_interleave(Hq // Hk, dim=1)
+                      for t in (c["cache_k"], c["cache_v"]))
+    s = torch.matmul(q.double(), full_k.transpose(-2, -1).contiguous()) * D ** -0.5
+    hide = torch.arange(end, device=DEV)[None] > torch.arange(pos, end, device=DEV)[:, None]
+    t = torch.matmul(torch.softmax(s.masked_fill(hide, float("-inf")), -1), full_v)
+    t = t.transpose(1, 2).reshape(B, T, Hq * D)
+    d = (y.double() - t).abs()
+    rel = (d.norm() / t.norm()).item()
+    print(f"rel {rel:.2e} max {d.max().item():.2e}")
+    # a flipped bf16 rounding of q moves a score, and so a row, by up to 2^-8
+    # of its size: the bound of one rounding in the 2-norm, twice that per value
+    assert rel <= 2.0 ** -8
+    assert bool((d <= 2.0 ** -7 * t.abs() + 2.0 ** -8 * full_v.abs().max()).all())
+
+
+# (B, T, Hq, Hk, D, S, pos): one token and verify steps (1-64 query rows per kv
+# head), the first row count past them, ragged prompts, later chunks; chunk and
+# tile edges of 32, 64 and 128 keys; group sizes 1, 2, 4, 5; a full cache
+CASES = [
+    (1, 1, 32, 8, 128, 64, 0), (1, 1, 32, 8, 128, 4096, 31), (2, 1, 16, 8, 128, 300, 128),
+    (1, 1, 8, 8, 64, 129, 128), (3, 1, 10, 2, 64, 513, 511), (1, 1, 32, 8, 128, 4096, 4095),
+    (1, 4, 32, 8, 128, 2048, 1000), (2, 9, 16, 8, 64, 700, 33), (1, 5, 32, 8, 128, 200, 60),
+    (1, 16, 32, 8, 128, 256, 0), (1, 17, 32, 8, 128, 256, 0), (1, 33, 4, 4, 64, 100, 30),
+    (1, 65, 8, 8, 128, 200, 127), (1, 100, 32, 8, 128, 100, 0), (2, 129, 10, 2, 64, 300, 5),
+    (1, 1000, 32, 8, 128, 1024, 0), (1, 70, 16, 8, 128, 3000, 2900), (1, 2048, 8, 2, 128, 2048, 0),
+]
+
+
+@pytest.mark.parametrize("B,T,Hq,Hk,D,S,pos", CASES)
+def test_matches_fp64_attention(B, T, Hq, Hk, D, S, pos):
+    print(B, T, Hq, Hk, D, S, pos, flush=True)
+    c = _inputs(T + pos, B, T, Hq, Hk, D, S, pos)
+    before = c["cache_v"][B].clone().view(torch.int16)
+    with torch.inference_mode():
+        y = attention_core(**c)
+        _check(c, B, T, Hq, Hk, D, y)
+        # the spare sequence and the slots past the tokens are untouched
+        assert torch.equal(c["cache_v"][B].view(torch.int16), before)
+        assert bool(c["cache_k"][:, :, pos + T:].isnan().all())
+        # a device position: the same values over the whole cache
+        yd = attention_core(**dict(c, start_pos=torch.tensor(pos, device=DEV)))
+        assert (yd.float() - y.float()).abs().max() <= 2.0 ** -7 * y.float().abs().max()
+        assert torch.equal(attention_core(**c), y)
+
+
+@pytest.mark.parametrize("T,pos", [(1, 200), (4, 77), (200, 40)])
+def test_infinities_and_nan_like_the_torch_form(T, pos):
+    """inf and NaN among the keys and values of visible positions reach the
+    output as in fp32: an infinite value stays infinite, a NaN or an infinite
+    score makes its row NaN."""
+    B, Hq, Hk, D, S = 1, 8, 2, 128, 512
+    for what in ("v inf", "v nan", "k nan", "k inf"):
+        print(T, pos, what, flush=True)
+        c = _inputs(3, B, T, Hq, Hk, D, S, pos)
+        t = c["cache_v" if what[0] == "v" else "cache_k"]
+        t[0, 1, pos - 9, 5] = float(what[2:])
+        with torch.inference_mode():
+            y = attention_core(**c).view(T, Hq, D)
+            q, k, v = _eager_rows(c, B, T, Hq, Hk, D)
+            fk, fv = (u[:B, :, :pos + T].repeat_interleave(Hq // Hk, dim=1)
+                      for u in (c["cache_k"], c["cache_v"]))
+            r = _eager.attend(q, fk, fv, pos)[0].transpose(0, 1)
+        for f in (torch.isnan, torch.isposinf, torch.isneginf):
+            assert torch.equal(f(y), f(r)), (what, f)
+        ok = torch.isfinite(r)
+        assert (y[ok].float() - r[ok].float()).abs().max() <= 2.0 ** -6 * r[ok].float().abs().max()
+
+
+def test_calls_left_to_the_torch_form():
+    """Nothing is launched or written for a call the kernels do not take."""
+    B, T, Hq, Hk, D, S, pos = 1, 2, 4, 2, 64, 40, 7
+    c = _inputs(1, B, T, Hq, Hk, D, S, pos)
+    k0 = c["cache_k"].clone().view(torch.int16)
+
+    class Other(_eager.RMSNorm):
+        pass
+
+    odd = c["cache_k"].transpose(-1, -2).contiguous().transpose(-1, -2)  # D not innermost
+    with torch.no_grad():
+        for change in (dict(start_pos=S - 1), dict(start_pos=-1), dict(q_norm=Other(D).to(DEV)),
+                       dict(cos=c["cos"].float()), dict(cos=c["cos"][:1]), dict(cache_k=odd),
+                       dict(cache_v=c["cache_v"].float()), dict(k=c["k"].float()),
+                       dict(start_pos=torch.tensor(7)), dict(num_heads=3),
+                       dict(start_pos=torch.tensor(7, device=DEV, dtype=torch.int32))):
+            print(list(change), flush=True)
+            assert attention_core(**dict(c, **change)) is None, change
+    with torch.enable_grad():  # the norm weights are parameters
+        assert attention_core(**c) is None
+    h = c["q_norm"].register_forward_hook(lambda *a: None)
+    with torch.no_grad():
+        assert attention_core(**c) is None
+    h.remove()
+    assert torch.equal(c["cache_k"].view(torch.int16), k0)
+    with torch.no_grad():
+        assert attention_core(**c) is not None
+
+
+def test_cache_layouts_and_strided_rows():
+    """A cache laid out [B, S, H, D], a padded one, and projections in a wider
+    buffer give the contiguous call's bits."""
+    B, T, Hq, Hk, D, S, pos = 2, 3, 8, 2, 128, 96, 50
+    c = _inputs(9, B, T, Hq, Hk, D, S, pos)
+    with torch.inference_mode():
+        want = attention_core(**c)
+        for f in (lambda t: t.transpose(1, 2).contiguous().transpose(1, 2),
+                  lambda t: torch.nn.functional.pad(t, (0, 8))[..., :D],
+                  lambda t: t[:B].clone()):
+            d = dict(c, cache_k=f(c["cache_k"]), cache_v=f(c["cache_v"]))
+            assert torch.equal(attention_core(**d), want)
+            assert torch.equal(d["cache_k"][:B, :, :pos + T], c["cache_k"][:B, :, :pos + T])
+        wide = torch.nn.functional.pad(torch.cat([c["q"], c["k"], c["v"]], -1), (4, 12))
+        n = Hq * D
+        d = dict(c, q=wide[..., 4:4 + n], k=wide[..., 4 + n:4 + n + Hk * D],
+                 v=wide[..., 4 + n + Hk * D:4 + n + 2 * Hk * D])
+        assert torch.equal(attention_core(**d), want)
