@@ -97,18 +97,39 @@ int64_t w8_workspace_bytes(int64_t M, int64_t N, int64_t K, bool gateup) {
   return p8.tile >= 0 ? 4 * gemm_split_ws_floats(p8, M, N, K, gateup) : 0;
 }
 
+// Where the rows kernel, if it takes the call, also normalises. Every one of its
+// workgroups (N / 8 of them, several rounds for gate-up) repeats the norm of all
+// the rows behind two barriers, which costs more with each element of x, while a
+// launch of rmsnorm_kernel costs 2-3.5 us once and lets the plain dispatch choose
+// its kernel (int8 from 2 rows: fp_xpanel.hip). One box, 12 weight sets in a
+// graph, us, in the rows kernel / as its own launch: bf16 one row, 4B QKV 8.70 /
+// 9.17, gate-up 18.05 / 18.85, 8B 10.89 / 12.50, 32.19 / 34.13; two rows, 0.6B
+// (K = 1024) 5.14 / 5.97, 6.60 / 7.28, 4B 10.94 / 10.37, 22.32 / 20.35, 8B 13.95 /
+// 13.14, 38.39 / 34.59; int8 one row, 0.6B 4.33 / 5.27, 5.49 / 5.95, 4B 8.37 /
+// 8.54, 16.24 / 13.55, 8B 9.84 / 9.67, 23.96 / 22.12; two rows, 0.6B 4.87 / 5.88,
+// 6.97 / 7.16, 4B 10.21 / 9.46, 20.69 / 19.29; three and four rows, 0.6B 6.90-8.80 /
+// 6.35-7.28, 4B 14.3-14.8 / 9.4-9.6, 29.7-31.2 / 19.3-19.4.
+template <bool GATEUP, bool W8>
+bool norm_in_rows(int64_t M, int64_t K) {
+  if (W8) return M <= 2 && M * K <= (GATEUP ? 2048 : 2560);
+  return M == 1 || M * K <= 2048;
+}
+
 // RMSNorm prologue + projection: one launch on the rows kernel (x normalised
-// while it is staged in LDS), else the norm into the workspace and the plain
-// dispatch on the normalised rows (any split workspace follows them).
+// while it is staged in LDS) where norm_in_rows says so or no workspace is
+// there, else the norm into the workspace and the plain dispatch on the
+// normalised rows (any split workspace follows them).
 // xaligned: x rows and K fit the vector path; waligned: the weights do.
 template <bool GATEUP, bool W8>
 int run_norm(StreamArgs a, bool xaligned, bool waligned, void* ws, int64_t ws_bytes,
              hipStream_t s) {
   if (a.M == 0) return FP_OK;
   const bool galigned = al16(a.gamma);
-  if (rows_supported<W8>(a, xaligned && waligned && galigned))
-    return launch_status(launch_rows<GATEUP, W8>(a, s));
   const int64_t xn_bytes = round_up(a.M * a.K * 2, 256);
+  const bool room = ws && ws_bytes >= xn_bytes;
+  if (rows_supported<W8>(a, xaligned && waligned && galigned) &&
+      (!room || norm_in_rows<GATEUP, W8>(a.M, a.K)))
+    return launch_status(launch_rows<GATEUP, W8>(a, s));
   if (!ws || ws_bytes < xn_bytes) return FP_ERR_WORKSPACE;
   uint16_t* xn = (uint16_t*)ws;
   int rc = launch_rmsnorm(a.x, a.ldx, a.gamma, a.eps, xn, a.M, a.K,

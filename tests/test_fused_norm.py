@@ -237,3 +237,35 @@ def test_norm_deterministic_and_raw_abi(M):
                                    need, stream) == 0
     torch.cuda.synchronize()
     assert torch.equal(y.view(torch.int16), a.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K", [(1, 2048), (1, 2064), (1, 2560), (1, 2576), (2, 1024), (2, 1032),
+                                 (2, 1280), (2, 1296), (3, 512), (4, 2560)])
+def test_norm_in_rows_or_apart(M, K):
+    """Row counts and sizes on both sides of the rule that leaves the norm to
+    the row kernel or to a launch of its own, and the call without a workspace
+    (always the row kernel): both are the oracle's result."""
+    from llms_amd import _lib
+
+    kern = _kern()
+    check_norm_qkv(M, K, 96, 16, seed=60 + K + M)
+    check_norm_gate_up(M, K, 100, seed=61 + K + M)
+    x, g = _x(62, M, K), _norm_weight(63, K)
+    _, wg, wu = ffn_inputs(64, 1, K, 100)
+    qg, sg = kern.quantize_w8_per_row(wg.to(DEV))
+    qu, su = kern.quantize_w8_per_row(wu.to(DEV))
+    if K % 16:
+        return
+    y = kern.fused_rmsnorm_gate_up_silu_w8(x.to(DEV), g.to(DEV), EPS, qg, sg, qu, su).cpu()
+    xd, gd = x.to(DEV), g.to(DEV)
+    y0 = torch.empty(M, 100, dtype=torch.bfloat16, device=DEV)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    assert _lib.capi().fp_rmsnorm_gate_up_silu_w8(
+        P(xd), K, P(gd), EPS, P(qg), K, P(sg), P(qu), K, P(su), P(y0), 100, M, 100, K, None, 0,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    out = ref.ref_rmsnorm_gate_up_silu_full(
+        bits(x), bits(g), EPS, ref.dequant_w8(qg.cpu().numpy(), sg.cpu().numpy()),
+        ref.dequant_w8(qu.cpu().numpy(), su.cpu().numpy()))
+    _check(y, out, f"int8 norm+gate-up M={M} K={K}")
+    _check(y0.cpu(), out, f"int8 norm+gate-up M={M} K={K}, no workspace")
