@@ -49,6 +49,7 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4_t;
 
+constexpr int kAttnMaxSplit = 64;  // one lane per split in attn_combine_kernel
 constexpr float kLog2e = 1.4426950408889634f;
 
 constexpr int vmcnt_imm(int v) { return (v & 15) | (7 << 4) | (15 << 8) | ((v >> 4) << 14); }
@@ -658,31 +659,44 @@ __global__ __launch_bounds__(256, 2) void attn_tiles_kernel(AttnArgs a, int n_rt
   }
 }
 
-// One output row per D / 4 lanes: the splits' partials in split order.
+// One output row per workgroup: lane s of each wave holds split s's statistics
+// (at most 64 splits), so the weights take one load and a few lane exchanges;
+// then each group of D / 4 threads sums every NG-th split's partials and the
+// groups' sums are added in group order (one serial chain over the splits ran
+// 7-8 us for 16 splits of 32 rows, this 3).
 template <int D>
 __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
-  constexpr int LPR = D / 4;
-  const int64_t rows = (int64_t)a.T * (a.Hq / a.Hk), total = (int64_t)a.B * a.Hk * rows;
-  const int64_t i = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
-  if (i >= total) return;
-  const int d = (threadIdx.x % LPR) * 4;
-  float m = -INFINITY;
-  for (int s = 0; s < a.nsplit; ++s) m = fmaxf(m, a.stat[(s * total + i) * 2]);
+  constexpr int LPR = D / 4, NG = 256 / LPR;
+  __shared__ __attribute__((aligned(16))) f32x4 part[NG][LPR];
+  const int rows = a.T * (a.Hq / a.Hk);
+  const int64_t total = (int64_t)a.B * a.Hk * rows, i = blockIdx.x;
+  const int lane = threadIdx.x & (kWave - 1), grp = threadIdx.x / LPR, q = threadIdx.x % LPR;
+  const bool has = lane < a.nsplit;
+  f32x2 st = {-INFINITY, 0.f};
+  if (has) st = *reinterpret_cast<const f32x2*>(a.stat + (lane * total + i) * 2);
+  float m = st.x;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
   const float base = m == -INFINITY ? 0.f : m;
-  float l = 0.f;
+  const float e = has ? exp2_fast(st.x - base) : 0.f;
+  const float l = wave_sum(has ? e * st.y : 0.f);
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int s = 0; s < a.nsplit; ++s) {
-    const int64_t pr = s * total + i;
-    const f32x2 st = *reinterpret_cast<const f32x2*>(a.stat + pr * 2);
-    const float e = exp2_fast(st.x - base);
-    l += e * st.y;
-    v += *reinterpret_cast<const f32x4*>(a.part + pr * D + d) * e;
+#pragma unroll
+  for (int n = 0; n < kAttnMaxSplit / NG; ++n) {
+    const int s = n * NG + grp;
+    const float w = __shfl(e, s);  // every lane takes part in the exchange
+    if (s < a.nsplit)
+      v += *reinterpret_cast<const f32x4*>(a.part + (s * total + i) * D + q * 4) * w;
   }
+  part[grp][q] = v;
+  __syncthreads();
+  if (grp != 0) return;
+#pragma unroll
+  for (int g = 1; g < NG; ++g) v += part[g][q];
   const int bh = (int)(i / rows), b = bh / a.Hk, kh = bh - b * a.Hk;
-  const int rr = (int)(i - bh * rows), G = a.Hq / a.Hk;
+  const int rr = (int)(i - (int64_t)bh * rows), G = a.Hq / a.Hk;
   const int t = rr / G, h = kh * G + (rr - t * G);
-  uint16_t* yp = a.y + (((int64_t)b * a.T + t) * a.Hq + h) * D + d;
+  uint16_t* yp = a.y + (((int64_t)b * a.T + t) * a.Hq + h) * D + q * 4;
   *reinterpret_cast<u32x2*>(yp) = u32x2{pack_bf16x2(v[0] / l, v[1] / l), pack_bf16x2(v[2] / l, v[3] / l)};
 }
 
@@ -696,7 +710,6 @@ struct AttnPlan {
 
 constexpr int kAttnRowsMax = 64;    // query rows per kv head of attn_rows_kernel
 constexpr int kAttnGroups = 512;    // workgroups a call aims at (two per CU)
-constexpr int kAttnMaxSplit = 64;
 
 // S: the keys a call may see (an int position: start + T; a device position:
 // the whole cache). Splits: as many key ranges as give about two workgroups
@@ -743,8 +756,7 @@ int launch_attn_d(AttnArgs a, int64_t S, hipStream_t s) {
   }
   e = (int)hipGetLastError();
   if (e || p.nsplit == 1) return e;
-  const int64_t rows = (int64_t)a.B * a.T * a.Hq, rpb = 256 / (D / 4);
-  hipLaunchKernelGGL(attn_combine_kernel<D>, dim3((unsigned)((rows + rpb - 1) / rpb)), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(attn_combine_kernel<D>, dim3((unsigned)((int64_t)a.B * a.T * a.Hq)), dim3(256), 0, s, a);
   return (int)hipGetLastError();
 }
 

@@ -360,6 +360,42 @@ int launch_rows_cfg(const StreamArgs& a, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
+// The same for rows of at most 2048 NV elements that fit the vector path: x and
+// the norm weight are loaded once, together, and stay in registers across the
+// sum (the squares are added in row_sumsq's order: bit-identical). The plain
+// form below waits for memory three times in a row, which at few rows is the
+// kernel, and reads x twice.
+template <int NV>
+__global__ __launch_bounds__(256) void rmsnorm_once_kernel(const uint16_t* x, int64_t ldx,
+                                                           const uint16_t* gamma, float eps,
+                                                           uint16_t* xn, int K) {
+  __shared__ float red[256 / kWave];
+  const uint16_t* row = x + (int64_t)blockIdx.x * ldx;
+  uint16_t* out = xn + (int64_t)blockIdx.x * K;
+  u32x4 v[NV], g[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int k = ((int)threadIdx.x + 256 * i) * 8;
+    v[i] = k < K ? ld16(row + k) : u32x4{0u, 0u, 0u, 0u};
+    g[i] = k < K ? ld16(gamma + k) : u32x4{0u, 0u, 0u, 0u};
+  }
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float lo = bf16_bits_to_f32(v[i][j] & 0xffffu), hi = bf16_bits_to_f32(v[i][j] >> 16);
+      s += __fmul_rn(lo, lo);
+      s += __fmul_rn(hi, hi);
+    }
+  const float r = rms_scale(block_sum<256>(s, red), K, eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int k = ((int)threadIdx.x + 256 * i) * 8;
+    if (k < K) *reinterpret_cast<u32x4*>(out + k) = norm_bf16x8(v[i], g[i], r);
+  }
+}
+
 // One workgroup per row: the row's scale, then the normalised row.
 template <bool VEC>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* x, int64_t ldx,
@@ -388,7 +424,14 @@ bool rows_fit(int64_t M, int64_t K, bool w8, bool norm) {
 
 int launch_rmsnorm(const uint16_t* x, int64_t ldx, const uint16_t* gamma, float eps,
                    uint16_t* xn, int64_t M, int64_t K, bool vec, hipStream_t s) {
-  if (vec)
+  const dim3 grid((unsigned)M), block(256);
+  if (vec && K <= 2048)
+    hipLaunchKernelGGL(rmsnorm_once_kernel<1>, grid, block, 0, s, x, ldx, gamma, eps, xn, (int)K);
+  else if (vec && K <= 4096)
+    hipLaunchKernelGGL(rmsnorm_once_kernel<2>, grid, block, 0, s, x, ldx, gamma, eps, xn, (int)K);
+  else if (vec && K <= 8192)
+    hipLaunchKernelGGL(rmsnorm_once_kernel<4>, grid, block, 0, s, x, ldx, gamma, eps, xn, (int)K);
+  else if (vec)
     hipLaunchKernelGGL(rmsnorm_kernel<true>, dim3((unsigned)M), dim3(256), 0, s, x, ldx, gamma,
                        eps, xn, K);
   else
