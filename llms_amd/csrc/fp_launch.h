@@ -76,12 +76,14 @@ bool splitk_supported(const StreamArgs& a, bool aligned, bool w8);
 // tiles (dequantising in registers) rather than the row, streaming or
 // dequantise-first paths. Measured on MI355X over Qwen3-4B/8B QKV, gate-up,
 // o and down: from 2 rows for gate-up and 3 for other outputs (5 for outputs
-// of at most 4096 columns with K <= 8192, where the row kernel holds up to
-// 4), up to 128 rows; above 64 rows only with K <= 8192 (the long-K down
+// under 2048 columns with K <= 8192, where the row kernel holds up to 4 and 64
+// tiles of 16 rows are too few: 0.6B o and down at 4 rows 3.9, 4.6 us against 4.3,
+// 5.4; at 2560 and 4096 columns, 4B and 8B o at 3 and 4 rows, 7.3-8.2 against
+// 6.3-6.7), up to 128 rows; above 64 rows only with K <= 8192 (the long-K down
 // projections keep the dequantise-first path with k split across
 // workgroups).
 inline bool splitk8_shape(int64_t M, int64_t N, int64_t K, bool gateup) {
-  const int64_t min_m = gateup ? 2 : ((N <= 4096 && K <= 8192) ? 5 : 3);
+  const int64_t min_m = gateup ? 2 : ((N < 2048 && K <= 8192) ? 5 : 3);
   if (M < min_m || M > kSplitkMaxM8 || K % 64 != 0) return false;
   return M <= 64 || K <= 8192;
 }

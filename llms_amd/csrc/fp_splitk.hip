@@ -295,15 +295,12 @@ bool splitk_supported(const StreamArgs& a, bool aligned, bool w8) {
 // sets, warm clocks): the x tile is M rounded up to 16 (up to 64 rows), then
 // 64 x 64 tiles; gate-up tiles hold 16 outputs (32 weight rows). int8 (half
 // the bytes per weight row, so more rows of LDS per wave) prefers 8 waves.
-// Narrow bf16 outputs at up to 16 rows with K >= 2560 (the per-GPU shards
-// of tensor parallelism: QKV of at most 2048 columns, gate-up of at most
-// 3072; also 0.6B down) have too few tiles for 256 CUs; 8 waves per tile put
-// twice the k-steps in flight there. Same-box A/B, µs at M = 4 and 8, 4 -> 8
-// waves: 8B QKV 1536 columns 8.1-8.4 -> 6.1-7.0, 768 columns 8.0-8.2 ->
-// 5.6-7.2; 8B gate-up 3072 columns 12.5-12.8 -> 11.0-11.7, 1536 columns
-// 10.7-11.2 -> 8.8-9.6; 4B QKV 768 and 1536 columns 6.0-6.8 -> 4.6-5.9;
-// 0.6B down (1024 x 3072) 6.5-7.0 -> 5.7-6.3. The full Qwen3-4B/8B outputs
-// keep 4 waves (8 were 2-14% slower there).
+// Narrow bf16 gate-up at up to 16 rows with K >= 2560 (at most 3072 columns:
+// shards of tensor parallelism) has too few tiles for 256 CUs; 8 waves per
+// tile put twice the k-steps in flight there. Same-box A/B, µs at M = 4 and
+// 8, 4 -> 8 waves: 8B gate-up 3072 columns 12.5-12.8 -> 11.0-11.7, 1536
+// columns 10.7-11.2 -> 8.8-9.6. The full Qwen3-4B/8B outputs keep 4 waves (8
+// were 2-14% slower there). Narrow QKV-like outputs: launch_splitk_narrow.
 // int8 gate-up over wide outputs (at least 7680 columns, so that 96-row
 // tiles number 160 or more: Qwen3-4B and 8B) from 17 rows: 96 weight rows
 // (48 outputs) per tile. Every tile reads the x rows of the call again from
@@ -318,8 +315,42 @@ bool splitk_supported(const StreamArgs& a, bool aligned, bool w8) {
 // Each weight is dequantised once per row tile, so one tile over all the
 // rows beats two. At 16 rows 96 x 16 was slower (29.8 / 18.9 against 26.6
 // / 18.5).
+// Narrow outputs (at most 4096 columns: o, down, the shards of tensor
+// parallelism): the finest weight tile whose grid is one round of the chip, 16
+// rows (8 waves, 4 for bf16 at 33-64 rows, where the x rows need the LDS) or from
+// 65 rows also 32. With the 32- and 64-row tiles of wider outputs, 2560 columns
+// gave 80 or 40 workgroups for 256 CUs. Same wave and step order per wave count:
+// bit-identical unless the count changed. One box, 6-36 weight sets in a graph,
+// us: int8 4B down M = 4, 16, 24, 64 16.7, 19.8, 23.2, 34.3 -> 11.5, 13.7, 16.7,
+// 27.3, o M = 8, 24, 64, 128 9.0, 11.9, 16.7, 25.7 -> 6.6, 9.1, 13.4, 17.5, 8B
+// down M = 4, 16, 64 22.0, 26.3, 44.4 -> 15.3, 18.3, 35.4, 0.6B down M = 100 20.8
+// -> 11.1; bf16 4B down M = 3, 16, 24 15.5, 18.5, 25.3 -> 11.8, 15.6, 18.5, o M =
+// 3, 24, 64, 126 8.2, 12.7, 17.2, 26.2 -> 6.3, 9.1, 14.5, 18.6, 8B down M = 8, 24
+// 22.0, 32.7 -> 18.5, 24.8, o M = 8 9.6 -> 7.8. Past one round the finer tile
+// loses (int8 8B QKV, 6144 columns, M = 100 on 32-row tiles 27.2 -> 32.5; 16-row
+// tiles of 4B o at M = 80, 320 of them, 23.4 against 17.1 on 32 rows).
+template <bool W8>
+int launch_splitk_narrow(const StreamArgs& a, hipStream_t s) {
+  const auto round = [&](int64_t bn, int64_t bm) {
+    return ((a.N + bn - 1) / bn) * ((a.M + bm - 1) / bm) <= 256;
+  };
+  if (a.M <= 16) return launch_splitk_cfg<16, 16, 8, 3, false, W8>(a, s);
+  if (a.M <= 32) return launch_splitk_cfg<16, 32, 8, 2, false, W8>(a, s);
+  if (a.M <= 64 || round(16, 64)) {
+    if constexpr (W8) return launch_splitk_cfg<16, 64, 8, 2, false, true>(a, s);
+    return launch_splitk_cfg<16, 64, 4, 3, false, W8>(a, s);
+  }
+  if (round(32, 64)) {
+    if constexpr (W8) return launch_splitk_cfg<32, 64, 8, 2, false, true>(a, s);
+    return launch_splitk_cfg<32, 64, 4, 3, false, W8>(a, s);
+  }
+  return launch_splitk_cfg<64, 64, 4, 2, false, W8>(a, s);
+}
+
 template <bool GATEUP, bool W8>
 int launch_splitk(const StreamArgs& a, hipStream_t s) {
+  if constexpr (!GATEUP)
+    if (a.N <= 4096) return launch_splitk_narrow<W8>(a, s);
   if constexpr (W8 && GATEUP) {
     if (a.M > 16 && a.N >= 7680) {
       if (a.M <= 32) return launch_splitk_cfg<96, 32, 4, 3, true, true>(a, s);
@@ -380,9 +411,7 @@ int launch_splitk(const StreamArgs& a, hipStream_t s) {
     // on Qwen3-8B, K = 4096, and 0.6B, K = 1024, they measured 3-12% slower)
     if (a.M <= 16 && a.N > 4096 && a.N <= 8192 && a.K >= 2048 && a.K <= 3072)
       return launch_splitk_cfg<32, 16, 8, 2, false, W8>(a, s);
-    if (a.M <= 16)
-      return a.N <= 2048 && a.K >= 2560 ? launch_splitk_cfg<16, 16, 8, 3, false, W8>(a, s)
-                         : launch_splitk_cfg<16, 16, 4, 3, false, W8>(a, s);
+    if (a.M <= 16) return launch_splitk_cfg<16, 16, 4, 3, false, W8>(a, s);
     if (a.M <= 32) return launch_splitk_cfg<32, 32, 4, 3, false, W8>(a, s);
     if (a.M <= 64) return launch_splitk_cfg<32, 64, 4, 3, false, W8>(a, s);
     return launch_splitk_cfg<64, 64, 4, 2, false, W8>(a, s);

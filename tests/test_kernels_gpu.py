@@ -1118,3 +1118,33 @@ def test_tile_loops_few_ksteps(K):
     _check(y[rows], ref.ref_gate_up_silu_w8_full(bits(x)[rows], qg.cpu().numpy(), sg.cpu().numpy(),
                                                  qu.cpu().numpy(), su.cpu().numpy()),
            f"int8 gate-up M={M} K={K}")
+
+
+# (M, K, N): one and two x rows on whole rows split over eight waves (K of every
+# chunk count from 5 to 24, a last chunk partly past the row, the first K past
+# the limit; N below, at and past 2, 3, 5 and 6 rows per workgroup, a partial last
+# workgroup), and the 16- and 32-row split-K tiles at their row edges, one past one
+# round of the chip (2560 columns at 65-128 rows: 32-row tiles; 1024: 16-row)
+NARROW = [(1, 2560, 2560), (2, 4104, 2555), (1, 9728, 2561), (2, 12288, 1300), (1, 12296, 1300),
+          (1, 4096, 1000), (2, 8192, 1025), (1, 2568, 7), (2, 5000, 2657), (1, 4112, 1328),
+          (3, 1024, 4096), (16, 2048, 2555), (17, 2112, 4095), (32, 4096, 1000), (33, 2560, 2560),
+          (64, 2048, 4096), (65, 2048, 1024), (96, 4096, 2550), (128, 2048, 2560), (127, 2048, 4090)]
+
+
+@pytest.mark.parametrize("M,K,N", NARROW)
+def test_narrow_outputs(M, K, N):
+    """Outputs of at most 4096 columns at few rows, bf16 and int8, with x as a
+    row-strided view."""
+    kern = _kernels()
+    x, w = qkv_inputs(700 + M, M, K, N, 0)
+    xd = torch.zeros(M, K + 16, dtype=torch.bfloat16, device=DEV)
+    xd[:, :K] = x.to(DEV)
+    wd = w.to(DEV)
+    y = kern.fused_linear(xd[:, :K], wd)
+    _check(y.cpu(), ref.ref_linear(bits(x), bits(w)), f"narrow M={M} K={K} N={N}")
+    q, s = kern.quantize_w8_per_row(wd)
+    y8 = kern.fused_linear_w8(xd[:, :K], q, s)
+    wq = ref.dequant_w8(q.cpu().numpy(), s.cpu().numpy())
+    _check(y8.cpu(), ref.ref_linear(bits(x), wq), f"narrow int8 M={M} K={K} N={N}")
+    assert torch.equal(kern.fused_linear(xd[:, :K], wd), y)
+    assert torch.equal(kern.fused_linear_w8(xd[:, :K], q, s), y8)
