@@ -38,6 +38,9 @@ namespace fp {
 
 namespace {
 
+// rows_narrow_kernel: 512-wide chunks of a row per wave
+constexpr int kNarrowChunks = 3;
+
 // k elements per wave instruction (64 lanes x 16 B)
 template <bool W8>
 constexpr int kc() { return W8 ? 1024 : 512; }
@@ -325,6 +328,104 @@ __global__ __launch_bounds__(NW * kWave) void rows_gate_up_w8_kernel(StreamArgs 
   }
 }
 
+// Narrow outputs (o and down) at one and two x rows, no norm: a workgroup holds R
+// whole rows, as many as make two workgroups per CU, and its eight waves split K,
+// wave w taking the 512-wide chunks w, w + 8, w + 16 of every row. All of the
+// chip's weights are then in flight at once (4B down: 97 KB per workgroup), each
+// wave keeps its part of x in registers for all the rows (no LDS copy, no barrier
+// before the stream), and every CU gets the same share, where 2560 rows in
+// rows_kernel's workgroups of eight give 64 CUs two and the others one. The dot
+// products are rows_kernel's MFMA diagonal; each row's 16-lane sums meet the
+// other waves' in LDS in a fixed order. One box, 13-36 weight sets in a graph,
+// us, rows_kernel -> this: bf16 one row, 4B down 11.64 -> 9.81 (5.1 TB/s), o 6.30
+// -> 5.66, 0.6B down 3.85 -> 3.47; two rows 12.90 -> 10.55, 7.00 -> 6.43, 4.26 ->
+// 3.75; int8 4B down 9.09 -> 8.07 and 11.09 -> 8.59, o 5.10 -> 4.88 and 6.04 ->
+// 6.01. One workgroup of ten rows per CU took 10.3 for 4B down, one of two rows
+// 10.6, R rows with K over four waves 10.4.
+template <int R, int MM, bool W8>
+__global__ __launch_bounds__(512) void rows_narrow_kernel(StreamArgs a) {
+  constexpr int NW = 8, KC = 512, C = kNarrowChunks;
+  constexpr int NQ = (R * MM + 15) / 16;  // groups of 16 outputs
+  constexpr int WB = W8 ? 1 : 2;
+  constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format
+  constexpr uint32_t kPastEnd = 0x80000000u;
+  __shared__ float red[NW][NQ][kWave];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int li = lane & 15;
+  const int K = (int)a.K;
+  const int64_t row0 = (int64_t)blockIdx.x * R;
+  // bytes from the workgroup's first row to the matrix's end: rows past N read
+  // as zeros, and so do lanes past the row's end (an offset past every buffer)
+  const int wbytes = (int)(((a.N - 1 - row0) * a.ldw0 + K) * WB);
+  const auto wrsrc = __builtin_amdgcn_make_buffer_rsrc(
+      (char*)const_cast<void*>(a.w0) + row0 * a.ldw0 * WB, 0, wbytes, kRsrcFlags);
+  const uint32_t ldb = (uint32_t)(a.ldw0 * WB);
+
+  u32x4 wf[C][R];  // int8: the first two dwords
+  u32x4 xv[C][MM];
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int c = wave + NW * i;
+    if (c * KC >= K) continue;  // uniform per wave
+    const int k = c * KC + 8 * lane;
+    const uint32_t voff = k < K ? (uint32_t)(k * WB) : kPastEnd;
+#pragma unroll
+    for (int m = 0; m < MM; ++m)
+      xv[i][m] = m < a.M ? load_bf16x8<true>(a.x + m * a.ldx, k, K) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      // non-temporal (cache-policy bit 1): read once per call
+      if constexpr (W8) {
+        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(wrsrc, voff, r * ldb, 2);
+        wf[i][r] = u32x4{v.x, v.y, 0u, 0u};
+      } else {
+        wf[i][r] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, voff, r * ldb, 2);
+      }
+    }
+  }
+  float keep[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) keep[q] = 0.f;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    float sc = 0.f;
+    if constexpr (W8) sc = row0 + r < a.N ? a.s0[row0 + r] : 0.f;
+    f32x4 d[MM];
+#pragma unroll
+    for (int m = 0; m < MM; ++m) d[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      if ((wave + NW * i) * KC >= K) continue;
+      u32x4 w = wf[i][r];
+      if constexpr (W8) w = dequant8_bf16(w.x, w.y, sc, -128.f * sc);
+#pragma unroll
+      for (int m = 0; m < MM; ++m) d[m] = mfma16(w, xv[i][m], d[m]);
+    }
+#pragma unroll
+    for (int m = 0; m < MM; ++m) {
+      float v = diag(d[m], lane);
+      v += dpp_f32<0xb1>(v);   // sums of the 16-lane rows, as in wave_sum
+      v += dpp_f32<0x4e>(v);
+      v += dpp_f32<0x141>(v);
+      v += dpp_f32<0x140>(v);
+      if (li == (r * MM + m) % 16) keep[(r * MM + m) / 16] = v;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) red[wave][q][lane] = keep[q];
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t >= R * MM) return;
+  float v = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) v += red[w][t / 16][16 * g + t % 16];
+  const int r = t / MM, m = t % MM;
+  if (m < a.M && row0 + r < a.N) a.y[m * a.ldy + row0 + r] = (uint16_t)f32_to_bf16_bits(v);
+}
+
 // x rows staged per workgroup: M rounded up to 1, 2 or 4
 inline int64_t rows_mm(int64_t M) { return M <= 2 ? M : 4; }
 
@@ -489,8 +590,41 @@ int launch_rows_m(const StreamArgs& a, hipStream_t s) {
   }
 }
 
+// Calls that rows_narrow_kernel takes from rows_kernel: where the latter's
+// workgroups of eight rows leave three eighths or more of their rounds idle (at N
+// = 3000, a quarter idle, K = 2560: 4.79 against 5.00; at N = 4096, two full
+// rounds, 8B o 7.44 against 7.72, two rows 7.94 against 11.27), K long enough to give the eight waves work (0.6B o, K
+// = 2048: 2.99 against 3.12; int8, half the bytes, 0.6B down, K = 3072: 3.30
+// against 3.35) and within their chunks, byte offsets below 2^31.
+template <bool W8>
+bool narrow_rows(const StreamArgs& a) {
+  const int64_t wgs = (a.N + 7) / 8, rounds = (wgs + 255) / 256;
+  return !a.gamma && a.M <= 2 && a.N <= 3072 && 8 * wgs <= 5 * 256 * rounds &&
+         a.K >= (W8 ? 4096 : 2560) && a.K <= kNarrowChunks * 8 * 512 &&
+         (a.N * a.ldw0 + a.K) * (W8 ? 1 : 2) < ((int64_t)1 << 31);
+}
+
+template <int R, int MM, bool W8>
+int launch_narrow_cfg(const StreamArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((rows_narrow_kernel<R, MM, W8>), dim3((unsigned)((a.N + R - 1) / R)), dim3(512),
+                     0, s, a);
+  return (int)hipGetLastError();
+}
+// R rows per workgroup: N / 512, rounded up to the next built count
+template <int MM, bool W8>
+int launch_narrow(const StreamArgs& a, hipStream_t s) {
+  const int64_t need = (a.N + 511) / 512;
+  if (need <= 2) return launch_narrow_cfg<2, MM, W8>(a, s);
+  if (need <= 3) return launch_narrow_cfg<3, MM, W8>(a, s);
+  if (need <= 5) return launch_narrow_cfg<5, MM, W8>(a, s);
+  return launch_narrow_cfg<6, MM, W8>(a, s);
+}
+
 template <bool GATEUP, bool W8>
 int launch_rows(const StreamArgs& a, hipStream_t s) {
+  if constexpr (!GATEUP)
+    if (narrow_rows<W8>(a))
+      return a.M == 1 ? launch_narrow<1, W8>(a, s) : launch_narrow<2, W8>(a, s);
   if (a.M == 1) return launch_rows_m<1, GATEUP, W8>(a, s);
   if (a.M == 2) return launch_rows_m<2, GATEUP, W8>(a, s);
   return launch_rows_m<4, GATEUP, W8>(a, s);
