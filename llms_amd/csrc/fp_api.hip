@@ -108,9 +108,11 @@ int64_t w8_workspace_bytes(int64_t M, int64_t N, int64_t K, bool gateup) {
 // 13.14, 38.39 / 34.59; int8 one row, 0.6B 4.33 / 5.27, 5.49 / 5.95, 4B 8.37 /
 // 8.54, 16.24 / 13.55, 8B 9.84 / 9.67, 23.96 / 22.12; two rows, 0.6B 4.87 / 5.88,
 // 6.97 / 7.16, 4B 10.21 / 9.46, 20.69 / 19.29; three and four rows, 0.6B 6.90-8.80 /
-// 6.35-7.28, 4B 14.3-14.8 / 9.4-9.6, 29.7-31.2 / 19.3-19.4.
+// 6.35-7.28, 4B 14.3-14.8 / 9.4-9.6, 29.7-31.2 / 19.3-19.4. A tied head's thousands
+// of workgroups repeat it too often: 151936 x 2560 at one row 120 / 109.
 template <bool GATEUP, bool W8>
-bool norm_in_rows(int64_t M, int64_t K) {
+bool norm_in_rows(int64_t M, int64_t N, int64_t K) {
+  if (N > 32768) return false;
   if (W8) return M <= 2 && M * K <= (GATEUP ? 2048 : 2560);
   return M == 1 || M * K <= 2048;
 }
@@ -128,7 +130,7 @@ int run_norm(StreamArgs a, bool xaligned, bool waligned, void* ws, int64_t ws_by
   const int64_t xn_bytes = round_up(a.M * a.K * 2, 256);
   const bool room = ws && ws_bytes >= xn_bytes;
   if (rows_supported<W8>(a, xaligned && waligned && galigned) &&
-      (!room || norm_in_rows<GATEUP, W8>(a.M, a.K)))
+      (!room || norm_in_rows<GATEUP, W8>(a.M, a.N, a.K)))
     return launch_status(launch_rows<GATEUP, W8>(a, s));
   if (!ws || ws_bytes < xn_bytes) return FP_ERR_WORKSPACE;
   uint16_t* xn = (uint16_t*)ws;

@@ -61,12 +61,10 @@ template <bool GATEUP, bool W8>
 int launch_tiled(const StreamArgs& a, bool aligned, hipStream_t s);
 
 // Split-K MFMA tiles for the middle regime (fp_splitk.hip). bf16: used by
-// launch_stream from kSplitkMinM rows (kSplitkMinMSmallN for calls with at
-// most kSplitkSmallN weight rows; wider gate-up from 4 rows with K > 3072,
-// else 6) and by launch_tiled for small-N calls up to
+// launch_stream from kSplitkMinM rows (gate-up over more than kSplitkSmallN
+// weight rows from 4 rows with K > 3072, else 6) and by launch_tiled for small-N calls up to
 // kSplitkMaxM rows with K >= kSplitkMinKTiled, when splitk_supported() holds.
-constexpr int64_t kSplitkMinM = 8;
-constexpr int64_t kSplitkMinMSmallN = 3;
+constexpr int64_t kSplitkMinM = 3;
 constexpr int64_t kSplitkSmallN = 8192;
 constexpr int64_t kSplitkMaxM = 256;
 constexpr int64_t kSplitkMinKTiled = 2048;

@@ -411,6 +411,16 @@ int launch_splitk(const StreamArgs& a, hipStream_t s) {
     // on Qwen3-8B, K = 4096, and 0.6B, K = 1024, they measured 3-12% slower)
     if (a.M <= 16 && a.N > 4096 && a.N <= 8192 && a.K >= 2048 && a.K <= 3072)
       return launch_splitk_cfg<32, 16, 8, 2, false, W8>(a, s);
+    // Wide outputs (a tied head: thousands of tiles) up to 32 rows: each tile
+    // reads the x rows again, so more weight rows per tile, fewer of them with
+    // a long K at up to 8 rows. One box, us, against the 16-row (from 17 rows
+    // 32-row) tiles: 151936 x 2560 at 8, 16, 24 rows 128.5, 160.4, 188.4 ->
+    // 121.6, 133.7, 158.6; 32000 x 4096 at 16, 32 rows 48.2, 58.4 -> 45.2, 53.8;
+    // 151936 x 4096 at 8 rows stays (193 against 205).
+    if (a.N > 8192 && a.M <= 32) {
+      if (a.M > 16) return launch_splitk_cfg<64, 32, 4, 2, false, W8>(a, s);
+      if (a.K <= 3072 || a.M > 8) return launch_splitk_cfg<32, 16, 4, 3, false, W8>(a, s);
+    }
     if (a.M <= 16) return launch_splitk_cfg<16, 16, 4, 3, false, W8>(a, s);
     if (a.M <= 32) return launch_splitk_cfg<32, 32, 4, 3, false, W8>(a, s);
     if (a.M <= 64) return launch_splitk_cfg<32, 64, 4, 3, false, W8>(a, s);

@@ -366,15 +366,19 @@ int launch_stream(const StreamArgs& a, bool aligned, hipStream_t s) {
   // against large weights): fp_gemm.hip
   if (!W8 && small_round_tile(a.M, a.N, a.K, GATEUP) >= 0 && gemm_supported(a, aligned, false))
     return launch_gemm<GATEUP, false>(a, s);
-  // bf16 from 3 (small N, e.g. QKV) or 8 rows: split-K tiles (fp_splitk.hip)
+  // bf16 outputs of more than 8192 columns from 33 rows: whole rounds of the
+  // prefill tiles (one box, us, 64 rows, against the 32-row split-K tiles:
+  // 151936 x 2560 247.8 -> 180.6, 32000 x 2560 55.0 -> 39.6)
+  if (!W8 && !GATEUP && a.N > kSplitkSmallN && a.M > 32 && gemm_supported(a, aligned, false))
+    return launch_gemm<GATEUP, false>(a, s);
+  // bf16 from 3 rows, wide gate-up from 4 or 6: split-K tiles (fp_splitk.hip)
   const int64_t wrows = GATEUP ? 2 * a.N : a.N;
   // (wide gate-up from fewer rows: 4 with K > 3072, 6 below. One box, µs,
   // stream -> split-K tiles: Qwen3-8B M = 4 34.0 -> 33.2, M = 6 35.1 -> 32.8,
   // M = 7 36.3-37.4 -> 33.0, M = 3 33.0 -> 34.0; Qwen3-4B M = 7 21.0 -> 20.2,
-  // M = 6 even, M = 4 19.3 -> 20.1)
-  const int64_t min_m = wrows <= kSplitkSmallN ? kSplitkMinMSmallN
-                        : GATEUP               ? (a.K > 3072 ? 4 : 6)
-                                               : kSplitkMinM;
+  // M = 6 even, M = 4 19.3 -> 20.1; other wide outputs, 151936 x 2560 at 3
+  // rows 135.8 -> 118.4, 32000 x 4096 at 4 rows 52.9 -> 44.3)
+  const int64_t min_m = GATEUP && wrows > kSplitkSmallN ? (a.K > 3072 ? 4 : 6) : kSplitkMinM;
   if (!W8 && a.M >= min_m && splitk_supported(a, aligned, false))
     return launch_splitk<GATEUP, false>(a, s);
   // (int8 dequantisation needs registers of its own: 2 k-blocks per buffer)

@@ -37,6 +37,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .kernels._eager import RMSNorm, apply_rope, attend, build_rope_tables, write_kv
+from .kernels.fused_norm import fused_rmsnorm_head
 
 
 @dataclass(frozen=True)
@@ -132,6 +133,7 @@ class Qwen3Model(nn.Module):
         self.embed = nn.Embedding(c.vocab_size, c.hidden_size)
         self.layers = nn.ModuleList([DecoderBlock(c) for _ in range(c.num_hidden_layers)])
         self.final_norm = RMSNorm(c.hidden_size, eps=c.rms_norm_eps)
+        self.fused_head = False  # set by apply_triton_kernels(..., linear_down_o=True)
         cos, sin = build_rope_tables(c.head_dim, c.max_position_embeddings, c.rope_theta)
         self.register_buffer("rope_cos", cos, persistent=False)
         self.register_buffer("rope_sin", sin, persistent=False)
@@ -161,10 +163,11 @@ class Qwen3Model(nn.Module):
             sin = self.rope_sin[start_pos:start_pos + T]
         for i, layer in enumerate(self.layers):
             h = layer(h, kv_cache=kv_cache, layer_idx=i, cos=cos, sin=sin, start_pos=start_pos)
-        h = self.final_norm(h)
         if not torch.is_tensor(start_pos):
             kv_cache.cur_len = start_pos + T
-        return F.linear(h, self.embed.weight)  # tied head: h @ embed.weight.T
+        # final norm and tied head: norm(h) @ embed.weight.T
+        logits = fused_rmsnorm_head(h, self.final_norm, self.embed.weight) if self.fused_head else None
+        return F.linear(self.final_norm(h), self.embed.weight) if logits is None else logits
 
 
 def tiny_state(c: Cfg, *, seed: int = 0, embed_scale: float = 1.0) -> dict[str, torch.Tensor]:

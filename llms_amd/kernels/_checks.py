@@ -3,6 +3,10 @@
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
+from torch.nn.modules import module as _module
+
+from ._eager import RMSNorm
 
 
 def require_bf16_hip(fn: str, **tensors: torch.Tensor) -> None:
@@ -34,3 +38,16 @@ def inner_contiguous(t: torch.Tensor) -> torch.Tensor:
     if t.dim() >= 1 and t.shape[-1] > 1 and t.stride(-1) != 1:
         return t.contiguous()
     return t
+
+
+def plain_norm(m) -> bool:
+    """Whether m is the RMSNorm of ``_eager.py`` with nothing attached to its
+    call (a fused kernel may then normalise with its weight and eps)."""
+    return (type(m) is RMSNorm and not m._forward_hooks and not m._forward_pre_hooks
+            and not _module._global_forward_hooks and not _module._global_forward_pre_hooks)
+
+
+def differentiated(*tensors: torch.Tensor) -> bool:
+    """Whether autograd, in either mode, may follow an operation on these."""
+    return ((torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
+            or getattr(forward_ad, "_current_level", -1) >= 0)

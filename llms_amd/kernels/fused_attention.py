@@ -15,23 +15,9 @@ Path: wrapper -> ``torch.ops.llms_amd.attention`` -> C ABI
 from __future__ import annotations
 
 import torch
-from torch.autograd import forward_ad
-from torch.nn.modules import module as _module
 
 from .. import _lib
-from ._eager import RMSNorm
-
-
-def _plain_norm(m) -> bool:
-    """Whether m is the RMSNorm of ``_eager.py`` with nothing attached to its
-    call (the kernel then normalises with its weight and eps)."""
-    return (type(m) is RMSNorm and not m._forward_hooks and not m._forward_pre_hooks
-            and not _module._global_forward_hooks and not _module._global_forward_pre_hooks)
-
-
-def _differentiated(*tensors) -> bool:
-    return ((torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
-            or getattr(forward_ad, "_current_level", -1) >= 0)
+from ._checks import differentiated, plain_norm
 
 
 def attention_core(q, k, v, *, q_norm, k_norm, num_heads: int, cache_k, cache_v, cos, sin,
@@ -42,9 +28,9 @@ def attention_core(q, k, v, *, q_norm, k_norm, num_heads: int, cache_k, cache_v,
     max_seq, D]`` at ``start_pos`` (an int, or a 0-dim int64 device tensor) ..;
     None, with nothing written, where the kernels do not take the call."""
     if (not q.is_cuda or q.dtype != torch.bfloat16 or cache_k.shape[-1] not in (64, 128)
-            or not (_plain_norm(q_norm) and _plain_norm(k_norm))):
+            or not (plain_norm(q_norm) and plain_norm(k_norm))):
         return None
-    if _differentiated(q, k, v, q_norm.weight, k_norm.weight, cos, sin, cache_k, cache_v):
+    if differentiated(q, k, v, q_norm.weight, k_norm.weight, cos, sin, cache_k, cache_v):
         return None
     if torch.is_tensor(start_pos):
         pos, start = start_pos, 0

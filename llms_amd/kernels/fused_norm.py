@@ -18,7 +18,8 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ._checks import inner_contiguous, require_bf16_hip, require_device
+from ._checks import (differentiated, inner_contiguous, plain_norm, require_bf16_hip,
+                      require_device)
 
 
 def _check_norm(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, fn: str) -> None:
@@ -117,3 +118,17 @@ def fused_rmsnorm_gate_up_silu_w8(x: torch.Tensor, norm_weight: torch.Tensor, ep
                                            inner_contiguous(qg), sg.contiguous(),
                                            inner_contiguous(qu), su.contiguous())
     return y.reshape(*lead, N)
+
+
+def fused_rmsnorm_head(h: torch.Tensor, norm, W: torch.Tensor) -> torch.Tensor | None:
+    """``F.linear(norm(h), W)``, the final norm and output head of a model, on
+    the fused kernels at decode and verify row counts (up to 16 rows of h); None
+    for the calls that stay with torch: more rows (the library GEMM's), other
+    types and devices, gradients, a norm that is not the plain ``RMSNorm``. One
+    row of 4B, 151936 x 2560: 109 us against 240 for ``F.linear`` alone."""
+    if (not h.is_cuda or h.dtype != torch.bfloat16 or W.dtype != torch.bfloat16
+            or not 1 <= h.numel() <= 16 * h.shape[-1] or not plain_norm(norm)
+            or norm.weight.dtype != torch.bfloat16 or W.device != h.device
+            or differentiated(h, W, norm.weight)):
+        return None
+    return fused_rmsnorm_qkv(h, norm.weight, norm.eps, W, n_q=W.shape[0], n_k=0)[0]

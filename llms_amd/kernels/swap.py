@@ -39,8 +39,13 @@ def apply_triton_kernels(
     ``int8`` is set. ``fuse_norm=True`` (not in the reference) moves each
     block's ``norm1`` / ``norm2`` RMSNorm into the fused QKV / gate-up module
     (``prenorm``) and leaves ``nn.Identity`` in its place, so the norm runs
-    inside the projection call; the block's forward is unchanged.
+    inside the projection call; the block's forward is unchanged. A model with
+    a ``fused_head`` flag (``harness.Qwen3Model``) has it set by
+    ``linear_down_o=True``: its final norm and tied head then run as one fused
+    call at decode and verify row counts.
     """
+    if linear_down_o and getattr(model, "fused_head", None) is False:
+        model.fused_head = True
     for block in model.layers:
         if fused_ffn and not isinstance(block.ffn, TritonFFN):
             block.ffn = TritonFFN.from_eager(block.ffn, int8=int8)

@@ -269,3 +269,33 @@ def test_norm_in_rows_or_apart(M, K):
         ref.dequant_w8(qu.cpu().numpy(), su.cpu().numpy()))
     _check(y, out, f"int8 norm+gate-up M={M} K={K}")
     _check(y0.cpu(), out, f"int8 norm+gate-up M={M} K={K}, no workspace")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,V", [(1, 256, 40000), (2, 1024, 33000), (3, 2560, 8200), (8, 2560, 8201),
+                                   (9, 4096, 8320), (16, 1024, 10000), (17, 256, 9000),
+                                   (33, 256, 8300)])
+def test_norm_and_wide_head(M, K, V):
+    """The final norm and head of a model: wide outputs at the row counts where
+    their tile changes, against the oracle; past 16 rows, with gradients or a
+    hooked norm the helper leaves the call to torch."""
+    from llms_amd.kernels._eager import RMSNorm
+    from llms_amd.kernels.fused_norm import fused_rmsnorm_head
+
+    x, g = _x(70 + M, M, K), _norm_weight(71, K)
+    _, w = qkv_inputs(72, 1, K, V, 0)
+    norm = RMSNorm(K, eps=EPS).to(DEV, torch.bfloat16)
+    with torch.no_grad():
+        norm.weight.copy_(g)
+        xd, wd = x.to(DEV), w.to(DEV)
+        y = fused_rmsnorm_head(xd[None], norm, wd)
+        if M > 16:
+            assert y is None
+            y = _kern().fused_rmsnorm_qkv(xd, norm.weight, EPS, wd, n_q=V, n_k=0)[0][None]
+        assert y.shape == (1, M, V)
+        _check(y[0].cpu(), ref.ref_rmsnorm_qkv_full(bits(x), bits(g), EPS, bits(w), V, 0),
+               f"head M={M} K={K} V={V}")
+        h = norm.register_forward_hook(lambda *a: None)
+        assert fused_rmsnorm_head(xd[None], norm, wd) is None
+        h.remove()
+    assert fused_rmsnorm_head(xd[None], norm, wd) is None  # the weight is a parameter
