@@ -64,6 +64,7 @@ template <int NW, int MT, int U, int SPLIT, bool GATEUP, bool W8, bool ALIGNED, 
           bool XP = false>
 __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
   static_assert(!XP || (MT == 1 && !XL), "packed x needs M <= 8 and x from L2");
+  static_assert(ALIGNED || (!XL && SPLIT == 0), "unaligned rows: x from L2, interleaved k-blocks");
   using F = Frag<MT, GATEUP, W8, XP>;
   constexpr int XV = F::XV;
   constexpr int SV = W8 ? 2 : 1;           // 8-element sub-chunks per lane per line half
@@ -73,7 +74,9 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
   constexpr int NACC = 2 * MT * NM;        // [half][matrix][mt]
 
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
+  // (unaligned rows: as a scalar, for the uniform branches of load_block)
+  const int wave = ALIGNED ? (int)(threadIdx.x / kWave)
+                           : __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
   const int li = lane & 15;                // MFMA row (A) / column (B)
   const int grp = lane >> 4;               // MFMA k-group
   const int64_t n0 = (int64_t)blockIdx.x * 8;
@@ -81,7 +84,10 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
   const int chunk = 4 * ((lane >> 3) & 1) + grp;
   const bool row_ok = row < a.N;
   const int64_t K = a.K;
-  const int64_t nkb = (K + KB - 1) / KB;
+  // k-blocks of the main loop; for unaligned rows the whole ones only, and the
+  // one that crosses the row's end comes after the loop (with its element reads
+  // inside the loop the compiler kept the buffers in scratch memory)
+  const int64_t nkb = ALIGNED ? (K + KB - 1) / KB : K / KB;
 
   const int64_t rsafe = row_ok ? row : 0;
   const char* w0row = (const char*)a.w0 + rsafe * a.ldw0 * (W8 ? 1 : 2);
@@ -131,6 +137,21 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
     const int64_t kb = kb_first + j * kb_stride;
     const int64_t kw = kb * KB + chunk * CK;
     const u32x4 z{0, 0, 0, 0};
+    if constexpr (!ALIGNED) {
+      // plain loads of any alignment, without a branch per load (rows and
+      // columns past the last are row 0 again, never stored)
+      if (!live) return;
+      f.a0 = ld16_any(w0row + kw * (W8 ? 1 : 2));
+      if constexpr (GATEUP) f.a1 = ld16_any(w1row + kw * (W8 ? 1 : 2));
+      if constexpr (!XL) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int v = 0; v < XV; ++v)
+            f.xb[mt][v] = ld16_any(xrow[mt] + xk(kb, XP ? xhalf : v / SV, XP ? v : v % SV));
+      }
+      return;
+    }
     if constexpr (W8) {
       f.a0 = (live && row_ok) ? load_w_i8x16<ALIGNED>((const int8_t*)w0row, kw, K) : z;
       if constexpr (GATEUP)
@@ -268,6 +289,27 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
     if (c + 3 < nchunks) load_chunk(fb, c + 3);
   }
 
+  // The k-block that crosses the row's end: the last one of its wave.
+  if constexpr (!ALIGNED) {
+    if (nkb * KB < K && wave == (int)(nkb % NW)) {
+      F f;
+      const int64_t kw = nkb * KB + chunk * CK;
+      if constexpr (W8) {
+        f.a0 = load_i8x16<false>((const int8_t*)w0row, kw, K);
+        if constexpr (GATEUP) f.a1 = load_i8x16<false>((const int8_t*)w1row, kw, K);
+      } else {
+        f.a0 = load_bf16x8<false>((const uint16_t*)w0row, kw, K);
+        if constexpr (GATEUP) f.a1 = load_bf16x8<false>((const uint16_t*)w1row, kw, K);
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int v = 0; v < XV; ++v)
+          f.xb[mt][v] = load_bf16x8<false>(xrow[mt], xk(nkb, XP ? xhalf : v / SV, XP ? v : v % SV), K);
+      compute_block(f, 0);
+    }
+  }
+
   // Fixed-order cross-wave reduction through LDS.
   __shared__ f32x4 red[NW > 1 ? NW - 1 : 1][NACC][kWave];
   if constexpr (NW > 1) {
@@ -381,13 +423,20 @@ int launch_stream(const StreamArgs& a, bool aligned, hipStream_t s) {
   const int64_t min_m = GATEUP && wrows > kSplitkSmallN ? (a.K > 3072 ? 4 : 6) : kSplitkMinM;
   if (!W8 && a.M >= min_m && splitk_supported(a, aligned, false))
     return launch_splitk<GATEUP, false>(a, s);
+  // More x rows than a wave's registers stream well (rows or K that the kernels
+  // above do not take): the general tiles from 33 rows, and from 9 for unaligned
+  // gate-up over at least 8192 weight rows, whose 32-row tiles fill the chip. One
+  // box, us, stream / 32 x 32 tiles: gate-up N = 9700, K = 2541 at 16 (int8), 20,
+  // 40 rows 55 / 44, 78 / 38, 121 / 51, N = 4800 at 4, 16 rows 32 / 38, 47 / 39; K =
+  // 2056 (aligned) at 16, 64 rows 27 / 29, 66 / 58; 6100 columns, K = 3001 at 16
+  // rows 36 / 37, 2541 columns at 20, 64 rows 30 / 37, 69 / 37.
+  if (a.M > 32 || (!aligned && GATEUP && a.M > 8 && wrows >= kSplitkSmallN))
+    return launch_tiled<GATEUP, W8>(a, aligned, s);
   // (int8 dequantisation needs registers of its own: 2 k-blocks per buffer)
   constexpr int U8 = (GATEUP && !W8) ? 4 : 2;
   if (a.M <= 8) return launch_stream_cfg<4, 1, U8, 0, GATEUP, W8, false, true>(a, aligned, s);
   if (a.M <= 16) return launch_stream_cfg<4, 1, 2, 0, GATEUP, W8, false>(a, aligned, s);
-  if (a.M <= 32) return launch_stream_cfg<4, 2, 2, 0, GATEUP, W8, false>(a, aligned, s);
-  if (a.M <= 48) return launch_stream_cfg<4, 3, 2, 0, GATEUP, W8, false>(a, aligned, s);
-  return launch_stream_cfg<4, 4, 1, 0, GATEUP, W8, false>(a, aligned, s);
+  return launch_stream_cfg<4, 2, 2, 0, GATEUP, W8, false>(a, aligned, s);
 }
 
 template int launch_stream<false, false>(const StreamArgs&, bool, hipStream_t);

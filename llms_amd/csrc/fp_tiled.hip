@@ -10,8 +10,10 @@
 //     in adjacent accumulators and silu(g)*u is applied in registers.
 //   - int8 weights are dequantised (w = bf16(q * s)) on the way into LDS, so
 //     the MFMA loop is the bf16 one.
-//   - Global -> register prefetch of k-step t+1 overlaps the MFMAs of step t;
-//     two LDS buffers, one barrier per k-step.
+//   - Loads run D k-steps ahead through D register sets (their latency is
+//     several steps of compute); two LDS buffers, one barrier per k-step.
+//   - Rows of any alignment are read 16 bytes at a time; the k-step that crosses
+//     the rows' end comes after the loop.
 #include "fp_common.h"
 #include "fp_launch.h"
 
@@ -21,7 +23,7 @@ namespace {
 
 constexpr int kPad = 8;  // bf16 elements of padding per LDS row (16 B)
 
-template <int BN, int BM, int BK, int WN, int WM, bool GATEUP, bool W8, bool ALIGNED>
+template <int BN, int BM, int BK, int WN, int WM, int D, bool GATEUP, bool W8, bool ALIGNED>
 __global__ __launch_bounds__(WN * WM * kWave) void tiled_kernel(StreamArgs a) {
   constexpr int NT = WN * WM * kWave;
   constexpr int TN = BN / WN, TM = BM / WM;   // per-wave tile
@@ -32,7 +34,6 @@ __global__ __launch_bounds__(WN * WM * kWave) void tiled_kernel(StreamArgs a) {
   constexpr int CX = BM * BK / 8 / NT;        // x chunks per thread per k-step
   static_assert(BN * BK / WCH % NT == 0 && BM * BK / 8 % NT == 0, "tile/threads");
   static_assert(!GATEUP || TN % 32 == 0, "gate-up needs whole gate/up pairs per wave");
-
   __shared__ __attribute__((aligned(16))) uint16_t sW[2][BN][LDP];
   __shared__ __attribute__((aligned(16))) uint16_t sX[2][BM][LDP];
 
@@ -90,33 +91,46 @@ __global__ __launch_bounds__(WN * WM * kWave) void tiled_kernel(StreamArgs a) {
     xsrc[j] = a.x + (xok[j] ? m : 0) * a.ldx;
   }
 
-  u32x4 rw[CW], rx[CX];
-  auto gload = [&](int64_t k0) {
+  // D register sets: the loads of k-steps k + 1 .. k + D are in flight or landed
+  // while step k is computed (a memory latency is several steps of these tiles)
+  u32x4 rw[D][CW], rx[D][CX];
+  // a whole k-step: no branch per load (rows past the last are row 0 again, their
+  // outputs never stored)
+  auto gload = [&](u32x4 (&w)[CW], u32x4 (&x)[CX], int64_t k0) {
 #pragma unroll
     for (int j = 0; j < CW; ++j) {
-      const int64_t k = k0 + wk_l[j];
-      if constexpr (W8)
-        rw[j] = wok[j] ? load_i8x16<ALIGNED>((const int8_t*)wsrc[j], k, K) : u32x4{0, 0, 0, 0};
-      else
-        rw[j] = wok[j] ? load_bf16x8<ALIGNED>((const uint16_t*)wsrc[j], k, K) : u32x4{0, 0, 0, 0};
+      const char* p = wsrc[j] + (k0 + wk_l[j]) * (W8 ? 1 : 2);
+      w[j] = ALIGNED ? ld16(p) : ld16_any(p);
     }
 #pragma unroll
-    for (int j = 0; j < CX; ++j)
-      rx[j] = xok[j] ? load_bf16x8<ALIGNED>(xsrc[j], k0 + xk_l[j], K) : u32x4{0, 0, 0, 0};
+    for (int j = 0; j < CX; ++j) {
+      const uint16_t* p = xsrc[j] + k0 + xk_l[j];
+      x[j] = ALIGNED ? ld16(p) : ld16_any(p);
+    }
   };
-  auto sstore = [&](int buf) {
+  // the k-step that crosses the rows' end: zeros past it
+  auto gload_tail = [&](u32x4 (&w)[CW], u32x4 (&x)[CX], int64_t k0) {
+#pragma unroll
+    for (int j = 0; j < CW; ++j) {
+      if constexpr (W8) w[j] = load_i8x16<ALIGNED>((const int8_t*)wsrc[j], k0 + wk_l[j], K);
+      else w[j] = load_bf16x8<ALIGNED>((const uint16_t*)wsrc[j], k0 + wk_l[j], K);
+    }
+#pragma unroll
+    for (int j = 0; j < CX; ++j) x[j] = load_bf16x8<ALIGNED>(xsrc[j], k0 + xk_l[j], K);
+  };
+  auto sstore = [&](int buf, const u32x4 (&w)[CW], const u32x4 (&x)[CX]) {
 #pragma unroll
     for (int j = 0; j < CW; ++j) {
       if constexpr (W8) {
         const float s = wsc[j], n128s = -128.f * s;
-        *reinterpret_cast<u32x4*>(&sW[buf][wrow_l[j]][wk_l[j]]) = dequant8(rw[j].x, rw[j].y, s, n128s);
-        *reinterpret_cast<u32x4*>(&sW[buf][wrow_l[j]][wk_l[j] + 8]) = dequant8(rw[j].z, rw[j].w, s, n128s);
+        *reinterpret_cast<u32x4*>(&sW[buf][wrow_l[j]][wk_l[j]]) = dequant8(w[j].x, w[j].y, s, n128s);
+        *reinterpret_cast<u32x4*>(&sW[buf][wrow_l[j]][wk_l[j] + 8]) = dequant8(w[j].z, w[j].w, s, n128s);
       } else {
-        *reinterpret_cast<u32x4*>(&sW[buf][wrow_l[j]][wk_l[j]]) = rw[j];
+        *reinterpret_cast<u32x4*>(&sW[buf][wrow_l[j]][wk_l[j]]) = w[j];
       }
     }
 #pragma unroll
-    for (int j = 0; j < CX; ++j) *reinterpret_cast<u32x4*>(&sX[buf][xrow_l[j]][xk_l[j]]) = rx[j];
+    for (int j = 0; j < CX; ++j) *reinterpret_cast<u32x4*>(&sX[buf][xrow_l[j]][xk_l[j]]) = x[j];
   };
 
   f32x4 acc[FN][FM];
@@ -124,14 +138,7 @@ __global__ __launch_bounds__(WN * WM * kWave) void tiled_kernel(StreamArgs a) {
   for (int i = 0; i < FN; ++i)
 #pragma unroll
     for (int j = 0; j < FM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int64_t nkt = (K + BK - 1) / BK;
-  gload(0);
-  sstore(0);
-  __syncthreads();
-  for (int64_t kt = 0; kt < nkt; ++kt) {
-    const int buf = (int)(kt & 1);
-    if (kt + 1 < nkt) gload((kt + 1) * BK);
+  auto compute = [&](int buf) {
 #pragma unroll
     for (int kk = 0; kk < BK / 32; ++kk) {
       u32x4 fa[FN], fb[FM];
@@ -146,8 +153,31 @@ __global__ __launch_bounds__(WN * WM * kWave) void tiled_kernel(StreamArgs a) {
 #pragma unroll
         for (int j = 0; j < FM; ++j) acc[i][j] = mfma16(fa[i], fb[j], acc[i][j]);
     }
-    if (kt + 1 < nkt) sstore(buf ^ 1);
+  };
+
+  const int64_t nkt = K / BK;  // whole k-steps
+#pragma unroll
+  for (int u = 0; u < D; ++u)
+    if (u < nkt) gload(rw[u], rx[u], (int64_t)u * BK);
+  if (nkt > 0) sstore(0, rw[0], rx[0]);
+  __syncthreads();
+  for (int64_t kt = 0; kt < nkt; kt += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) {
+      const int64_t k = kt + u;  // in LDS buffer k % 2; its register set is free
+      if (k >= nkt) break;
+      if (k + D < nkt) gload(rw[u], rx[u], (k + D) * BK);
+      const int buf = D % 2 == 0 ? u & 1 : (int)(k & 1);
+      compute(buf);
+      if (k + 1 < nkt) sstore(buf ^ 1, rw[(u + 1) % D], rx[(u + 1) % D]);
+      __syncthreads();
+    }
+  }
+  if (nkt * BK < K) {
+    gload_tail(rw[0], rx[0], nkt * BK);
+    sstore(0, rw[0], rx[0]);  // every wave is past its last read
     __syncthreads();
+    compute(0);
   }
 
   // ---- epilogue ----
@@ -192,15 +222,15 @@ __global__ __launch_bounds__(WN * WM * kWave) void tiled_kernel(StreamArgs a) {
   }
 }
 
-template <int BN, int BM, int BK, int WN, int WM, bool GATEUP, bool W8>
+template <int BN, int BM, int BK, int WN, int WM, int D, bool GATEUP, bool W8>
 int launch_cfg(const StreamArgs& a, bool aligned, hipStream_t s) {
   const int64_t cols = GATEUP ? BN / 2 : BN;
   const dim3 grid((unsigned)((a.N + cols - 1) / cols), (unsigned)((a.M + BM - 1) / BM));
   const dim3 block(WN * WM * kWave);
   if (aligned)
-    hipLaunchKernelGGL((tiled_kernel<BN, BM, BK, WN, WM, GATEUP, W8, true>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((tiled_kernel<BN, BM, BK, WN, WM, D, GATEUP, W8, true>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((tiled_kernel<BN, BM, BK, WN, WM, GATEUP, W8, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((tiled_kernel<BN, BM, BK, WN, WM, D, GATEUP, W8, false>), grid, block, 0, s, a);
   return (int)hipGetLastError();
 }
 
@@ -235,7 +265,16 @@ int launch_tiled(const StreamArgs& a, bool aligned, hipStream_t s) {
   // int8 that reaches here either suits the in-register gemm or had no
   // workspace to dequantise into: gemm_kernel either way
   if (W8 && gemm_supported(a, aligned, true)) return launch_gemm<GATEUP, true>(a, s);
-  return launch_cfg<128, 128, 64, 2, 2, GATEUP, W8>(a, aligned, s);
+  // The general tiles: 128 x 128 where they give a workgroup for every CU, then
+  // 64 x 64, then (few rows or narrow outputs) 32 x 32. One box, us, K = 2541 or
+  // 3001, 128 x 128 / 64 x 64 / 32 x 32: gate-up N = 9700 at 300 rows 75 / 121 /
+  // 199, at 100 68 / 62 / 97, at 20 - / 44 / 38; 2541 columns at 1000 rows 59 / 51 /
+  // 85, at 128 75 / 45 / 37; 6000 columns at 200 rows 46 / 31 / 34.
+  const auto count = [&](int64_t t) { return ((wrows + t - 1) / t) * ((a.M + t - 1) / t); };
+  if (a.M <= 32 || (count(128) < 256 && count(64) < 192))
+    return launch_cfg<32, 32, 64, 1, 2, 4, GATEUP, W8>(a, aligned, s);
+  if (count(128) < 256) return launch_cfg<64, 64, 64, 2, 2, 4, GATEUP, W8>(a, aligned, s);
+  return launch_cfg<128, 128, 64, 2, 2, 1, GATEUP, W8>(a, aligned, s);
 }
 
 template int launch_tiled<false, false>(const StreamArgs&, bool, hipStream_t);

@@ -1148,3 +1148,35 @@ def test_narrow_outputs(M, K, N):
     _check(y8.cpu(), ref.ref_linear(bits(x), wq), f"narrow int8 M={M} K={K} N={N}")
     assert torch.equal(kern.fused_linear(xd[:, :K], wd), y)
     assert torch.equal(kern.fused_linear_w8(xd[:, :K], q, s), y8)
+
+
+# (M, K, N): k tails of every kind against 64-wide (int8 128-wide) steps, rows at any
+# byte, on the streaming kernel (to 32 rows) and the 32 x 32, 64 x 64 and 128 x 128
+# tiles, at their row counts' edges and with partial tiles both ways
+RAGGED = [(1, 1, 5), (1, 63, 33), (2, 65, 40), (3, 127, 129), (8, 129, 100), (9, 200, 4100),
+          (16, 2541, 70), (17, 255, 65), (32, 513, 31), (33, 64 * 3 + 1, 200), (48, 71, 33),
+          (64, 1000, 130), (65, 137, 6200), (100, 193, 4200), (130, 321, 8300), (300, 130, 5000)]
+
+
+@pytest.mark.parametrize("M,K,N", RAGGED)
+def test_rows_of_any_alignment(M, K, N):
+    """K that no vector width divides and x rows that start at odd elements
+    (a view at offset 1 of wider rows), bf16 and int8, linear and gate-up; the
+    bytes past each row hold NaN, so a value read past a row's end would show."""
+    kern = _kernels()
+
+    def at_odd(t):
+        wide = torch.full((t.shape[0], K + 3), float("nan"), dtype=torch.bfloat16, device=DEV)
+        wide[:, 1:K + 1] = t.to(DEV)
+        return wide[:, 1:K + 1]
+
+    x, wg, wu = ffn_inputs(900 + M + K, M, K, N, w_std=0.05)
+    xd, gd, ud = at_odd(x), at_odd(wg), at_odd(wu)
+    _check(kern.fused_linear(xd, gd).cpu(), ref.ref_linear(bits(x), bits(wg)), "linear")
+    _check(kern.triton_fused_gate_up_silu(xd, gd, ud).cpu(),
+           ref.ref_gate_up_silu_full(bits(x), bits(wg), bits(wu)), "gate-up")
+    (qg, sg), (qu, su) = (kern.quantize_w8_per_row(w.to(DEV)) for w in (wg, wu))
+    dg, du = (ref.dequant_w8(q.cpu().numpy(), s.cpu().numpy()) for q, s in ((qg, sg), (qu, su)))
+    _check(kern.fused_linear_w8(xd, qg, sg).cpu(), ref.ref_linear(bits(x), dg), "int8 linear")
+    _check(kern.fused_gate_up_silu_w8(xd, qg, sg, qu, su).cpu(),
+           ref.ref_gate_up_silu_full(bits(x), dg, du), "int8 gate-up")
