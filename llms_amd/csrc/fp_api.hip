@@ -34,6 +34,71 @@ __global__ __launch_bounds__(256) void quantize_w8_kernel(const uint16_t* w, int
   }
 }
 
+// The same with the row in registers, 16 bytes per load (one pass over memory
+// instead of two of 2-byte loads). A row that starts off a 16-byte boundary is
+// cut into chunks at those boundaries, the partial ones at its two ends read and
+// stored by elements, so loads are aligned for any K and stride; the int8 chunks
+// are stored as they fall, 8 bytes at any address. Bit-identical (a maximum, and
+// the same division and rounding per element). Measured on MI355X, 12288 x 4096
+// 103.9 -> 37.9 us (4.0 TB/s), 6409 x 10234 134 -> 62.6, 9728 x 2560 38.7 -> 20.7.
+// NV chunks of 8 elements per thread: rows of up to 2048 NV - 7 elements.
+template <int NV>
+__global__ __launch_bounds__(256) void quantize_w8_row_kernel(const uint16_t* w, int64_t ldw,
+                                                              int8_t* q, int64_t ldq, float* scale,
+                                                              int K) {
+  const int64_t r = blockIdx.x;
+  const uint16_t* wr = w + r * ldw;
+  const int off = (int)((reinterpret_cast<uintptr_t>(wr) & 15) / 2);  // elements past a boundary
+  u32x4 v[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int k = ((int)threadIdx.x + 256 * i) * 8 - off;  // element of the chunk's first
+    v[i] = u32x4{0u, 0u, 0u, 0u};
+    if (k >= 0 && k + 8 <= K) {
+      v[i] = ld16(wr + k);
+    } else if (k < K) {  // the row's two ends
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (k + e >= 0 && k + e < K) v[i][e / 2] |= (uint32_t)wr[k + e] << (16 * (e & 1));
+    }
+  }
+  float mx = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      mx = fmaxf(mx, fmaxf(fabsf(bf16_bits_to_f32(v[i][d] & 0xffffu)), fabsf(bf16_bits_to_f32(v[i][d] >> 16))));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  __shared__ float part[4];
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+  const float s = mx / 127.0f;
+  if (threadIdx.x == 0) scale[r] = s;
+  int8_t* qr = q + r * ldq;
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int k = ((int)threadIdx.x + 256 * i) * 8 - off;
+    if (k >= K) continue;
+    uint32_t b[2] = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint32_t h = e & 1 ? v[i][e / 2] >> 16 : v[i][e / 2] & 0xffffu;
+      float f = 0.f;
+      if (s > 0.f) f = fminf(fmaxf(rintf(bf16_bits_to_f32(h) / s), -127.f), 127.f);
+      b[e / 4] |= (uint32_t)(uint8_t)(int8_t)(int)f << (8 * (e % 4));
+    }
+    if (k >= 0 && k + 8 <= K) {
+      __builtin_memcpy(qr + k, b, 8);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (k + e >= 0 && k + e < K) qr[k + e] = (int8_t)(b[e / 4] >> (8 * (e % 4)));
+    }
+  }
+}
+
 inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // rc is the hipError_t of the launch (hipGetLastError right after it).
@@ -479,8 +544,22 @@ int fp_quantize_w8_per_row(const void* w, int64_t ldw, int8_t* q, int64_t ldq, f
   if (ldw < K || ldq < K) return FP_ERR_STRIDE;
   if (N == 0) return FP_OK;
   if (!w || !q || !scale) return FP_ERR_NULL;
-  hipLaunchKernelGGL(fp::quantize_w8_kernel, dim3((unsigned)N), dim3(256), 0,
-                     (hipStream_t)stream, (const uint16_t*)w, ldw, q, ldq, scale, K);
+  const dim3 grid((unsigned)N), block(256);
+  const hipStream_t hs = (hipStream_t)stream;
+  const uint16_t* wp = (const uint16_t*)w;
+  // rows of more than 8 chunks per thread, and bases off an element boundary
+  if (K > 8 * 2048 - 7 || (reinterpret_cast<uintptr_t>(w) & 1))
+    hipLaunchKernelGGL(fp::quantize_w8_kernel, grid, block, 0, hs, wp, ldw, q, ldq, scale, K);
+  else if (K <= 2048 - 7)
+    hipLaunchKernelGGL(fp::quantize_w8_row_kernel<1>, grid, block, 0, hs, wp, ldw, q, ldq, scale, (int)K);
+  else if (K <= 2 * 2048 - 7)
+    hipLaunchKernelGGL(fp::quantize_w8_row_kernel<2>, grid, block, 0, hs, wp, ldw, q, ldq, scale, (int)K);
+  else if (K <= 3 * 2048 - 7)
+    hipLaunchKernelGGL(fp::quantize_w8_row_kernel<3>, grid, block, 0, hs, wp, ldw, q, ldq, scale, (int)K);
+  else if (K <= 5 * 2048 - 7)
+    hipLaunchKernelGGL(fp::quantize_w8_row_kernel<5>, grid, block, 0, hs, wp, ldw, q, ldq, scale, (int)K);
+  else
+    hipLaunchKernelGGL(fp::quantize_w8_row_kernel<8>, grid, block, 0, hs, wp, ldw, q, ldq, scale, (int)K);
   return fp::launch_status((int)hipGetLastError());
 }
 

@@ -1180,3 +1180,24 @@ def test_rows_of_any_alignment(M, K, N):
     _check(kern.fused_linear_w8(xd, qg, sg).cpu(), ref.ref_linear(bits(x), dg), "int8 linear")
     _check(kern.fused_gate_up_silu_w8(xd, qg, sg, qu, su).cpu(),
            ref.ref_gate_up_silu_full(bits(x), dg, du), "int8 gate-up")
+
+
+@pytest.mark.parametrize("K", [1, 7, 8, 15, 16, 255, 2041, 2042, 4089, 4090, 6137, 6138, 10233, 10234,
+                               16377, 16378])
+def test_quantise_rows_of_any_size_and_alignment(K):
+    """Row lengths on both sides of each chunk count per thread, the rows
+    contiguous (an odd K moves each row's start) and as views at every offset of
+    wider rows (NaN beside them), bit for bit."""
+    rng = np.random.default_rng(K)
+    w = torch.from_numpy(rng.normal(0, 0.02, (19, K)).astype(np.float32)).bfloat16()
+    w[3] = 0
+    qo, so = ref.quantize_w8_per_row(bits(w))
+    for off in [None, *range(8)]:
+        if off is None:
+            wd = w.to(DEV)
+        else:
+            wide = torch.full((19, K + 9), float("nan"), dtype=torch.bfloat16, device=DEV)
+            wide[:, off:off + K] = w.to(DEV)
+            wd = wide[:, off:off + K]
+        q, s = _kernels().quantize_w8_per_row(wd)
+        assert np.array_equal(q.cpu().numpy(), qo) and np.array_equal(s.cpu().numpy(), so), off
