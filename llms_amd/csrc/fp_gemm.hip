@@ -395,8 +395,27 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_kernel(StreamArgs a, int
 // may take three or four LDS stages (NS), and then (SPLIT) contract one
 // range of k-steps per work item into fp32 partials for
 // splitk_reduce_kernel, as gemm_kernel's split form does.
+// W3 (four waves, 64-wide steps): three stages of weight rows and two of x, one
+// load instruction at a time between the MFMAs of the whole step. With one wave
+// per SIMD a burst of LDS-DMA instructions holds back the MFMAs behind it (each
+// occupies the wave's issue for the time its 64 addresses take), so the loads
+// are spread: while a step's first half computes, the weights of step k + 2 go
+// out (their stage was last read in step k - 1), and while its second half
+// computes, the x rows of step k + 2 (theirs is free after the step's barrier).
+// Both have half a step to a step and a half to land, the weights more, and the
+// third weight stage is what the LDS holds at 256 x 256 (160 KB). The next
+// half's fragment reads go out over the first three quarters of a half, so the
+// barrier never waits for one. Bound: with the loads reading nothing (a timing
+// copy) 8B gate-up at 4096 rows takes 424 us; so the rest to 575 is the wait for
+// the operands' L2 -> LDS stream. Same k order: bit-identical to the other tiles.
+// One box, us, the eight-wave or two-stage tiles -> W3: 4B QKV M = 2048 (192 x 256)
+// 58.6 -> 52.5 (1.23 PFLOP/s), 8B QKV M = 4096 180 -> 159, gate-up M = 4096 (256 x
+// 256) 634 -> 575 (1.43), down M = 4096 311 -> 274 (1.51), 4B o M = 2048 (160 x 128)
+// 44.5 -> 39.9. Spreading alone, two stages each: 8B gate-up 577-585 (with the
+// loads in one burst 643), 4B QKV 57; a load every second or every MFMA 605, 631;
+// three stages of both operands with all loads in the second half: 4B o 43.5.
 template <int BN, int BM, int WN, int WM, bool GATEUP, bool W8, int BK = kBK, int NS = 2,
-          bool SPLIT = false>
+          bool SPLIT = false, bool W3 = false>
 __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs a, int n_mt,
                                                                     int n_nt, int nsplit,
                                                                     int per, float* ws) {
@@ -420,6 +439,8 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
                 "32-wide k-substeps: two per k-step, or four with four bf16 waves");
   static_assert(NS == 2 || ((NS == 3 || NS == 4) && WN * WM == 4 && !W8),
                 "three or four LDS stages: four bf16 waves");
+  static_assert(!W3 || (NS == 2 && BK == 64 && WN * WM == 4 && !W8 && !SPLIT),
+                "three weight stages: 64-wide steps, four bf16 waves, unsplit");
   static_assert(!SPLIT || NS > 2, "k split across workgroups: the staged four-wave loop");
   static_assert(BN % WRPI == 0 && BM % (RPI * NW) == 0, "tile/waves");
   static_assert(W8 || NWI % NW == 0, "bf16 weight loads spread evenly over the waves");
@@ -432,7 +453,7 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
   // int8 the raw weight rows of the next k-steps
   __shared__ __attribute__((aligned(1024))) uint16_t sW0[BN][BK];
   __shared__ __attribute__((aligned(1024))) uint16_t sW1[BN][BK];
-  __shared__ __attribute__((aligned(1024))) uint16_t sW2[NS > 2 ? BN : 1][BK];
+  __shared__ __attribute__((aligned(1024))) uint16_t sW2[NS > 2 || W3 ? BN : 1][BK];
   __shared__ __attribute__((aligned(1024))) uint16_t sW3[NS > 3 ? BN : 1][BK];
   __shared__ __attribute__((aligned(1024))) uint16_t sX0[BM][BK];
   __shared__ __attribute__((aligned(1024))) uint16_t sX1[BM][BK];
@@ -523,6 +544,17 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
                  (uint32_t)((kb * BK + k0) * WB));
     }
   };
+  auto issue_w1 = [&](void* dst, int j, int64_t k0, bool live) {
+    const int q = wave + NW * j;
+    const bool up = wrow_up(q * WRPI);
+    load_lds16(up ? wptr1 : a.w0, live ? (up ? wbytes1 : wbytes0) : 0,
+               (lds_ptr_t)((char*)dst + q * WRPI * BK * WB), woff[j], (uint32_t)((kb * BK + k0) * WB));
+  };
+  auto issue_x1 = [&](uint16_t (*tx)[BK], int j, int64_t k0, bool live) {
+    load_lds16(a.x, live ? xbytes : 0, (lds_ptr_t)&tx[(wave + NW * j) * RPI][0], xoff[j],
+               (uint32_t)((kb * BK + k0) * 2));
+  };
+  auto nothing = [](int) {};
   auto issue_x = [&](uint16_t (*tx)[BK], int64_t k0, bool live = true) {
 #pragma unroll
     for (int j = 0; j < IX; ++j)
@@ -564,6 +596,13 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
     const uint32_t ob = offb ^ (uint32_t)(kk * 64);
     f.b[j] = *reinterpret_cast<const u32x4*>((const char*)tx + ob + j * 16 * BK * 2);
   };
+  // read r of a k-half, in the order in which the half's MFMAs first need them:
+  // weight fragment 0, every x fragment, the other weight fragments
+  auto rd_slot = [&](Frag& f, const uint16_t (*tw)[BK], const uint16_t (*tx)[BK], int kk, int r) {
+    if (r == 0) rd_a(f, tw, kk, 0);
+    else if (r <= FM) rd_b(f, tx, kk, r - 1);
+    else rd_a(f, tw, kk, r - FM);
+  };
   // Wave tiles of up to 24 MFMA blocks (192 x 256) keep the plain loop: all
   // of a k-half's reads, then its MFMAs (measured on MI355X, 4B QKV at M =
   // 2048: 60.1 us against 61.6 pipelined; gate-up 320 x 256 175.7 -> 169.5).
@@ -583,7 +622,7 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
   // writes in the middle of the block.
   auto mma = [&](auto RD, auto DQ, const Frag& f, Frag& g, const uint16_t (*tw)[BK],
                  const uint16_t (*tx)[BK], int kk, const uint8_t (*sq)[BK],
-                 uint16_t (*dw)[BK]) {
+                 uint16_t (*dw)[BK], auto&& between) {
     constexpr bool rd = decltype(RD)::value;
     constexpr bool dq = decltype(DQ)::value;
     u32x4 qv[QCH];
@@ -603,10 +642,20 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
                        : "v"(f.a[i]), "v"(f.b[j]));
         else
           acc[i][j] = mfma16(f.a[i], f.b[j], acc[i][j]);
-        if constexpr (rd)
+        if constexpr (rd && NW == 4) {
+          // four waves: the next half's reads over the first three quarters
+          const int n = i * FM + j;
+          constexpr int RG = FN * FM * 3 / 4 / (FN + FM) < 1 ? 1 : FN * FM * 3 / 4 / (FN + FM);
+          if (n % RG == 0 && n / RG < FN + FM) rd_slot(g, tw, tx, kk, n / RG);
+          if (n == FN * FM - 1)
+#pragma unroll
+            for (int r = n / RG + 1; r < FN + FM; ++r) rd_slot(g, tw, tx, kk, r);
+        } else if constexpr (rd) {
           if (i == FN - 1) rd_b(g, tx, kk, j);
+        }
+        between(i * FM + j);
       }
-      if constexpr (rd) rd_a(g, tw, kk, i);
+      if constexpr (rd && NW != 4) rd_a(g, tw, kk, i);
       if constexpr (dq) {
         if (i == FN / 2) {
 #pragma unroll
@@ -615,7 +664,7 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
         }
       }
     }
-    if constexpr (rd && !dq) {
+    if constexpr (rd && !dq && NW != 4) {
 #pragma unroll
       for (int i = 0; i < FN - 1; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, FM, 0);
@@ -732,17 +781,43 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
         // otherwise wait for all of them before the next stage's reads).
         constexpr int LPS = IW + IX;  // load instructions per wave and k-step
         static_assert((NS - 2) * LPS < 64, "loads in flight within the vmcnt range");
+        if constexpr (W3) {
+          // step k: weight stage k % 3, x stage k % 2; any step count
+          constexpr int GW = FN * FM / IW, GX = FN * FM / IX;
+          static_assert(GW >= 1 && GX >= 1, "a load or none per MFMA");
+          for (int64_t kt = 0; kt < nloc; kt += 6) {
+#pragma unroll
+            for (int u = 0; u < 6; ++u) {
+              const int64_t k = kt + u;
+              if (k >= nloc) break;
+              const bool live = k + 2 < nloc;
+              const int64_t kn = live ? (k + 2) * BK : 0;
+              mma(std::true_type{}, std::false_type{}, F, G, stw(u % 3), stx(u % 2), 1, sQ0, sW0,
+                  [&](int n) {
+                    if (n % GW == 0 && n / GW < IW) issue_w1(stw((u + 2) % 3), n / GW, kn, live);
+                  });
+              // step k + 1 has landed (the weights of k + 2 may be in flight)
+              // and this wave's reads of step k are done
+              __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(IW));
+              __builtin_amdgcn_s_barrier();
+              mma(std::true_type{}, std::false_type{}, G, F, stw((u + 1) % 3), stx((u + 1) % 2), 0,
+                  sQ0, sW0, [&](int n) {
+                    if (n % GX == 0 && n / GX < IX) issue_x1(stx(u % 2), n / GX, kn, live);
+                  });
+            }
+          }
+        } else
         for (int64_t kt = 0; kt < nloc; kt += NS) {
 #pragma unroll
           for (int u = 0; u < NS; ++u) {
             const int64_t k = kt + u;
             if constexpr (NS > 2)
               if (k >= nloc) break;
-            mma(std::true_type{}, std::false_type{}, F, G, stw(u), stx(u), 1, sQ0, sW0);
+            mma(std::true_type{}, std::false_type{}, F, G, stw(u), stx(u), 1, sQ0, sW0, nothing);
             if constexpr (BK == 128) {
               // substeps 1 and 2 of the four, each reading the next
-              mma(std::true_type{}, std::false_type{}, G, F, stw(u), stx(u), 2, sQ0, sW0);
-              mma(std::true_type{}, std::false_type{}, F, G, stw(u), stx(u), 3, sQ0, sW0);
+              mma(std::true_type{}, std::false_type{}, G, F, stw(u), stx(u), 2, sQ0, sW0, nothing);
+              mma(std::true_type{}, std::false_type{}, F, G, stw(u), stx(u), 3, sQ0, sW0, nothing);
             }
             if constexpr (NS > 2) {
               // this wave's loads of step k + 1 have landed and its reads of
@@ -754,16 +829,17 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
               __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
               __syncthreads();
             }
+            const bool live = k + NS < nloc;
+            const int64_t kn = live ? (k + NS) * BK : 0;
             if constexpr (NS > 2) {
-              const bool live = k + NS < nloc;
-              issue_x(stx(u), live ? (k + NS) * BK : 0, live);
-              issue_w(stw(u), live ? (k + NS) * BK : 0, live);
-            } else if (k + NS < nloc) {
-              issue_x(stx(u), (k + NS) * BK);
-              issue_w(stw(u), (k + NS) * BK);
+              issue_x(stx(u), kn, live);
+              issue_w(stw(u), kn, live);
+            } else if (live) {
+              issue_x(stx(u), kn);
+              issue_w(stw(u), kn);
             }
             mma(std::true_type{}, std::false_type{}, G, F, stw((u + 1) % NS), stx((u + 1) % NS), 0,
-                sQ0, sW0);
+                sQ0, sW0, nothing);
           }
         }
       } else
@@ -773,7 +849,7 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
           const int64_t k = kt + u;
           if (k >= nkt) break;
           mma(std::true_type{}, std::integral_constant<bool, W8>{}, F, G, stw(u), stx(u), 1,
-              stq(u ^ 1), stw(u ^ 1));
+              stq(u ^ 1), stw(u ^ 1), nothing);
           __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
           __syncthreads();
           if (k + 2 < nkt) {
@@ -782,7 +858,7 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
           }
           if constexpr (W8)
             if (k + 3 < nkt) issue_w(stq(u ^ 1), (k + 3) * BK);
-          mma(std::true_type{}, std::false_type{}, G, F, stw(u ^ 1), stx(u ^ 1), 0, sQ0, sW0);
+          mma(std::true_type{}, std::false_type{}, G, F, stw(u ^ 1), stx(u ^ 1), 0, sQ0, sW0, nothing);
         }
       }
     } else {
@@ -803,7 +879,7 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
             for (int i = 0; i < FN; ++i) rd_a(F, stw(u), kk, i);
 #pragma unroll
             for (int j = 0; j < FM; ++j) rd_b(F, stx(u), kk, j);
-            mma(std::false_type{}, std::false_type{}, F, G, sW0, sX0, kk, sQ0, sW0);
+            mma(std::false_type{}, std::false_type{}, F, G, sW0, sX0, kk, sQ0, sW0, nothing);
           }
           __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
           __syncthreads();
@@ -812,9 +888,9 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
     }
     // four waves: the last MFMAs' results land before the epilogue reads them
     if constexpr (NW == 4) agpr_fence();
-    // three stages: the empty-range loads of the last steps have landed in
+    // three stages (W3: of the weights): the empty-range loads of the last steps have landed in
     // every wave before the epilogue strips take stage 1
-    if constexpr (NS > 2) {
+    if constexpr (NS > 2 || W3) {
       __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
       __syncthreads();
     }
@@ -969,16 +1045,23 @@ int launch_gemm_cfg(const StreamArgs& a, hipStream_t s) {
 // The persistent form of a one-tile-per-CU grid: one workgroup per CU (at
 // most one per tile).
 constexpr int kTilesGrid = 256;
-template <int BN, int BM, int WN, int WM, bool GATEUP, bool W8 = false, int BK = kBK, int NS = 2>
+template <int BN, int BM, int WN, int WM, bool GATEUP, bool W8 = false, int BK = kBK, int NS = 2,
+          bool W3 = false>
 int launch_tiles_cfg(const StreamArgs& a, hipStream_t s) {
   const int64_t cols = GATEUP ? BN / 2 : BN;
   const int n_nt = (int)((a.N + cols - 1) / cols);
   const int n_mt = (int)((a.M + BM - 1) / BM);
   const int64_t tiles = (int64_t)n_nt * n_mt;
   const int grid = tiles < kTilesGrid ? (int)((tiles + 7) / 8 * 8) : kTilesGrid;
-  hipLaunchKernelGGL((gemm_tiles_kernel<BN, BM, WN, WM, GATEUP, W8, BK, NS>), dim3((unsigned)grid),
+  hipLaunchKernelGGL((gemm_tiles_kernel<BN, BM, WN, WM, GATEUP, W8, BK, NS, false, W3>), dim3((unsigned)grid),
                      dim3(WN * WM * kWave), 0, s, a, n_mt, n_nt, 1, 0, (float*)nullptr);
   return (int)hipGetLastError();
+}
+
+// Four waves with three weight stages (W3).
+template <int BN, int BM, int WN, int WM, bool GATEUP>
+int launch_w3_cfg(const StreamArgs& a, hipStream_t s) {
+  return launch_tiles_cfg<BN, BM, WN, WM, GATEUP, false, kBK, 2, true>(a, s);
 }
 
 // The staged four-wave tiles with k split across workgroups: `used` ranges
@@ -1056,7 +1139,7 @@ bool gemm_supported(const StreamArgs& a, bool aligned, bool w8) {
 // 128 KB).
 enum GemmTile { kT64x32, kT128x64, kT64x128, kT128x128, kT256x256, kT192x256,
                 kK64x64, kK96x128, kK128x128, kT320x256, kT192x128, kT160x128,
-                kT128x160, kT96x64, kT64x128w, kT96x128, kT160x256 };
+                kT128x160, kT96x64, kT64x128w, kT96x128, kT160x256, kT256x128 };
 struct TileInfo {
   int bn, bm, per_cu;
 };
@@ -1065,7 +1148,7 @@ constexpr TileInfo kTiles[] = {{64, 32, 4},   {128, 64, 3},  {64, 128, 2},
                                {64, 64, 2},   {96, 128, 1},  {128, 128, 1},
                                {320, 256, 1}, {192, 128, 1}, {160, 128, 1},
                                {128, 160, 1}, {96, 64, 1},   {64, 128, 1},  {96, 128, 1},
-                               {160, 256, 1}};
+                               {160, 256, 1}, {256, 128, 1}};
 constexpr int kCUs = 256;
 
 int64_t tile_count(int tile, int64_t M, int64_t N, bool gateup) {
@@ -1112,17 +1195,33 @@ constexpr TileCost kCost256x256{1.086, 0.0, 7.200};
 constexpr TileCost kCost192x256{0.948, 0.0, 4.843};
 constexpr TileCost kCost320x256{1.331, 0.0, 7.814};
 constexpr double kCostLaunch = 1.925;  // the tail plan's second launch
+// bf16: the four-wave tiles with three weight stages (one unit is about 1.36 us):
+// 256 x 256 4B QKV M = 2048 56.4 us, 8B down M = 4096 272, 192 x 256 4B QKV M =
+// 2048 52.2, 8B QKV M = 4096 154, 192 x 128 4096 -> 3072 at 2048 rows 44.4, 160 x
+// 128 4B o M = 2048 41.1.
+// The gate-up epilogue of 256 x 256 costs four units more (4B M = 2048 in two
+// rounds 137.5, 8B M = 4096 in six 574). With under 32 k-steps (0.6B) 256 x 256 and
+// 192 x 256 keep eight waves: 4096 x 1024 at 4096 rows 33.0 against 33.9.
+constexpr TileCost kCostW256x256{0.87, 0.0, 8.5};
+constexpr TileCost kCostW192x256{0.79, 0.0, 6.0};
+constexpr TileCost kCostW256x128{0.54, 0.0, 6.0};
+constexpr TileCost kCostW192x128{0.42, 0.0, 6.0};
+constexpr TileCost kCostW160x128{0.37, 0.0, 6.5};
 
-double grid_cost(int tile, int64_t M, int64_t N, int64_t nkt, bool gateup) {
+double grid_cost(int tile, int64_t M, int64_t N, int64_t nkt, bool gateup, bool bf16) {
   const int64_t n = tile_count(tile, M, N, gateup);
   if (n == 0) return 0.0;
   const int64_t k = (n + kCUs - 1) / kCUs;
   const TileCost& c = tile == kT64x128    ? kCost64x128
                       : tile == kT128x128 ? kCost128x128
-                      : tile == kT192x256 ? kCost192x256
+                      : tile == kT192x256 ? (bf16 ? kCostW192x256 : kCost192x256)
                       : tile == kT320x256 ? kCost320x256
-                                          : kCost256x256;
-  if (kTiles[tile].per_cu == 1) return (double)k * ((double)nkt * c.single + c.tile);
+                      : tile == kT256x128 ? kCostW256x128
+                      : tile == kT192x128 ? kCostW192x128
+                      : tile == kT160x128 ? kCostW160x128
+                                          : (bf16 ? kCostW256x256 : kCost256x256);
+  const double extra = bf16 && gateup && tile == kT256x256 ? 4.0 : 0.0;
+  if (kTiles[tile].per_cu == 1) return (double)k * ((double)nkt * c.single + c.tile + extra);
   const int64_t pairs = k / 2, singles = k % 2;
   return (double)nkt * ((double)pairs * c.pair + (double)singles * c.single) +
          (double)(pairs + singles) * c.tile;
@@ -1246,83 +1345,163 @@ int small_round_tile(int64_t M, int64_t N, int64_t K, bool gateup) {
 GemmPlan gemm_plan_unsplit(int64_t M, int64_t N, int64_t K, bool gateup, bool bf16) {
   if (bf16) {
     const int ts = small_round_tile(M, N, K, gateup);
-    if (ts >= 0) return GemmPlan{ts, 0};
+    if (ts >= 0) return GemmPlan{ts, 0, -1};
     // gate-up: one round of 96 x 128 four-wave tiles (96 weight rows, 48
     // outputs; an even number of 128-wide k-steps) on at least 192 CUs:
     // 8B TP=4 gate-up 4096 -> 2 x 3072 at M = 512 57.6 -> 39.5 us (hipBLASLt
     // 35.8), 4B TP=4 2560 -> 2 x 2432 at 512 31.2 -> 27.6 (26.8)
     if (gateup && K % (2 * kBK) == 0 && (K / (2 * kBK)) % 2 == 0) {
       const int64_t n = tile_count(kT96x128, M, N, true);
-      if (n >= 192 && n <= kCUs) return GemmPlan{kT96x128, 0};
+      if (n >= 192 && n <= kCUs) return GemmPlan{kT96x128, 0, -1};
     }
     const int t = k128_tile(M, N, K, gateup);
-    if (t >= 0) return GemmPlan{t, 0};
+    if (t >= 0) return GemmPlan{t, 0, -1};
   }
   const int64_t nkt = K / kBK;
-  GemmPlan best{kT64x128, 0};
-  double cbest = grid_cost(kT64x128, M, N, nkt, gateup);
-  for (int t : {kT128x128, kT256x256, kT192x256, kT320x256}) {
-    // 320 x 256 (bf16 only); QKV-like outputs for at most two rounds: beyond,
-    // the model underrates it (4B QKV M = 8192 226 against 206 us on 256 x
-    // 256). Gate-up at any count (same-box A/B against 256 x 256 and its
-    // tail, 4B gate-up: M = 3072 260 -> 248 us, 4096 345 -> 332, 6144 509 ->
-    // 483, 8192 668 -> 651).
-    if (t == kT320x256 && (!bf16 || (!gateup && tile_count(t, M, N, gateup) > 2 * kCUs))) continue;
-    const double c = grid_cost(t, M, N, nkt, gateup);
-    if (c < cbest) best = GemmPlan{t, 0}, cbest = c;
-  }
+  // The cheapest tile for N output columns (without the tail form).
+  const auto cheapest = [&](int64_t n_cols, double* cost) {
+    int best = kT64x128;
+    *cost = grid_cost(best, M, n_cols, nkt, gateup, bf16);
+    for (int t : {kT128x128, kT256x256, kT192x256, kT320x256, kT256x128, kT192x128, kT160x128}) {
+      // 320 x 256 (bf16 only); QKV-like outputs for at most two rounds: beyond,
+      // the model underrates it (4B QKV M = 8192 226 against 206 us on 256 x
+      // 256). Gate-up at any count (same-box A/B against eight-wave 256 x 256 and
+      // its tail, 4B gate-up: M = 3072 260 -> 248 us, 4096 345 -> 332, 6144 509 ->
+      // 483, 8192 668 -> 651).
+      if (t == kT320x256 && (!bf16 || (!gateup && tile_count(t, M, n_cols, gateup) > 2 * kCUs)))
+        continue;
+      // the smaller four-wave tiles: bf16
+      if (!bf16 && (t == kT256x128 || t == kT192x128 || t == kT160x128)) continue;
+      const double c = grid_cost(t, M, n_cols, nkt, gateup, bf16);
+      if (c < *cost) best = t, *cost = c;
+    }
+    return best;
+  };
+  double cbest;
+  GemmPlan best{cheapest(N, &cbest), 0, -1};
   const int64_t cols = gateup ? 128 : 256;  // output columns of a 256 x 256 tile
   const int64_t n_nt = (N + cols - 1) / cols, n_mt = (M + 255) / 256;
   const int64_t rounds = n_nt * n_mt / kCUs;
   const int64_t main_nt = rounds >= 1 ? rounds * kCUs / n_mt : 0;
   if (main_nt > 0 && main_nt < n_nt) {
     const int64_t nmain = main_nt * cols;
-    const double c = grid_cost(kT256x256, M, nmain, nkt, gateup) +
-                     grid_cost(kT128x128, M, N - nmain, nkt, gateup) + kCostLaunch;
-    if (c < cbest) best = GemmPlan{kT256x256, nmain}, cbest = c;
+    double ctail;
+    int tail = cheapest(N - nmain, &ctail);
+    if (!bf16) tail = kT128x128, ctail = grid_cost(tail, M, N - nmain, nkt, gateup, false);
+    const double c = grid_cost(kT256x256, M, nmain, nkt, gateup, bf16) + ctail + kCostLaunch;
+    if (c < cbest) best = GemmPlan{kT256x256, nmain, tail}, cbest = c;
   }
   const auto per_cu = [&](int t) { return (tile_count(t, M, N, gateup) + kCUs - 1) / kCUs; };
   if (best.tile == kT128x128 && per_cu(kT128x128) == 1 && per_cu(kT64x128) <= 2)
-    best = GemmPlan{kT64x128, 0};
-  // A single round of four-wave tiles (accumulators in AGPRs) on at least
-  // 240 CUs: 192 x 128, else 128 x 160 or 160 x 128, with an even number of
-  // 128-wide k-steps (192 x 128 also with an even number of at least 32
-  // 64-wide ones). Faster than the plan above wherever measured on MI355X
-  // (µs, previous plan -> 64-wide steps -> 128-wide steps): 8B gate-up M =
-  // 256 80.8 -> 73.4 -> 64.8; gate-up 4096 -> 2 x 6144 at M = 512 73.7 ->
-  // 67.2 -> 56.5, 4096 -> 2 x 1536 at M = 2048 66.1 -> 62.9 -> 52.6; QKV 2560
-  // -> 3072 at M = 2048 47.7 -> 44.3 -> 38.1, 4096 -> 3072 at M = 2048 66.8
-  // -> 63.1 -> 52.7; 128 x 160 for gate-up 2560 -> 2 x 1216 at M = 2048 42.2
-  // -> 32.1; 160 x 128 for gate-up 2560 -> 2 x 4864 at M = 512 52.8 -> 36.3.
-  // At 204-208 tiles 192 x 128 was 6% faster once and 9% slower once
-  // (64-wide steps), at 128 or fewer up to 46% slower.
+    best = GemmPlan{kT64x128, 0, -1};
+  // A single round of four-wave tiles on at least 240 CUs: 192 x 128, else
+  // 160 x 256 (gate-up; 80 outputs), 128 x 160 or 160 x 128. Measured on MI355X
+  // with two stages of 64- or 128-wide steps against the plans before (µs): QKV
+  // 2560 -> 3072 at M = 2048 47.7 -> 38.1, 4096 -> 3072 66.8 -> 52.7; gate-up 2560
+  // -> 2 x 1216 at M = 2048 (128 x 160) 42.2 -> 32.1, 2560 -> 2 x 4864 at M = 512
+  // (160 x 128) 52.8 -> 36.3, 4B at M = 512 (160 x 256) 62.8 -> 58.3; with three
+  // weight stages (W3 of gemm_tiles_kernel, one box) 8B gate-up M = 256 74.9 ->
+  // 66.2, 4096 -> 2 x 1536 at 2048 rows 54.6 -> 45.2, 2560 -> 2 x 1216 31.8 ->
+  // 29.3, 2560 -> 2 x 4864 32.9 -> 29.5, 4096 -> 2 x 6144 at 512 61.6 -> 57.1, 4B M
+  // = 512 69.3 -> 59.0, 4B o M = 2048 46.9 -> 41.1.
   if (bf16) {
-    const bool k128 = K % (2 * kBK) == 0 && (K / (2 * kBK)) % 2 == 0;
     const auto one_round = [&](int t) {
       const int64_t n = tile_count(t, M, N, gateup);
       return n >= 240 && n <= kCUs;
     };
-    if (one_round(kT192x128) && (k128 || (nkt % 2 == 0 && nkt >= 32))) return GemmPlan{kT192x128, 0};
-    // gate-up: one round of 160 x 256 four-wave tiles (80 outputs, 64-wide
-    // steps) in place of the fewer 192 x 256 ones: 4B gate-up 2560 -> 2 x
-    // 9728 at M = 512 62.8-63.1 -> 58.3-58.5 us (244 tiles against 204; with
-    // three LDS stages 60.6-61.2)
-    if (gateup && nkt % 2 == 0 && nkt >= 32 && one_round(kT160x256)) return GemmPlan{kT160x256, 0};
-    if (k128 && one_round(kT128x160)) return GemmPlan{kT128x160, 0};
-    if (k128 && one_round(kT160x128)) return GemmPlan{kT160x128, 0};
+    if (one_round(kT192x128)) return GemmPlan{kT192x128, 0, -1};
+    if (gateup && nkt >= 32 && one_round(kT160x256)) return GemmPlan{kT160x256, 0, -1};
+    if (one_round(kT128x160)) return GemmPlan{kT128x160, 0, -1};
+    if (one_round(kT160x128)) return GemmPlan{kT160x128, 0, -1};
   }
-  // QKV: two nearly whole rounds of 192 x 256 tiles (four waves) over 256 x
-  // 256 rounds plus a 128 x 128 tail (same box, µs, bit-identical
-  // plans aside: 4B M = 4096 120.7 -> 117.3, 8B M = 4096 178.4 -> 175.6).
-  // int8 too, on eight-wave dequantise-once tiles, in place of a 256 x 256
-  // round and a 128 x 128 tail of gemm_kernel, which dequantises every
-  // fragment in each wave that reads it (same box, bit-identical: 8B M =
-  // 4096 202.2 -> 181.6 us, 4B M = 4096 133.1 -> 120.6)
-  if (!gateup && nkt % 2 == 0 && nkt >= 32 && best.tile == kT256x256) {
+  // int8 QKV: two nearly whole rounds of 192 x 256 dequantise-once tiles over a
+  // 256 x 256 round and a 128 x 128 tail of gemm_kernel, which dequantises every
+  // fragment in each wave that reads it (same box, bit-identical: 8B M = 4096
+  // 202.2 -> 181.6 us, 4B M = 4096 133.1 -> 120.6)
+  if (!bf16 && !gateup && nkt % 2 == 0 && nkt >= 32 && best.tile == kT256x256) {
     const int64_t n = tile_count(kT192x256, M, N, false);
-    if (n > kCUs && n <= 2 * kCUs && n >= 2 * kCUs - kCUs / 16) return GemmPlan{kT192x256, 0};
+    if (n > kCUs && n <= 2 * kCUs && n >= 2 * kCUs - kCUs / 16) return GemmPlan{kT192x256, 0, -1};
   }
   return best;
+}
+
+// One grid of a plan's tile (a GemmTile).
+template <bool GATEUP, bool W8>
+int launch_gemm_tile(const StreamArgs& a, int tile, hipStream_t s) {
+  if constexpr (W8) {
+    switch (tile) {
+      case kT64x128: return launch_gemm_cfg<64, 128, 2, 2, GATEUP, 3, true>(a, s);
+      case kT128x128: return launch_gemm_cfg<128, 128, 4, 2, GATEUP, 2, true>(a, s);
+      // eight waves: four measured slower, 8B QKV M = 4096 181.6 -> 198.5 us,
+      // 4B M = 2048 61.3 -> 69.0
+      case kT192x256: return launch_tiles_cfg<192, 256, 2, 4, GATEUP, true>(a, s);
+      case kT256x256: return launch_tiles_cfg<256, 256, 4, 2, GATEUP, true>(a, s);
+      default: return (int)hipErrorInvalidValue;  // never planned for int8
+    }
+  } else {
+    const bool k128 = a.K % (2 * kBK) == 0;            // whole 128-wide steps
+    const bool k128e = k128 && (a.K / (2 * kBK)) % 2 == 0;  // ... an even number
+    switch (tile) {
+      case kT64x128: return launch_gemm_cfg<64, 128, 2, 2, GATEUP, 3>(a, s);
+      case kT128x128: return launch_gemm_cfg<128, 128, 4, 2, GATEUP, 2>(a, s);
+      case kT320x256:
+        if constexpr (GATEUP) return launch_tiles_cfg<320, 256, 2, 4, true>(a, s);
+        return launch_tiles_cfg<320, 256, 4, 2, false>(a, s);
+      // four waves with three weight stages (gate-up tiles whose weight rows
+      // cannot be split into whole gate/up pairs per wave column take one wave
+      // column)
+      case kT256x256:
+        if (a.K < 32 * kBK) return launch_tiles_cfg<256, 256, 4, 2, GATEUP>(a, s);
+        return launch_w3_cfg<256, 256, 2, 2, GATEUP>(a, s);
+      case kT192x256:
+        if (a.K < 32 * kBK) return launch_tiles_cfg<192, 256, 2, 4, GATEUP>(a, s);
+        return launch_w3_cfg<192, 256, 2, 2, GATEUP>(a, s);
+      case kT256x128: return launch_w3_cfg<256, 128, 4, 1, GATEUP>(a, s);
+      case kT192x128: return launch_w3_cfg<192, 128, 2, 2, GATEUP>(a, s);
+      case kT128x160: return launch_w3_cfg<128, 160, 2, 2, GATEUP>(a, s);
+      case kT160x128:
+        if constexpr (GATEUP) return launch_w3_cfg<160, 128, 1, 4, true>(a, s);
+        return launch_w3_cfg<160, 128, 2, 2, false>(a, s);
+      case kT160x256:
+        if constexpr (GATEUP) return launch_w3_cfg<160, 256, 1, 4, true>(a, s);
+        return (int)hipErrorInvalidValue;  // planned for gate-up only
+      case kK64x64: return launch_gemm_cfg<64, 64, 2, 2, GATEUP, 2, false, 128>(a, s);
+      // The one-per-CU tiles with 128-wide k-steps run as the pipelined
+      // four-wave tile loop where their step count is even (measured on
+      // MI355X against gemm_kernel, bit-identical, µs: 4B QKV M = 512 30.9
+      // -> 27.5, M = 384 30.8 -> 27.2; 8B QKV M = 512 44.1 -> 39.8; 0.6B
+      // QKV M = 1024 16.4 -> 14.7, gate-up M = 512 15.7 -> 14.8; other
+      // shapes even). 64 x 64 tiles run two per CU in gemm_kernel, which
+      // one persistent workgroup per CU does not match (0.6B QKV M = 512
+      // 11.9 -> 16.8). With three weight stages of 64-wide steps 96 x 128 was
+      // 2-5% slower (4B QKV M = 400, 512).
+      case kK128x128:
+        if (k128e) return launch_tiles_cfg<128, 128, 2, 2, GATEUP, false, 2 * kBK>(a, s);
+        return launch_gemm_cfg<128, 128, 4, 2, GATEUP, 2, false, 128>(a, s);
+      case kK96x128:
+        if constexpr (!GATEUP) {
+          if (k128e) return launch_tiles_cfg<96, 128, 2, 2, false, false, 2 * kBK>(a, s);
+          return launch_gemm_cfg<96, 128, 2, 2, false, 2, false, 128>(a, s);
+        }
+        return (int)hipErrorInvalidValue;  // never planned for gate-up
+      // Four waves, 128-wide k-steps: 96 x 64 and 64 x 128 with three LDS stages
+      // (any step count; with three weight stages of 64-wide steps 3-15% slower);
+      // 96 x 128 with two (an even step count).
+      case kT96x64:
+        if (!k128) return (int)hipErrorInvalidValue;  // never planned so
+        if constexpr (GATEUP) return launch_tiles_cfg<96, 64, 1, 4, true, false, 2 * kBK, 3>(a, s);
+        return launch_tiles_cfg<96, 64, 2, 2, false, false, 2 * kBK, 3>(a, s);
+      case kT64x128w:
+        if (!k128) return (int)hipErrorInvalidValue;
+        if constexpr (GATEUP) return launch_tiles_cfg<64, 128, 1, 4, true, false, 2 * kBK, 3>(a, s);
+        return launch_tiles_cfg<64, 128, 2, 2, false, false, 2 * kBK, 3>(a, s);
+      case kT96x128:
+        if (!k128e) return (int)hipErrorInvalidValue;
+        if constexpr (GATEUP) return launch_tiles_cfg<96, 128, 1, 4, true, false, 2 * kBK>(a, s);
+        return launch_tiles_cfg<96, 128, 2, 2, false, false, 2 * kBK>(a, s);
+      default: return (int)hipErrorInvalidValue;
+    }
+  }
 }
 
 template <bool GATEUP, bool W8>
@@ -1338,94 +1517,10 @@ int launch_gemm(const StreamArgs& a, hipStream_t s) {
     if (a.M <= 256 && n >= 192 && n <= kCUs) return launch_tiles_cfg<192, 128, 2, 4, true, true>(a, s);
   }
   const GemmPlan p = gemm_plan_unsplit(a.M, a.N, a.K, GATEUP, !W8);
-  if constexpr (!W8) {
-    switch (p.tile) {
-      case kT320x256:
-        if constexpr (GATEUP) return launch_tiles_cfg<320, 256, 2, 4, true>(a, s);
-        return launch_tiles_cfg<320, 256, 4, 2, false>(a, s);
-      case kK64x64: return launch_gemm_cfg<64, 64, 2, 2, GATEUP, 2, false, 128>(a, s);
-      // The one-per-CU tiles with 128-wide k-steps run as the pipelined
-      // four-wave tile loop where their step count is even (measured on
-      // MI355X against gemm_kernel, bit-identical, µs: 4B QKV M = 512 30.9
-      // -> 27.5, M = 384 30.8 -> 27.2; 8B QKV M = 512 44.1 -> 39.8; 0.6B
-      // QKV M = 1024 16.4 -> 14.7, gate-up M = 512 15.7 -> 14.8; other
-      // shapes even). 64 x 64 tiles run two per CU in gemm_kernel, which
-      // one persistent workgroup per CU does not match (0.6B QKV M = 512
-      // 11.9 -> 16.8).
-      case kK128x128:
-        if ((a.K / (2 * kBK)) % 2 == 0)
-          return launch_tiles_cfg<128, 128, 2, 2, GATEUP, false, 2 * kBK>(a, s);
-        return launch_gemm_cfg<128, 128, 4, 2, GATEUP, 2, false, 128>(a, s);
-      case kK96x128:
-        if constexpr (!GATEUP) {
-          if ((a.K / (2 * kBK)) % 2 == 0)
-            return launch_tiles_cfg<96, 128, 2, 2, false, false, 2 * kBK>(a, s);
-          return launch_gemm_cfg<96, 128, 2, 2, false, 2, false, 128>(a, s);
-        }
-        return (int)hipErrorInvalidValue;  // never planned for gate-up
-      // Four waves, 128-wide k-steps. 96 x 64 and 64 x 128 with three LDS
-      // stages (any step count); 96 x 128 with two (an even step count).
-      // Gate-up tiles whose weight rows cannot be split into whole gate/up
-      // pairs per wave column take one wave column.
-      case kT96x64:
-        if (a.K % (2 * kBK) != 0) return (int)hipErrorInvalidValue;  // never planned so
-        if constexpr (GATEUP) return launch_tiles_cfg<96, 64, 1, 4, true, false, 2 * kBK, 3>(a, s);
-        return launch_tiles_cfg<96, 64, 2, 2, false, false, 2 * kBK, 3>(a, s);
-      case kT64x128w:
-        if (a.K % (2 * kBK) != 0) return (int)hipErrorInvalidValue;
-        if constexpr (GATEUP) return launch_tiles_cfg<64, 128, 1, 4, true, false, 2 * kBK, 3>(a, s);
-        return launch_tiles_cfg<64, 128, 2, 2, false, false, 2 * kBK, 3>(a, s);
-      case kT96x128:
-        if (a.K % (2 * kBK) != 0 || (a.K / (2 * kBK)) % 2 != 0) return (int)hipErrorInvalidValue;
-        if constexpr (GATEUP) return launch_tiles_cfg<96, 128, 1, 4, true, false, 2 * kBK>(a, s);
-        return launch_tiles_cfg<96, 128, 2, 2, false, false, 2 * kBK>(a, s);
-      default: break;
-    }
-  }
-  switch (p.tile) {
-    case kT64x128: return launch_gemm_cfg<64, 128, 2, 2, GATEUP, 3, W8>(a, s);
-    case kT128x128: return launch_gemm_cfg<128, 128, 4, 2, GATEUP, 2, W8>(a, s);
-    case kT192x128:
-    case kT160x128:
-    case kT128x160:
-      // four waves, 128-wide k-steps where their count is even (planned
-      // only so, except 192 x 128, which may take 64-wide ones)
-      if constexpr (!W8) {
-        const bool k128 = a.K % (2 * kBK) == 0 && (a.K / (2 * kBK)) % 2 == 0;
-        if (p.tile == kT192x128) {
-          if (k128) return launch_tiles_cfg<192, 128, 2, 2, GATEUP, false, 2 * kBK>(a, s);
-          return launch_tiles_cfg<192, 128, 2, 2, GATEUP, false>(a, s);
-        }
-        if (!k128) return (int)hipErrorInvalidValue;  // never planned so
-        if (p.tile == kT128x160) return launch_tiles_cfg<128, 160, 2, 2, GATEUP, false, 2 * kBK>(a, s);
-        // 160 x 128: gate-up needs whole gate/up pairs per wave (one wave column)
-        if constexpr (GATEUP) return launch_tiles_cfg<160, 128, 1, 4, true, false, 2 * kBK>(a, s);
-        return launch_tiles_cfg<160, 128, 2, 2, false, false, 2 * kBK>(a, s);
-      }
-      return (int)hipErrorInvalidValue;  // never planned for int8
-    case kT160x256:
-      // bf16 gate-up, an even number of at least 32 k-steps (planned only
-      // so): four waves in one column of 160 weight rows
-      if constexpr (GATEUP && !W8)
-        if ((a.K / kBK) % 2 == 0 && a.K / kBK >= 32)
-          return launch_tiles_cfg<160, 256, 1, 4, true, false>(a, s);
-      return (int)hipErrorInvalidValue;
-    case kT192x256:
-      // bf16 with an even number of at least 32 k-steps: four waves (QKV
-      // too, same box, bit-identical: 4B M = 2048 61.1 -> 60.4 us, M = 4096
-      // 120.7 -> 117.3; 8B M = 2048 91.2 -> 88.4, M = 4096 178.4 -> 175.6)
-      // (int8 keeps eight waves: four measured slower, 8B QKV M = 4096
-      // 181.6 -> 198.5 us, 4B M = 2048 61.3 -> 69.0)
-      if constexpr (!W8)
-        if ((a.K / kBK) % 2 == 0 && a.K / kBK >= 32)
-          return launch_tiles_cfg<192, 256, 2, 2, GATEUP, false>(a, s);
-      return launch_tiles_cfg<192, 256, 2, 4, GATEUP, W8>(a, s);
-    default: break;
-  }
-  if (p.nmain == 0) return launch_tiles_cfg<256, 256, 4, 2, GATEUP, W8>(a, s);
+  if (p.nmain == 0) return launch_gemm_tile<GATEUP, W8>(a, p.tile, s);
   StreamArgs m = a;
   m.N = p.nmain;
-  int e = launch_tiles_cfg<256, 256, 4, 2, GATEUP, W8>(m, s);
+  int e = launch_gemm_tile<GATEUP, W8>(m, kT256x256, s);
   if (e) return e;
   // the tail: output columns nmain .. N-1 (weight rows and, for int8, their
   // scales from nmain on)
@@ -1452,7 +1547,7 @@ int launch_gemm(const StreamArgs& a, hipStream_t s) {
     if (n >= 192 && n <= kCUs) return launch_tiles_cfg<192, 128, 2, 4, true, true>(t, s);
     return launch_tiles_cfg<256, 128, 4, 2, true, true>(t, s);
   }
-  return launch_gemm_cfg<128, 128, 4, 2, GATEUP, 2, W8>(t, s);
+  return launch_gemm_tile<GATEUP, W8>(t, p.tail, s);
 }
 
 // When to split k across workgroups, measured on MI355X over Qwen3-0.6B/4B/8B
@@ -1543,6 +1638,12 @@ GemmSplit gemm_split_plan_bf16(int64_t M, int64_t N, int64_t K, bool gateup) {
 bool use_gemm_split(const StreamArgs& a, bool aligned, bool gateup, GemmSplit* p) {
   if (!a.ws || !gemm_supported(a, aligned, false)) return false;
   *p = gemm_split_plan_bf16(a.M, a.N, a.K, gateup);
+  // Above 1024 rows, where the split takes 256 x 256 tiles, a round of the
+  // four-wave tiles needs no partials and the workspace stays unused: 4B down M =
+  // 1200, 1500, 1700, 2048 84.5, 78.3, 133.4, 96.1 split, 78.2, 78.9, 84.5, 83.6
+  // not, 4B o M = 1200, 1500 49.8, 47.0 against 35.1, 36.0, 8B down M = 1200 117.8
+  // against 120.3 (us, one box).
+  if (p->tile == kT256x256) return false;
   return p->tile >= 0 && gemm_split_ws_floats(*p, a.M, a.N, a.K, gateup) <= a.ws_floats;
 }
 
@@ -1563,7 +1664,9 @@ int launch_gemm_split(const StreamArgs& a, const GemmSplit& p, hipStream_t s) {
     case kT128x64: return launch_gemm_splitk_cfg<128, 64, 4, 2, GATEUP, 2, W8>(a, p.nsplit, a.ws, s);
     case kT64x128: return launch_gemm_splitk_cfg<64, 128, 2, 2, GATEUP, 3, W8>(a, p.nsplit, a.ws, s);
     case kT128x128: return launch_gemm_splitk_cfg<128, 128, 4, 2, GATEUP, 2, W8>(a, p.nsplit, a.ws, s);
-    default: return launch_gemm_splitk_cfg<256, 256, 4, 2, GATEUP, 2, W8>(a, p.nsplit, a.ws, s);
+    default:  // int8 only (use_gemm_split)
+      if constexpr (W8) return launch_gemm_splitk_cfg<256, 256, 4, 2, GATEUP, 2, true>(a, p.nsplit, a.ws, s);
+      return (int)hipErrorInvalidValue;
   }
 }
 

@@ -129,11 +129,12 @@ template <bool GATEUP, bool W8>
 int launch_gemm(const StreamArgs& a, hipStream_t s);
 // The unsplit grid launch_gemm runs: tile (a GemmTile of fp_gemm.hip) and,
 // when nmain > 0, whole 256 x 256 rounds over the first nmain output columns
-// followed by 128 x 128 tiles over the rest. bf16: whether the tiles with
+// followed by tiles `tail` over the rest. bf16: whether the tiles with
 // 128-wide k-steps (bf16 weights only) are candidates.
 struct GemmPlan {
   int tile;
   int64_t nmain;
+  int tail;
 };
 GemmPlan gemm_plan_unsplit(int64_t M, int64_t N, int64_t K, bool gateup, bool bf16);
 // Whether the bf16 plan is a single round of tiles with 128-wide k-steps with

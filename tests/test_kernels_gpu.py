@@ -1201,3 +1201,49 @@ def test_quantise_rows_of_any_size_and_alignment(K):
             wd = wide[:, off:off + K]
         q, s = _kernels().quantize_w8_per_row(wd)
         assert np.array_equal(q.cpu().numpy(), qo) and np.array_equal(s.cpu().numpy(), so), off
+
+
+# (op, M, K, N) that run each four-wave tile with three weight stages: fewer k-steps
+# than stages would hold is not planned (32 at least for the two largest), odd and even
+# step counts, several tiles per workgroup, partial tiles both ways, the two-launch
+# form with its tail
+W3_TILES = [
+    ("linear", 4090, 2112, 4090),    # 256 x 256, odd step count, one round
+    ("linear", 2040, 2560, 6140),    # 192 x 256
+    ("linear", 2048, 4160, 4096),    # 256 x 128
+    ("linear", 2040, 4096, 3070),    # 192 x 128
+    ("linear", 2040, 2624, 2550),    # 160 x 128, odd step count
+    ("linear", 1900, 640, 2550),     # a short K
+    ("gate-up", 2048, 2560, 1216),   # 128 x 160
+    ("gate-up", 510, 2560, 4860),    # 160 x 128, one wave column
+    ("gate-up", 500, 2560, 9700),    # 160 x 256, one wave column
+    ("gate-up", 250, 4096, 12280),   # 192 x 128
+    ("gate-up", 1000, 4096, 8000),   # 256 x 256 or its tail form
+    ("linear", 4000, 2112, 6100),    # more than a round
+]
+
+
+@pytest.mark.parametrize("op,M,K,N", W3_TILES)
+def test_three_weight_stage_tiles(op, M, K, N):
+    """Against the oracle on rows at the tiles' edges, bit-identical on a second
+    call, and bit-identical to the same rows computed as part of a smaller
+    call, which runs another tile (every plan sums in the same k order)."""
+    kern = _kernels()
+    rows = np.array([0, 1, M // 2, M - 2, M - 1])
+    if op == "linear":
+        x, w = qkv_inputs(77, M, K, N, 0)
+        run = lambda t: kern.fused_linear(t, wd)  # noqa: E731
+        wd = w.to(DEV)
+        out = ref.ref_linear(bits(x)[rows], bits(w))
+    else:
+        x, wg, wu = ffn_inputs(78, M, K, N)
+        gd, ud = wg.to(DEV), wu.to(DEV)
+        run = lambda t: kern.triton_fused_gate_up_silu(t, gd, ud)  # noqa: E731
+        out = ref.ref_gate_up_silu_full(bits(x)[rows], bits(wg), bits(wu))
+    xd = x.to(DEV)
+    y = run(xd)
+    _check(y.cpu()[rows], out, f"{op} M={M} K={K} N={N}")
+    assert torch.equal(run(xd), y)
+    if M >= 1900:
+        half = M // 2 + 100
+        assert torch.equal(run(xd[:half].contiguous()), y[:half])
