@@ -439,9 +439,9 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
                 "32-wide k-substeps: two per k-step, or four with four bf16 waves");
   static_assert(NS == 2 || ((NS == 3 || NS == 4) && WN * WM == 4 && !W8),
                 "three or four LDS stages: four bf16 waves");
-  static_assert(!W3 || (NS == 2 && BK == 64 && WN * WM == 4 && !W8 && !SPLIT),
-                "three weight stages: 64-wide steps, four bf16 waves, unsplit");
-  static_assert(!SPLIT || NS > 2, "k split across workgroups: the staged four-wave loop");
+  static_assert(!W3 || (NS == 2 && BK == 64 && WN * WM == 4 && !W8),
+                "three weight stages: 64-wide steps, four bf16 waves");
+  static_assert(!SPLIT || NS > 2 || W3, "k split across workgroups: the staged four-wave loop");
   static_assert(BN % WRPI == 0 && BM % (RPI * NW) == 0, "tile/waves");
   static_assert(W8 || NWI % NW == 0, "bf16 weight loads spread evenly over the waves");
   static_assert(NQC % kWave == 0, "int8 chunks: whole waves");
@@ -1120,6 +1120,26 @@ int launch_gemm_splitk_cfg(const StreamArgs& a, int nsplit, float* ws, hipStream
   return (int)hipGetLastError();
 }
 
+// The same on the four-wave tiles with three weight stages (bf16; 4B down M = 2048
+// 105 -> 94 us, at 1200 rows 86 -> 66, 8B down at 1200 121 -> 107).
+template <int BN, int BM, int WN, int WM, bool GATEUP>
+int launch_w3_split_cfg(const StreamArgs& a, int nsplit, float* ws, hipStream_t s) {
+  const int64_t cols = GATEUP ? BN / 2 : BN;
+  const int n_nt = (int)((a.N + cols - 1) / cols);
+  const int n_mt = (int)((a.M + BM - 1) / BM);
+  const int per = (int)gemm_splitk_ksteps(a.K, nsplit), used = gemm_splitk_used(a.K, nsplit);
+  const int64_t items = (int64_t)n_nt * n_mt * used;
+  const int grid = items < kTilesGrid ? (int)((items + 7) / 8 * 8) : kTilesGrid;
+  hipLaunchKernelGGL((gemm_tiles_kernel<BN, BM, WN, WM, GATEUP, false, kBK, 2, true, true>),
+                     dim3((unsigned)grid), dim3(WN * WM * kWave), 0, s, a, n_mt, n_nt, used, per, ws);
+  const int e = (int)hipGetLastError();
+  if (e) return e;
+  const int64_t threads = a.M * ((a.N + 3) / 4);
+  hipLaunchKernelGGL(splitk_reduce_kernel<GATEUP>, dim3((unsigned)((threads + 255) / 256)),
+                     dim3(256), 0, s, ws, used, a);
+  return (int)hipGetLastError();
+}
+
 // Whether gemm_kernel can run this call: whole 64-wide k-steps, 16-byte
 // aligned rows, every operand's byte size below 2^31 (buffer-resource sizes
 // and 32-bit lane offsets); int8 also needs its row scales.
@@ -1199,7 +1219,7 @@ constexpr double kCostLaunch = 1.925;  // the tail plan's second launch
 // 256 x 256 4B QKV M = 2048 56.4 us, 8B down M = 4096 272, 192 x 256 4B QKV M =
 // 2048 52.2, 8B QKV M = 4096 154, 192 x 128 4096 -> 3072 at 2048 rows 44.4, 160 x
 // 128 4B o M = 2048 41.1.
-// The gate-up epilogue of 256 x 256 costs four units more (4B M = 2048 in two
+// The gate-up epilogue of 256 x 256 costs six units more (4B M = 2048 in two
 // rounds 137.5, 8B M = 4096 in six 574). With under 32 k-steps (0.6B) 256 x 256 and
 // 192 x 256 keep eight waves: 4096 x 1024 at 4096 rows 33.0 against 33.9.
 constexpr TileCost kCostW256x256{0.87, 0.0, 8.5};
@@ -1220,7 +1240,7 @@ double grid_cost(int tile, int64_t M, int64_t N, int64_t nkt, bool gateup, bool 
                       : tile == kT192x128 ? kCostW192x128
                       : tile == kT160x128 ? kCostW160x128
                                           : (bf16 ? kCostW256x256 : kCost256x256);
-  const double extra = bf16 && gateup && tile == kT256x256 ? 4.0 : 0.0;
+  const double extra = bf16 && gateup && tile == kT256x256 ? 6.0 : 0.0;
   if (kTiles[tile].per_cu == 1) return (double)k * ((double)nkt * c.single + c.tile + extra);
   const int64_t pairs = k / 2, singles = k % 2;
   return (double)nkt * ((double)pairs * c.pair + (double)singles * c.single) +
@@ -1638,12 +1658,12 @@ GemmSplit gemm_split_plan_bf16(int64_t M, int64_t N, int64_t K, bool gateup) {
 bool use_gemm_split(const StreamArgs& a, bool aligned, bool gateup, GemmSplit* p) {
   if (!a.ws || !gemm_supported(a, aligned, false)) return false;
   *p = gemm_split_plan_bf16(a.M, a.N, a.K, gateup);
-  // Above 1024 rows, where the split takes 256 x 256 tiles, a round of the
-  // four-wave tiles needs no partials and the workspace stays unused: 4B down M =
-  // 1200, 1500, 1700, 2048 84.5, 78.3, 133.4, 96.1 split, 78.2, 78.9, 84.5, 83.6
-  // not, 4B o M = 1200, 1500 49.8, 47.0 against 35.1, 36.0, 8B down M = 1200 117.8
-  // against 120.3 (us, one box).
-  if (p->tile == kT256x256) return false;
+  // Above 1024 rows, where the split takes 256 x 256 tiles, and up to K = 4096 a
+  // round of the four-wave tiles needs no partials and the workspace stays unused
+  // (weights cycled through HBM, us, split / not: 4B o M = 1200 50.5 / 35.8; with
+  // a longer K it loses: 4B down M = 1200, 1500, 2048 67, 74, 94 / 97, 105, 116, 8B
+  // down M = 1200 107 / 149).
+  if (p->tile == kT256x256 && a.K <= 4096) return false;
   return p->tile >= 0 && gemm_split_ws_floats(*p, a.M, a.N, a.K, gateup) <= a.ws_floats;
 }
 
@@ -1664,9 +1684,9 @@ int launch_gemm_split(const StreamArgs& a, const GemmSplit& p, hipStream_t s) {
     case kT128x64: return launch_gemm_splitk_cfg<128, 64, 4, 2, GATEUP, 2, W8>(a, p.nsplit, a.ws, s);
     case kT64x128: return launch_gemm_splitk_cfg<64, 128, 2, 2, GATEUP, 3, W8>(a, p.nsplit, a.ws, s);
     case kT128x128: return launch_gemm_splitk_cfg<128, 128, 4, 2, GATEUP, 2, W8>(a, p.nsplit, a.ws, s);
-    default:  // int8 only (use_gemm_split)
-      if constexpr (W8) return launch_gemm_splitk_cfg<256, 256, 4, 2, GATEUP, 2, true>(a, p.nsplit, a.ws, s);
-      return (int)hipErrorInvalidValue;
+    default:
+      if constexpr (!W8) return launch_w3_split_cfg<256, 256, 2, 2, GATEUP>(a, p.nsplit, a.ws, s);
+      return launch_gemm_splitk_cfg<256, 256, 4, 2, GATEUP, 2, W8>(a, p.nsplit, a.ws, s);
   }
 }
 
