@@ -355,9 +355,12 @@ __global__ __launch_bounds__(512) void rows_narrow_kernel(StreamArgs a) {
   const int li = lane & 15;
   const int K = (int)a.K;
   const int64_t row0 = (int64_t)blockIdx.x * R;
-  // bytes from the workgroup's first row to the matrix's end: rows past N read
-  // as zeros, and so do lanes past the row's end (an offset past every buffer)
-  const int wbytes = (int)(((a.N - 1 - row0) * a.ldw0 + K) * WB);
+  // bytes from the workgroup's first row to the matrix's end: lanes past the
+  // row's end read as zeros (an offset past every buffer). The row is the scalar
+  // offset, which the range check need not see, so rows past N are row N - 1
+  // again (their outputs are not stored)
+  const int last = (int)(a.N - 1 - row0);
+  const int wbytes = (int)((last * a.ldw0 + K) * WB);
   const auto wrsrc = __builtin_amdgcn_make_buffer_rsrc(
       (char*)const_cast<void*>(a.w0) + row0 * a.ldw0 * WB, 0, wbytes, kRsrcFlags);
   const uint32_t ldb = (uint32_t)(a.ldw0 * WB);
@@ -375,12 +378,13 @@ __global__ __launch_bounds__(512) void rows_narrow_kernel(StreamArgs a) {
       xv[i][m] = m < a.M ? load_bf16x8<true>(a.x + m * a.ldx, k, K) : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int r = 0; r < R; ++r) {
+      const uint32_t soff = (uint32_t)(r < last ? r : last) * ldb;
       // non-temporal (cache-policy bit 1): read once per call
       if constexpr (W8) {
-        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(wrsrc, voff, r * ldb, 2);
+        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(wrsrc, voff, soff, 2);
         wf[i][r] = u32x4{v.x, v.y, 0u, 0u};
       } else {
-        wf[i][r] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, voff, r * ldb, 2);
+        wf[i][r] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, voff, soff, 2);
       }
     }
   }

@@ -1150,6 +1150,37 @@ def test_narrow_outputs(M, K, N):
     assert torch.equal(kern.fused_linear_w8(xd[:, :K], q, s), y8)
 
 
+# (M, K, N) on whole rows split over eight waves whose last workgroup is partial: 1-4
+# of five rows past N, 1-2 of three, 1 of two; the first, second and third K chunk of a
+# wave partly past the row, the largest K and the first past it (K a multiple of 16: the
+# int8 kernel takes the call too)
+NARROW_PARTIAL = [(1, 2576, 2551), (2, 4112, 2552), (1, 8208, 2053), (2, 9744, 2559),
+                  (1, 12288, 2051), (1, 12304, 2051), (2, 4112, 1027), (1, 8208, 1028), (1, 5008, 513)]
+
+
+@pytest.mark.parametrize("M,K,N", NARROW_PARTIAL)
+def test_narrow_outputs_partial_last_workgroup(M, K, N):
+    """bf16 and int8 weights with padded rows (NaN, int8 127, beside and after
+    them): against the oracle, and the same bits as the contiguous weights'."""
+    kern = _kernels()
+    x, w = qkv_inputs(710 + M, M, K, N, 0)
+    xd, wd = x.to(DEV), w.to(DEV)
+
+    def padded(t, fill):
+        wide = torch.full((N + 8, K + 32), fill, dtype=t.dtype, device=DEV)
+        wide[:N, :K] = t
+        return wide[:N, :K]
+
+    y = kern.fused_linear(xd, padded(wd, float("nan")))
+    _check(y.cpu(), ref.ref_linear(bits(x), bits(w)), f"narrow M={M} K={K} N={N}")
+    assert torch.equal(kern.fused_linear(xd, wd), y)
+    q, s = kern.quantize_w8_per_row(wd)
+    y8 = kern.fused_linear_w8(xd, padded(q, 127), s)
+    wq = ref.dequant_w8(q.cpu().numpy(), s.cpu().numpy())
+    _check(y8.cpu(), ref.ref_linear(bits(x), wq), f"narrow int8 M={M} K={K} N={N}")
+    assert torch.equal(kern.fused_linear_w8(xd, q, s), y8)
+
+
 # (M, K, N): k tails of every kind against 64-wide (int8 128-wide) steps, rows at any
 # byte, on the streaming kernel (to 32 rows) and the 32 x 32, 64 x 64 and 128 x 128
 # tiles, at their row counts' edges and with partial tiles both ways
