@@ -532,7 +532,11 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
   // weight rows of k-step k0 / BK: bf16 into an operand stage, int8 into a
   // staging buffer
   // live false: the same instructions with an empty buffer range (they read
-  // nothing and land zeros), so that every step issues the same loads
+  // nothing and land zeros), so that every step issues the same loads; the
+  // scalar offset is then 0, since one past the range need not be checked
+  auto soff = [&](int64_t k0, int bytes, bool live) {
+    return live ? (uint32_t)((kb * BK + k0) * bytes) : 0u;
+  };
   auto issue_w = [&](void* dst, int64_t k0, bool live = true) {
 #pragma unroll
     for (int j = 0; j < IW; ++j) {
@@ -541,25 +545,25 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
       const bool up = wrow_up(q * WRPI);
       load_lds16(up ? wptr1 : a.w0, live ? (up ? wbytes1 : wbytes0) : 0,
                  (lds_ptr_t)((char*)dst + q * WRPI * BK * WB), woff[j],
-                 (uint32_t)((kb * BK + k0) * WB));
+                 soff(k0, WB, live));
     }
   };
   auto issue_w1 = [&](void* dst, int j, int64_t k0, bool live) {
     const int q = wave + NW * j;
     const bool up = wrow_up(q * WRPI);
     load_lds16(up ? wptr1 : a.w0, live ? (up ? wbytes1 : wbytes0) : 0,
-               (lds_ptr_t)((char*)dst + q * WRPI * BK * WB), woff[j], (uint32_t)((kb * BK + k0) * WB));
+               (lds_ptr_t)((char*)dst + q * WRPI * BK * WB), woff[j], soff(k0, WB, live));
   };
   auto issue_x1 = [&](uint16_t (*tx)[BK], int j, int64_t k0, bool live) {
     load_lds16(a.x, live ? xbytes : 0, (lds_ptr_t)&tx[(wave + NW * j) * RPI][0], xoff[j],
-               (uint32_t)((kb * BK + k0) * 2));
+               soff(k0, 2, live));
   };
   auto nothing = [](int) {};
   auto issue_x = [&](uint16_t (*tx)[BK], int64_t k0, bool live = true) {
 #pragma unroll
     for (int j = 0; j < IX; ++j)
       load_lds16(a.x, live ? xbytes : 0, (lds_ptr_t)&tx[(wave + NW * j) * RPI][0], xoff[j],
-                 (uint32_t)((kb * BK + k0) * 2));
+                 soff(k0, 2, live));
   };
   // int8: chunk c of this lane (16 weights of row r, k-range 16 q .. 16 q +
   // 15 of the step) from staging buffer sq to bf16(q * s) in stage tw, in
@@ -749,7 +753,7 @@ __global__ __launch_bounds__(WN * WM * kWave) void gemm_tiles_kernel(StreamArgs 
           issue_w(stw(st), live ? st * BK : 0, live);
         }
       } else {
-        if (nkt > 1) {
+        if (nloc > 1) {
           issue_x(sX1, BK);
           issue_w(sW1, BK);
         }

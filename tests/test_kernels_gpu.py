@@ -875,6 +875,16 @@ def test_split_k_across_workgroups(M, N, K, op):
     _check(y.cpu()[rows], ref.ref_linear(bits(x)[rows], bits(w)), f"split {op} M={M} N={N} K={K}")
 
 
+@pytest.mark.parametrize("M,N,K,op", [
+    (1201, 2555, 9728, "linear"), (1025, 2052, 4672, "linear"), (1300, 2101, 4672, "linear"),
+    (1100, 2001, 8192, "gate-up"), (1100, 1100, 8192, "gate-up")])
+def test_split_k_above_1024_rows(M, N, K, op):
+    """The split on 256 x 256 tiles with three weight stages: partial tiles in M
+    and N, widths on both sides of a multiple of 4, an odd step count (4672),
+    both forms, 240-250 and 270 (more than one per CU) work items."""
+    test_split_k_across_workgroups(M, N, K, op)
+
+
 @pytest.mark.parametrize("M,K,N,op,split", [(47, 2576, 6144, "qkv", False),
                                             (48, 2576, 6144, "qkv", False),
                                             (48, 2560, 6144, "qkv", False),
