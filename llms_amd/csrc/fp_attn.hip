@@ -57,18 +57,17 @@ constexpr int vmcnt_imm(int v) { return (v & 15) | (7 << 4) | (15 << 8) | ((v >>
 // 16 bytes per lane from base + voff into LDS at dst + 16 * lane; bytes at or
 // past nbytes read as zero.
 __device__ __forceinline__ void load_lds16(const void* base, int nbytes, lds_ptr_t dst,
-                                           uint32_t voff, uint32_t soff) {
+                                           uint32_t voff) {
   constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format
   __builtin_amdgcn_raw_ptr_buffer_load_lds(
       __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, nbytes, kRsrcFlags), dst, 16,
-      voff, soff, 0, 0);
+      voff, 0, 0, 0);
 }
-__device__ __forceinline__ u32x4 load_buf16(const void* base, int nbytes, uint32_t voff,
-                                            uint32_t soff) {
+__device__ __forceinline__ u32x4 load_buf16(const void* base, int nbytes, uint32_t voff) {
   constexpr int kRsrcFlags = 0x00020000;
   return __builtin_amdgcn_raw_buffer_load_b128(
       __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, nbytes, kRsrcFlags), voff,
-      soff, 0);
+      0, 0);
 }
 
 // First position of the call's tokens (a device position far outside any cache
@@ -295,13 +294,13 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(AttnArgs a) {
     for (int n = 0; n < NV; ++n) {
       const int r = n * RPI + vr;
       load_lds16(vb, vbytes, (lds_ptr_t)(sv + n * 1024),
-                 (uint32_t)(c * KC + r) * vstep + (uint32_t)(((lane % CH) ^ (r & (CH - 1))) * 16), 0);
+                 (uint32_t)(c * KC + r) * vstep + (uint32_t)(((lane % CH) ^ (r & (CH - 1))) * 16));
     }
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int i = 0; i < DK; ++i)
-        kf[kt][i] = load_buf16(kb, kbytes, koff + (uint32_t)(c * KC + 16 * kt) * kstep + 64 * i, 0);
+        kf[kt][i] = load_buf16(kb, kbytes, koff + (uint32_t)(c * KC + 16 * kt) * kstep + 64 * i);
   };
 
   const float sc = kLog2e / sqrtf((float)D);
@@ -512,16 +511,20 @@ __global__ __launch_bounds__(256, 2) void attn_tiles_kernel(AttnArgs a, int n_rt
     koff[n] = (uint32_t)r * kstep + ch;
     voff[n] = (uint32_t)r * vstep + ch;
   }
+  // each tile's rows through a buffer that starts at the tile and ends with the
+  // last key, so that the lane offset alone tells whether a row is past it
   auto issue_k = [&](char* sk, int kt) {
+    const int off = (int)((uint32_t)(kt * KT) * kstep);
 #pragma unroll
     for (int n = 0; n < NL; ++n)
-      load_lds16(kb, kbytes, (lds_ptr_t)(sk + (wave * NL + n) * 1024), koff[n],
-                 (uint32_t)(kt * KT) * kstep);
+      load_lds16((const char*)kb + off, kbytes - off, (lds_ptr_t)(sk + (wave * NL + n) * 1024),
+                 koff[n]);
   };
   u32x4 vr[NL];
   auto load_v = [&](int kt) {
+    const int off = (int)((uint32_t)(kt * KT) * vstep);
 #pragma unroll
-    for (int n = 0; n < NL; ++n) vr[n] = load_buf16(vb, vbytes, voff[n], (uint32_t)(kt * KT) * vstep);
+    for (int n = 0; n < NL; ++n) vr[n] = load_buf16((const char*)vb + off, vbytes - off, voff[n]);
   };
   auto store_v = [&](char* sv, int st) {
     bool bad = false;

@@ -183,3 +183,21 @@ def test_cache_layouts_and_strided_rows():
         d = dict(c, q=wide[..., 4:4 + n], k=wide[..., 4 + n:4 + n + Hk * D],
                  v=wide[..., 4 + n + Hk * D:4 + n + 2 * Hk * D])
         assert torch.equal(attention_core(**d), want)
+
+
+@pytest.mark.parametrize("B,T,Hq,Hk,D,S,pos", [(1, 100, 8, 2, 128, 100, 0), (2, 65, 8, 8, 64, 201, 136),
+                                               (1, 1, 8, 2, 128, 97, 96), (1, 9, 16, 2, 128, 70, 61)])
+def test_full_cache_at_the_end_of_its_memory(B, T, Hq, Hk, D, S, pos):
+    """The last tile's rows past the last key are not read: with NaN right behind
+    a full cache that is no whole number of tiles, the same bits as without."""
+    c = _inputs(11, B, T, Hq, Hk, D, S, pos)
+    with torch.inference_mode():
+        n = B * Hk * S * D
+        for name in ("cache_k", "cache_v"):
+            flat = torch.full((n + 64 * D,), float("nan"), dtype=torch.bfloat16, device=DEV)
+            flat[:n] = c[name][:B].reshape(-1)
+            c[name] = flat[:n].view(B, Hk, S, D)
+        y = attention_core(**c)
+        _check(c, B, T, Hq, Hk, D, y)
+        d = dict(c, cache_k=c["cache_k"].clone(), cache_v=c["cache_v"].clone())
+        assert torch.equal(attention_core(**d), y)
