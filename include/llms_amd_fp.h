@@ -300,7 +300,9 @@ int fp_rmsnorm_qkv_bf16_noalloc(const void* x, int64_t ldx, const void* gamma, f
  * head_dim is 64 or 128; n_heads a multiple of n_kv_heads. q, k, v and the gammas
  * are 8-byte aligned with row strides that are multiples of 4, the caches
  * 16-byte aligned with strides that are multiples of 8, one head's cache (64
- * positions more than cache_len) under 2^31 bytes. workspace: at least
+ * positions more than cache_len) under 2^31 bytes. No two (b, head, position)
+ * of the B sequences share cache memory (a stride of 0 over more than one, say),
+ * nor keys with values or with q, k, v: FP_ERR_STRIDE. workspace: at least
  * fp_attention_workspace_bytes(..., keys) with keys = pos + T, or cache_len with
  * pos_dev; 16-byte aligned; written in full before it is read.
  */

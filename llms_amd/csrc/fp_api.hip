@@ -238,6 +238,60 @@ int check_attention(int64_t B, int64_t T, int64_t Hq, int64_t Hk, int64_t D) {
   return FP_OK;
 }
 
+// A dimension of a strided layout, in elements.
+struct Dim {
+  int64_t size, stride;
+};
+
+// Elements from the first to the last, if every dimension's stride passes over
+// all that the smaller ones reach (inner: the contiguous elements below them);
+// else -1: two indices may be one element.
+template <int N>
+int64_t nested_extent(Dim (&d)[N], int64_t inner) {
+  for (int i = 1; i < N; ++i)
+    for (int j = i; j > 0 && d[j].stride < d[j - 1].stride; --j) {
+      const Dim t = d[j];
+      d[j] = d[j - 1], d[j - 1] = t;
+    }
+  int64_t extent = inner;
+  for (const Dim& x : d) {
+    if (x.size <= 1) continue;
+    if (x.stride < extent) return -1;
+    extent += (x.size - 1) * x.stride;
+  }
+  return extent;
+}
+
+// Whether a call could write one cache element for two (sequence, head,
+// position) or as a key and as a value, or write what it reads as q, k or v:
+// its workgroups run in no order. Keys and values may interleave (a cache
+// [B][S][2][heads][D]) when their strides are the same.
+bool attention_overlaps(const fp_attention_args& g) {
+  const int64_t D = g.head_dim;
+  Dim k[] = {{g.B, g.k_s_b}, {g.n_kv_heads, g.k_s_h}, {g.cache_len, g.k_s_p}};
+  Dim v[] = {{g.B, g.v_s_b}, {g.n_kv_heads, g.v_s_h}, {g.cache_len, g.v_s_p}};
+  const auto same = [](int64_t size, int64_t a, int64_t b) { return size <= 1 || a == b; };
+  const bool alike = same(g.B, g.k_s_b, g.v_s_b) && same(g.n_kv_heads, g.k_s_h, g.v_s_h) &&
+                     same(g.cache_len, g.k_s_p, g.v_s_p);
+  const int64_t ek = nested_extent(k, D), ev = nested_extent(v, D);
+  if (ek < 0 || ev < 0) return true;
+  const uintptr_t kp = (uintptr_t)g.cache_k, vp = (uintptr_t)g.cache_v;
+  const auto meet = [](uintptr_t a, int64_t na, uintptr_t b, int64_t nb) {
+    return a < b + 2 * (uintptr_t)nb && b < a + 2 * (uintptr_t)na;
+  };
+  if (meet(kp, ek, vp, ev)) {
+    Dim kv[] = {{2, (int64_t)(kp < vp ? vp - kp : kp - vp) / 2}, k[0], k[1], k[2]};
+    if (!alike || nested_extent(kv, D) < 0) return true;
+  }
+  const int64_t last = g.B * g.T - 1;
+  const struct { const void* p; int64_t n; } in[] = {{g.q, last * g.ldq + g.n_heads * D},
+                                                     {g.k, last * g.ldk + g.n_kv_heads * D},
+                                                     {g.v, last * g.ldv + g.n_kv_heads * D}};
+  for (const auto& i : in)
+    if (meet(kp, ek, (uintptr_t)i.p, i.n) || meet(vp, ev, (uintptr_t)i.p, i.n)) return true;
+  return false;
+}
+
 }  // namespace
 
 int rmsnorm_qkv_args(const void* x, int64_t ldx, const void* gamma, float eps, const void* w,
@@ -517,6 +571,7 @@ int fp_attention_bf16(const fp_attention_args* g, void* workspace, int64_t works
   if (!al8(g->q) || !al8(g->k) || !al8(g->v) || !al8(g->q_gamma) || !al8(g->k_gamma) ||
       !al8(g->y) || !fp::al16(g->cache_k) || !fp::al16(g->cache_v))
     return FP_ERR_STRIDE;
+  if (fp::attention_overlaps(*g)) return FP_ERR_STRIDE;
   const int64_t keys = g->pos_dev ? S : g->pos + T;
   if (!workspace || !fp::al16(workspace) ||
       workspace_bytes < fp::attn_workspace_bytes(g->B, T, g->n_heads, g->n_kv_heads, D, keys))

@@ -201,3 +201,23 @@ def test_full_cache_at_the_end_of_its_memory(B, T, Hq, Hk, D, S, pos):
         _check(c, B, T, Hq, Hk, D, y)
         d = dict(c, cache_k=c["cache_k"].clone(), cache_v=c["cache_v"].clone())
         assert torch.equal(attention_core(**d), y)
+
+
+def test_overlapping_caches_stay_with_the_torch_form():
+    """A cache whose sequences or heads share memory (an expanded one), and keys
+    and values in one memory: nothing is launched or written (the torch form
+    refuses the first two). Keys and values interleaved in one buffer are taken."""
+    B, T, Hq, Hk, D, S, pos = 2, 2, 8, 4, 64, 40, 7
+    c = _inputs(2, B, T, Hq, Hk, D, S, pos)
+    ck, cv = c["cache_k"][:B].clone(), c["cache_v"][:B].clone()
+    with torch.inference_mode():
+        want = attention_core(**dict(c, cache_k=ck.clone(), cache_v=cv.clone()))
+        for change in (dict(cache_k=ck[:1].clone().expand(B, -1, -1, -1)),
+                       dict(cache_v=cv[:, :1].clone().expand(-1, Hk, -1, -1)),
+                       dict(cache_k=ck, cache_v=ck), dict(cache_k=c["k"].as_strided(ck.shape, (0, 0, 0, 1)))):
+            before = [t.clone().view(torch.int16) for t in (ck, cv)]
+            assert attention_core(**dict(c, cache_k=ck, cache_v=cv) | change) is None, list(change)
+            assert all(torch.equal(a, b.view(torch.int16)) for a, b in zip(before, (ck, cv)))
+        both = torch.stack([ck, cv], dim=2).permute(0, 3, 2, 1, 4).contiguous()  # [B, S, 2, H, D]
+        d = dict(c, cache_k=both[:, :, 0].transpose(1, 2), cache_v=both[:, :, 1].transpose(1, 2))
+        assert torch.equal(attention_core(**d), want)

@@ -166,6 +166,65 @@ def test_argument_errors_return_before_launch():
     assert lib.fp_quantize_w8_per_row(None, 64, None, 64, None, 0, 64, None) == 0
 
 
+class _AttentionArgs(ctypes.Structure):
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("q", "k", "v")]
+                + [(n, ctypes.c_int64) for n in ("ldq", "ldk", "ldv")]
+                + [(n, ctypes.c_void_p) for n in ("q_gamma", "k_gamma", "cos", "sin")]
+                + [(n, ctypes.c_int64) for n in ("ld_cos", "ld_sin")]
+                + [(n, ctypes.c_void_p) for n in ("cache_k", "cache_v")]
+                + [(n, ctypes.c_int64) for n in ("k_s_b", "k_s_h", "k_s_p", "v_s_b", "v_s_h", "v_s_p")]
+                + [("y", ctypes.c_void_p)]
+                + [(n, ctypes.c_int64) for n in ("B", "T", "n_heads", "n_kv_heads", "head_dim",
+                                                 "cache_len", "pos")]
+                + [("pos_dev", ctypes.c_void_p), ("q_eps", ctypes.c_float), ("k_eps", ctypes.c_float)])
+
+
+def _attention_args(B=2, T=3, Hq=4, Hk=2, D=64, S=32, pos=5):
+    """A valid call on addresses that nothing reads: the tests below change one
+    thing, or leave the workspace out, which is looked at last."""
+    n, c = B * T * D, B * Hk * S * D
+    a = _AttentionArgs(q=1 << 20, k=2 << 20, v=3 << 20, ldq=Hq * D, ldk=Hk * D, ldv=Hk * D,
+                       q_gamma=4 << 20, k_gamma=5 << 20, cos=6 << 20, sin=7 << 20, ld_cos=D, ld_sin=D,
+                       cache_k=8 << 20, cache_v=9 << 20, k_s_b=Hk * S * D, k_s_h=S * D, k_s_p=D,
+                       v_s_b=Hk * S * D, v_s_h=S * D, v_s_p=D, y=10 << 20, B=B, T=T, n_heads=Hq,
+                       n_kv_heads=Hk, head_dim=D, cache_len=S, pos=pos, q_eps=1e-6, k_eps=1e-6)
+    assert max(n * Hq, c) * 2 <= 1 << 20
+    return a
+
+
+def _attention_status(**change):
+    from llms_amd import _lib
+
+    a = _attention_args()
+    for k, v in change.items():
+        setattr(a, k, v)
+    return _lib.capi().fp_attention_bf16(ctypes.byref(a), None, 0, None)
+
+
+FP_ERR_NULL, FP_ERR_SHAPE, FP_ERR_STRIDE, FP_ERR_WORKSPACE = 1, 2, 3, 6
+
+
+def test_attention_refuses_overlapping_caches():
+    """Memory that two of a call's workgroups would write, or one write and
+    another read, is refused before any launch; layouts that only interleave,
+    and one sequence or head with any stride, are not (the missing workspace
+    is then what is reported)."""
+    B, Hk, D, S = 2, 2, 64, 32
+    k, v, c = 8 << 20, 9 << 20, 2 * B * Hk * S * D
+    both = lambda **kw: {p + n: x for n, x in kw.items() for p in "kv"}  # noqa: E731
+    inter = both(_s_b=2 * S * Hk * D, _s_p=2 * Hk * D, _s_h=D)  # [B][S][2][heads][D]
+    for ok in (dict(), inter | dict(cache_v=k + 2 * Hk * D), dict(cache_v=k + c),
+               both(_s_b=S * Hk * D, _s_p=Hk * D, _s_h=D), dict(B=1, k_s_b=0), dict(k=k + c),
+               dict(n_kv_heads=1, ldk=D, ldv=D, k_s_h=0, k_s_b=S * D)):
+        assert _attention_status(**ok) == FP_ERR_WORKSPACE, ok
+    for bad in (dict(k_s_b=0), dict(v_s_h=0), dict(cache_v=k), dict(cache_v=k + 16),
+                dict(cache_v=k + c - 16), dict(cache_k=v + 2 * Hk * D), dict(k_s_b=S * D),
+                dict(k_s_h=(S - 1) * D), dict(k_s_p=D + 8), inter | dict(cache_v=k + 2 * D),
+                inter | dict(cache_v=k + 2 * Hk * D, v_s_b=4 * S * Hk * D), dict(k=k + c - 16),
+                dict(q=v), dict(v=v + 64)):
+        assert _attention_status(**bad) == FP_ERR_STRIDE, bad
+
+
 def test_python_wrappers_raise_reference_errors():
     """The wrappers' shape checks run before anything else, with the
     reference's messages (tests/test_kernels_fused_ffn.py:203-229,
