@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import torch
+from torch._C import _functorch
 from torch.autograd import forward_ad
 from torch.nn.modules import module as _module
 
@@ -47,7 +48,10 @@ def plain_norm(m) -> bool:
             and not _module._global_forward_hooks and not _module._global_forward_pre_hooks)
 
 
-def differentiated(*tensors: torch.Tensor) -> bool:
-    """Whether autograd, in either mode, may follow an operation on these."""
+def transformed(*tensors: torch.Tensor) -> bool:
+    """Whether autograd, in either mode, or a torch.func transform (vmap, grad,
+    jvp) may follow an operation on these. What torch does not say about its
+    forward mode counts as yes."""
     return ((torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
-            or getattr(forward_ad, "_current_level", -1) >= 0)
+            or getattr(forward_ad, "_current_level", 0) >= 0
+            or _functorch.peek_interpreter_stack() is not None)

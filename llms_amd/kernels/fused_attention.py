@@ -17,7 +17,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ._checks import differentiated, plain_norm
+from ._checks import plain_norm, transformed
 
 
 def attention_core(q, k, v, *, q_norm, k_norm, num_heads: int, cache_k, cache_v, cos, sin,
@@ -30,7 +30,7 @@ def attention_core(q, k, v, *, q_norm, k_norm, num_heads: int, cache_k, cache_v,
     if (not q.is_cuda or q.dtype != torch.bfloat16 or cache_k.shape[-1] not in (64, 128)
             or not (plain_norm(q_norm) and plain_norm(k_norm))):
         return None
-    if differentiated(q, k, v, q_norm.weight, k_norm.weight, cos, sin, cache_k, cache_v):
+    if transformed(q, k, v, q_norm.weight, k_norm.weight, cos, sin, cache_k, cache_v):
         return None
     if torch.is_tensor(start_pos):
         pos, start = start_pos, 0

@@ -18,8 +18,8 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ._checks import (differentiated, inner_contiguous, plain_norm, require_bf16_hip,
-                      require_device)
+from ._checks import (inner_contiguous, plain_norm, require_bf16_hip, require_device,
+                      transformed)
 
 
 def _check_norm(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, fn: str) -> None:
@@ -129,6 +129,6 @@ def fused_rmsnorm_head(h: torch.Tensor, norm, W: torch.Tensor) -> torch.Tensor |
     if (not h.is_cuda or h.dtype != torch.bfloat16 or W.dtype != torch.bfloat16
             or not 1 <= h.numel() <= 16 * h.shape[-1] or not plain_norm(norm)
             or norm.weight.dtype != torch.bfloat16 or W.device != h.device
-            or differentiated(h, W, norm.weight)):
+            or transformed(h, W, norm.weight)):
         return None
     return fused_rmsnorm_qkv(h, norm.weight, norm.eps, W, n_q=W.shape[0], n_k=0)[0]

@@ -119,3 +119,28 @@ def test_attend_device_position_form(dtype, T, start_pos):
         assert d <= 1e-6
     else:
         assert d <= 2.0 ** -7 * b.double().abs().max().item()
+
+
+def test_transformed_calls_are_seen():
+    """What the attention kernels and the fused head step aside for: autograd in
+    either mode and the torch.func transforms, on any of the operands."""
+    from torch.autograd import forward_ad
+
+    from llms_amd.kernels._checks import transformed
+
+    x, p = torch.ones(3), torch.ones(3, requires_grad=True)
+    seen = []
+
+    def f(t):
+        seen.append(transformed(x, x))
+        return t * 2.0
+
+    assert not transformed(x, x) and transformed(x, p)
+    with torch.no_grad():
+        assert not transformed(x, p)
+        with forward_ad.dual_level():
+            assert transformed(x)
+    torch.func.vmap(f)(x)
+    torch.func.jvp(f, (x,), (x,))
+    torch.func.grad(lambda t: f(t).sum())(x)
+    assert seen == [True] * 3 and not transformed(x)

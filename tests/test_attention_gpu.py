@@ -221,3 +221,39 @@ def test_overlapping_caches_stay_with_the_torch_form():
         both = torch.stack([ck, cv], dim=2).permute(0, 3, 2, 1, 4).contiguous()  # [B, S, 2, H, D]
         d = dict(c, cache_k=both[:, :, 0].transpose(1, 2), cache_v=both[:, :, 1].transpose(1, 2))
         assert torch.equal(attention_core(**d), want)
+
+
+def _module(**swap):
+    """The swapped attention layer of a one-layer model with heads of 64, its
+    cache, an input and the arguments of a step at position 5."""
+    from llms_amd import harness
+    from llms_amd.kernels import apply_triton_kernels
+
+    cfg = harness.Cfg(vocab_size=64, hidden_size=256, num_hidden_layers=1, num_attention_heads=4,
+                      num_key_value_heads=2, head_dim=64, intermediate_size=256,
+                      max_position_embeddings=64)
+    m = apply_triton_kernels(harness.tiny_model(cfg, device=DEV), **swap)
+    g = torch.Generator(device=DEV).manual_seed(6)
+    r = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()  # noqa: E731
+    cache = harness.KVCache([r(1, 2, 32, 64)], [r(1, 2, 32, 64)])
+    kw = dict(layer_idx=0, cos=m.rope_cos[5:8], sin=m.rope_sin[5:8], start_pos=5)
+    return m, cache, r(1, 3, 256), kw
+
+
+def test_vmap_over_the_module():
+    """torch.func.vmap over the layer with a cache per example runs as it does
+    over the torch form: each example's output and cache."""
+    from llms_amd.harness import KVCache
+
+    m, cache, x, kw = _module()
+    xs, ks, vs = (torch.stack([t, t.flip(-1)]) for t in (x, cache.k[0], cache.v[0]))
+
+    def f(x, k, v):
+        return m.layers[0].attn(x, kv_cache=KVCache([k], [v]), **kw), k, v
+
+    with torch.no_grad():
+        want = [f(x, k.clone(), v.clone()) for x, k, v in zip(xs, ks, vs)]
+        got = torch.func.vmap(f)(xs, ks.clone(), vs.clone())
+    for i in range(2):
+        for a, b in zip(got, want[i]):
+            assert (a[i].float() - b.float()).abs().max() <= 2.0 ** -6 * b.float().abs().max()
