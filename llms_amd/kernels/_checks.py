@@ -43,8 +43,9 @@ def inner_contiguous(t: torch.Tensor) -> torch.Tensor:
 
 def plain_norm(m) -> bool:
     """Whether m is the RMSNorm of ``_eager.py`` with nothing attached to its
-    call (a fused kernel may then normalise with its weight and eps)."""
-    return (type(m) is RMSNorm and not m._forward_hooks and not m._forward_pre_hooks
+    call and no ``forward`` of its own set on it (a fused kernel may then
+    normalise with its weight and eps)."""
+    return (type(m) is RMSNorm and "forward" not in m.__dict__ and not m._forward_hooks and not m._forward_pre_hooks
             and not _module._global_forward_hooks and not _module._global_forward_pre_hooks)
 
 

@@ -34,7 +34,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from llms_amd.kernels._eager import attend
+from llms_amd.kernels._eager import RMSNorm, attend
 
 H, HKV, D = 8, 2, 64
 
@@ -144,3 +144,20 @@ def test_transformed_calls_are_seen():
     torch.func.jvp(f, (x,), (x,))
     torch.func.grad(lambda t: f(t).sum())(x)
     assert seen == [True] * 3 and not transformed(x)
+
+
+def test_plain_norm_sees_what_is_attached():
+    """A hooked norm, a subclass and one whose ``forward`` was replaced on the
+    instance are not the plain one."""
+    from llms_amd.kernels._checks import plain_norm
+
+    m = RMSNorm(8)
+    assert plain_norm(m)
+    for register in (m.register_forward_hook, m.register_forward_pre_hook):
+        h = register(lambda *a: None)
+        assert not plain_norm(m)
+        h.remove()
+    m.forward = lambda x: x
+    assert not plain_norm(m)
+    del m.forward
+    assert plain_norm(m) and not plain_norm(type("Sub", (RMSNorm,), {})(8))
