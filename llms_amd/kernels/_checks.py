@@ -56,3 +56,8 @@ def transformed(*tensors: torch.Tensor) -> bool:
     return ((torch.is_grad_enabled() and any(t.requires_grad for t in tensors))
             or getattr(forward_ad, "_current_level", 0) >= 0
             or _functorch.peek_interpreter_stack() is not None)
+
+
+def autocast() -> bool:
+    """Whether torch's autocast would choose the types of a matmul here."""
+    return torch.is_autocast_enabled("cuda")

@@ -6,7 +6,8 @@ projection and before ``o`` (reference ``src/kernels/fused_qkv.py:242-282``) as
 two or three launches (``llms_amd/csrc/fp_attn.hip``), at the rounding points
 of the torch form in ``_eager.py`` and in fp32 between them. It takes bf16
 inference on a HIP device with heads of 64 or 128; every other call (other
-types and head sizes, gradients, a CPU model) is the torch form's.
+types and head sizes, gradients, torch.func transforms, autocast, a CPU model)
+is the torch form's.
 
 Path: wrapper -> ``torch.ops.llms_amd.attention`` -> C ABI
 ``fp_attention_bf16`` -> HIP kernels on torch's current stream.
@@ -17,7 +18,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ._checks import plain_norm, transformed
+from ._checks import autocast, plain_norm, transformed
 
 
 def attention_core(q, k, v, *, q_norm, k_norm, num_heads: int, cache_k, cache_v, cos, sin,
@@ -28,7 +29,7 @@ def attention_core(q, k, v, *, q_norm, k_norm, num_heads: int, cache_k, cache_v,
     max_seq, D]`` at ``start_pos`` (an int, or a 0-dim int64 device tensor) ..;
     None, with nothing written, where the kernels do not take the call."""
     if (not q.is_cuda or q.dtype != torch.bfloat16 or cache_k.shape[-1] not in (64, 128)
-            or not (plain_norm(q_norm) and plain_norm(k_norm))):
+            or not (plain_norm(q_norm) and plain_norm(k_norm)) or autocast()):
         return None
     if transformed(q, k, v, q_norm.weight, k_norm.weight, cos, sin, cache_k, cache_v):
         return None

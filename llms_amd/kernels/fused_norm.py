@@ -18,7 +18,7 @@ from __future__ import annotations
 import torch
 
 from .. import _lib
-from ._checks import (inner_contiguous, plain_norm, require_bf16_hip, require_device,
+from ._checks import (autocast, inner_contiguous, plain_norm, require_bf16_hip, require_device,
                       transformed)
 
 
@@ -124,11 +124,11 @@ def fused_rmsnorm_head(h: torch.Tensor, norm, W: torch.Tensor) -> torch.Tensor |
     """``F.linear(norm(h), W)``, the final norm and output head of a model, on
     the fused kernels at decode and verify row counts (up to 16 rows of h); None
     for the calls that stay with torch: more rows (the library GEMM's), other
-    types and devices, gradients, a norm that is not the plain ``RMSNorm``. One
+    types and devices, gradients, torch.func transforms, autocast, a norm that is not the plain ``RMSNorm``. One
     row of 4B, 151936 x 2560: 109 us against 240 for ``F.linear`` alone."""
     if (not h.is_cuda or h.dtype != torch.bfloat16 or W.dtype != torch.bfloat16
             or not 1 <= h.numel() <= 16 * h.shape[-1] or not plain_norm(norm)
             or norm.weight.dtype != torch.bfloat16 or W.device != h.device
-            or transformed(h, W, norm.weight)):
+            or autocast() or transformed(h, W, norm.weight)):
         return None
     return fused_rmsnorm_qkv(h, norm.weight, norm.eps, W, n_q=W.shape[0], n_k=0)[0]

@@ -257,3 +257,17 @@ def test_vmap_over_the_module():
     for i in range(2):
         for a, b in zip(got, want[i]):
             assert (a[i].float() - b.float()).abs().max() <= 2.0 ** -6 * b.float().abs().max()
+
+
+def test_autocast_keeps_its_types():
+    """Under autocast the layer's core and the head are torch's, with the type
+    that autocast gives a matmul (the model's blocks return theirs in bf16)."""
+    m, cache, x, kw = _module(linear_down_o=True)
+    c = _inputs(4, 1, 2, 4, 2, 64, 32, 5)
+    ids = torch.tensor([[3, 1, 4]], device=DEV)
+    with torch.inference_mode():
+        assert m(ids, m.alloc_cache(32)).dtype == torch.bfloat16
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert m(ids, m.alloc_cache(32)).dtype == torch.float16
+            assert attention_core(**c) is None
+        assert attention_core(**c) is not None
