@@ -311,6 +311,9 @@ at::Tensor attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor&
   for (const at::Tensor* t : {&q, &k, &v, &cos, &sin, (const at::Tensor*)&cache_k,
                               (const at::Tensor*)&cache_v})
     if (!bf16_here(*t)) return none();
+  // torch refuses to write an inference tensor outside inference mode
+  if (!c10::InferenceMode::is_enabled() && (cache_k.is_inference() || cache_v.is_inference()))
+    return none();
   if (!q.is_cuda() || q.dim() != 3 || cache_k.dim() != 4 || cache_v.dim() != 4) return none();
   const int64_t B = q.size(0), T = q.size(1), Hk = cache_k.size(1), S = cache_k.size(2);
   const int64_t D = cache_k.size(3);

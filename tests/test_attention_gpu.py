@@ -271,3 +271,21 @@ def test_autocast_keeps_its_types():
             assert m(ids, m.alloc_cache(32)).dtype == torch.float16
             assert attention_core(**c) is None
         assert attention_core(**c) is not None
+
+
+def test_inference_cache_is_written_in_inference_mode_only():
+    """torch refuses in-place updates of an inference tensor outside inference
+    mode; so does the layer. Other caches are written in either mode, and their
+    version counts the write."""
+    m, cache, x, kw = _module()
+    run = lambda c: m.layers[0].attn(x, kv_cache=c, **kw)  # noqa: E731
+    with torch.inference_mode():
+        inf = type(cache)([cache.k[0].clone()], [cache.v[0].clone()])
+    with torch.no_grad():
+        with pytest.raises(RuntimeError, match="[Ii]nference"):
+            run(inf)
+        version = cache.k[0]._version
+        want = run(cache)
+        assert cache.k[0]._version > version
+    with torch.inference_mode():
+        assert torch.equal(run(inf), want)
