@@ -127,13 +127,16 @@ class DecoderBlock(nn.Module):
 
 
 class Qwen3Model(nn.Module):
+    # Set on a model by apply_triton_kernels(..., linear_down_o=True); on the
+    # class, so that a model saved whole without it loads and runs as it did.
+    fused_head = False
+
     def __init__(self, c: Cfg) -> None:
         super().__init__()
         self.cfg = c
         self.embed = nn.Embedding(c.vocab_size, c.hidden_size)
         self.layers = nn.ModuleList([DecoderBlock(c) for _ in range(c.num_hidden_layers)])
         self.final_norm = RMSNorm(c.hidden_size, eps=c.rms_norm_eps)
-        self.fused_head = False  # set by apply_triton_kernels(..., linear_down_o=True)
         cos, sin = build_rope_tables(c.head_dim, c.max_position_embeddings, c.rope_theta)
         self.register_buffer("rope_cos", cos, persistent=False)
         self.register_buffer("rope_sin", sin, persistent=False)

@@ -125,6 +125,17 @@ def test_apply_linear_down_o_swaps_and_keeps_keys():
         FusedLinear.from_linear(nn.Linear(4, 4, bias=True))
 
 
+def test_fused_head_flag_is_not_part_of_a_saved_model():
+    """A model pickled whole by code that did not know the flag still runs, and
+    the swap sets the flag on the model alone."""
+    m = tiny_model(TINY)
+    assert "fused_head" not in m.__dict__ and not m.fused_head
+    ids = torch.tensor([PROMPTS[0]])
+    assert _logits(m, ids).shape == (1, len(PROMPTS[0]), TINY.vocab_size)
+    assert apply_triton_kernels(m, linear_down_o=True).fused_head
+    assert not tiny_model(TINY).fused_head
+
+
 def test_apply_fuse_norm_moves_the_norms():
     """``fuse_norm=True`` hands each block's norm1 / norm2 module to the fused
     QKV / gate-up module (``prenorm``) and leaves ``nn.Identity`` behind;
