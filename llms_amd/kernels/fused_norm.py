@@ -124,11 +124,16 @@ def fused_rmsnorm_head(h: torch.Tensor, norm, W: torch.Tensor) -> torch.Tensor |
     """``F.linear(norm(h), W)``, the final norm and output head of a model, on
     the fused kernels at decode and verify row counts (up to 16 rows of h); None
     for the calls that stay with torch: more rows (the library GEMM's), other
-    types and devices, gradients, torch.func transforms, autocast, a norm that is not the plain ``RMSNorm``. One
-    row of 4B, 151936 x 2560: 109 us against 240 for ``F.linear`` alone."""
+    types and devices, gradients, torch.func transforms, autocast, a norm that is
+    not the plain ``RMSNorm`` or has another weight shape or eps than the kernels
+    take, a head whose rows are not contiguous (its copy would cost more than the
+    call). One row of 4B, 151936 x 2560: 109 us against 240 for ``F.linear``
+    alone."""
     if (not h.is_cuda or h.dtype != torch.bfloat16 or W.dtype != torch.bfloat16
             or not 1 <= h.numel() <= 16 * h.shape[-1] or not plain_norm(norm)
-            or norm.weight.dtype != torch.bfloat16 or W.device != h.device
+            or norm.weight.dtype != torch.bfloat16 or norm.weight.shape != h.shape[-1:]
+            or not 0.0 <= norm.eps < float("inf") or W.device != h.device
+            or W.dim() != 2 or W.shape[1] != h.shape[-1] or W.stride(1) != 1
             or autocast() or transformed(h, W, norm.weight)):
         return None
     return fused_rmsnorm_qkv(h, norm.weight, norm.eps, W, n_q=W.shape[0], n_k=0)[0]

@@ -299,3 +299,21 @@ def test_norm_and_wide_head(M, K, V):
         assert fused_rmsnorm_head(xd[None], norm, wd) is None
         h.remove()
     assert fused_rmsnorm_head(xd[None], norm, wd) is None  # the weight is a parameter
+
+
+@pytest.mark.gpu
+def test_head_calls_left_to_torch():
+    """What ``F.linear(norm(h), W)`` takes and the kernels do not: a weight that
+    broadcasts, a negative eps, a column-major head; and its own shape error."""
+    from llms_amd.kernels._eager import RMSNorm
+    from llms_amd.kernels.fused_norm import fused_rmsnorm_head
+
+    K, V = 256, 512
+    h, w = (t.to(DEV) for t in (_x(80, 2, K)[None], _x(81, V, K)))
+    norm = lambda n, eps: RMSNorm(n, eps=eps).to(DEV, torch.bfloat16)  # noqa: E731
+    with torch.no_grad():
+        assert fused_rmsnorm_head(h, norm(K, EPS), w) is not None
+        for n, t in ((norm(1, EPS), w), (norm(K, -1e-3), w), (norm(K, float("inf")), w),
+                     (norm(K, EPS), w.T.contiguous().T), (norm(K, EPS), w[:, :-8]),
+                     (norm(K, EPS), w[0])):
+            assert fused_rmsnorm_head(h, n, t) is None
