@@ -144,8 +144,7 @@ int fp_linear_w8(const void* x, int64_t ldx,
  * grid would leave CUs idle while each tile runs a long k loop split k across
  * workgroups: fp32 partial sums go to the workspace and a second kernel sums
  * them in a fixed order and applies the epilogue (results stay
- * deterministic). Above 1024 rows a call may run unsplit and leave the
- * workspace unused. A NULL or smaller workspace runs the unsplit kernels of the
+ * deterministic). A NULL or smaller workspace runs the unsplit kernels of the
  * plain entry points. The workspace must be 16-byte aligned (any hipMalloc or
  * torch allocation is) and is overwritten.
  */

@@ -1638,6 +1638,11 @@ GemmSplit gemm_split_plan_bf16(int64_t M, int64_t N, int64_t K, bool gateup) {
   if (small_round_tile(M, N, K, gateup) >= 0) return GemmSplit{-1, 1};
   if (!gateup && splitk24_shape(M, N, K)) return GemmSplit{-1, 1};  // 24-row split-K tiles
   const GemmSplit p = gemm_split_plan(M, N, K, gateup);
+  // Above 1024 rows, where the split takes 256 x 256 tiles, and up to K = 4096 a
+  // round of the four-wave tiles needs no partials (weights cycled through HBM,
+  // us, split / not: 4B o M = 1200 50.5 / 35.8; with a longer K it loses: 4B down
+  // M = 1200, 1500, 2048 67, 74, 94 / 97, 105, 116, 8B down M = 1200 107 / 149).
+  if (p.tile == kT256x256 && K <= 4096) return GemmSplit{-1, 1};
   if (p.tile < 0 || K % (2 * kBK) != 0) return p;
   // The staged 96 x 64 four-wave tiles (three LDS stages), k split into
   // ranges of 4 to 32 128-wide steps, as many as one round of at most 256
@@ -1662,12 +1667,6 @@ GemmSplit gemm_split_plan_bf16(int64_t M, int64_t N, int64_t K, bool gateup) {
 bool use_gemm_split(const StreamArgs& a, bool aligned, bool gateup, GemmSplit* p) {
   if (!a.ws || !gemm_supported(a, aligned, false)) return false;
   *p = gemm_split_plan_bf16(a.M, a.N, a.K, gateup);
-  // Above 1024 rows, where the split takes 256 x 256 tiles, and up to K = 4096 a
-  // round of the four-wave tiles needs no partials and the workspace stays unused
-  // (weights cycled through HBM, us, split / not: 4B o M = 1200 50.5 / 35.8; with
-  // a longer K it loses: 4B down M = 1200, 1500, 2048 67, 74, 94 / 97, 105, 116, 8B
-  // down M = 1200 107 / 149).
-  if (p->tile == kT256x256 && a.K <= 4096) return false;
   return p->tile >= 0 && gemm_split_ws_floats(*p, a.M, a.N, a.K, gateup) <= a.ws_floats;
 }
 

@@ -116,6 +116,19 @@ def test_workspace_bytes_plan():
     assert planes(32, 2560, 2048) <= 4
 
 
+def test_no_workspace_where_nothing_is_split():
+    """Above 1024 rows and up to K = 4096 no call splits k, so none asks for
+    partials; with a longer K narrow outputs do."""
+    from llms_amd import _lib
+
+    wb = _lib.capi().fp_workspace_bytes
+    for M in (1025, 1200, 2048):
+        for N, K, gu in ((2560, 4096, 0), (3000, 2048, 0), (4096, 4096, 0), (1100, 4096, 1)):
+            assert wb(M, N, K, gu) == 0, (M, N, K)
+            assert _lib.capi().fp_rmsnorm_workspace_bytes(M, N, K, gu, 0) == -(-M * K * 2 // 256) * 256
+        assert wb(M, 2560, 9728, 0) > 0
+
+
 def test_status_strings():
     from llms_amd import _lib
 
