@@ -17,11 +17,9 @@
 //     sums, the other halves are discarded. The MFMA pipe is ~90% idle in this
 //     regime, so the doubled MFMA count is free; x^T (M <= 16*MT columns,
 //     zero-padded) is the B operand.
-//   - K is split across the NW waves of the workgroup, interleaved by k-block
-//     (SPLIT 0) or in contiguous ranges (SPLIT 1). Each wave double-buffers U
-//     k-blocks of loads in registers.
-//   - x is read either from L2 per k-block or, XL, staged once per workgroup
-//     in LDS.
+//   - K is split across the NW waves of the workgroup, interleaved by k-block.
+//     Each wave double-buffers U k-blocks of loads in registers.
+//   - x is read from L2 per k-block.
 //   - The NW partial tiles are summed through LDS in fixed wave order; the
 //     epilogue (bf16 store, or silu(g)*u) runs in registers, so the fp32
 //     intermediate never reaches HBM and results are bit-reproducible.
@@ -56,15 +54,11 @@ __device__ __forceinline__ u32x4 ror8(u32x4 v) {
                (uint32_t)__builtin_amdgcn_mov_dpp((int)v.w, kRowRor8, 0xf, 0xf, false)};
 }
 
-// XL: x is staged once per workgroup in LDS (M rows x K, dynamic shared
-// memory) and the B operand is read from there instead of from L2.
 // XP: packed x operand for M <= 8 (one x load per sub-chunk; the B operand of
 // line half 1 is the half-0 register rotated by 8 lanes).
-template <int NW, int MT, int U, int SPLIT, bool GATEUP, bool W8, bool ALIGNED, bool XL,
-          bool XP = false>
+template <int NW, int MT, int U, bool GATEUP, bool W8, bool ALIGNED, bool XP = false>
 __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
-  static_assert(!XP || (MT == 1 && !XL), "packed x needs M <= 8 and x from L2");
-  static_assert(ALIGNED || (!XL && SPLIT == 0), "unaligned rows: x from L2, interleaved k-blocks");
+  static_assert(!XP || MT == 1, "packed x needs M <= 8");
   using F = Frag<MT, GATEUP, W8, XP>;
   constexpr int XV = F::XV;
   constexpr int SV = W8 ? 2 : 1;           // 8-element sub-chunks per lane per line half
@@ -112,19 +106,8 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
   }
   const int xhalf = XP ? (li >> 3) : 0;
 
-  // k-blocks of this wave
-  int64_t kb_first, kb_stride, nmine;
-  if constexpr (SPLIT == 0) {
-    kb_first = wave;
-    kb_stride = NW;
-    nmine = nkb > wave ? (nkb - wave + NW - 1) / NW : 0;
-  } else {
-    const int64_t per = (nkb + NW - 1) / NW;
-    kb_first = wave * per;
-    kb_stride = 1;
-    const int64_t end = kb_first + per < nkb ? kb_first + per : nkb;
-    nmine = end > kb_first ? end - kb_first : 0;
-  }
+  // k-blocks of this wave: wave, wave + NW, ...
+  const int64_t nmine = nkb > wave ? (nkb - wave + NW - 1) / NW : 0;
 
   // First k of the 8 x values group grp supplies to the MFMA of line half h,
   // sub-chunk s (int8 lines carry two 8-element sub-chunks per lane).
@@ -134,7 +117,7 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
 
   auto load_block = [&](F& f, int64_t j) {
     const bool live = j < nmine;
-    const int64_t kb = kb_first + j * kb_stride;
+    const int64_t kb = wave + j * NW;
     const int64_t kw = kb * KB + chunk * CK;
     const u32x4 z{0, 0, 0, 0};
     if constexpr (!ALIGNED) {
@@ -143,13 +126,11 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
       if (!live) return;
       f.a0 = ld16_any(w0row + kw * (W8 ? 1 : 2));
       if constexpr (GATEUP) f.a1 = ld16_any(w1row + kw * (W8 ? 1 : 2));
-      if constexpr (!XL) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-          for (int v = 0; v < XV; ++v)
-            f.xb[mt][v] = ld16_any(xrow[mt] + xk(kb, XP ? xhalf : v / SV, XP ? v : v % SV));
-      }
+        for (int v = 0; v < XV; ++v)
+          f.xb[mt][v] = ld16_any(xrow[mt] + xk(kb, XP ? xhalf : v / SV, XP ? v : v % SV));
       return;
     }
     if constexpr (W8) {
@@ -161,42 +142,21 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
       if constexpr (GATEUP)
         f.a1 = (live && row_ok) ? load_w_bf16x8<ALIGNED>((const uint16_t*)w1row, kw, K) : z;
     }
-    if constexpr (!XL) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int v = 0; v < XV; ++v) {
-          // packed: v = sub-chunk, half from the lane; else v = h * SV + s
-          const int h = XP ? xhalf : v / SV;
-          const int s = XP ? v : v % SV;
-          f.xb[mt][v] = (live && xok[mt]) ? load_bf16x8<ALIGNED>(xrow[mt], xk(kb, h, s), K) : z;
-        }
-    }
+      for (int v = 0; v < XV; ++v) {
+        // packed: v = sub-chunk, half from the lane; else v = h * SV + s
+        const int h = XP ? xhalf : v / SV;
+        const int s = XP ? v : v % SV;
+        f.xb[mt][v] = (live && xok[mt]) ? load_bf16x8<ALIGNED>(xrow[mt], xk(kb, h, s), K) : z;
+      }
   };
 
-  extern __shared__ __attribute__((aligned(16))) uint16_t xs[];
-  // B operand for line half h, sub-chunk s of m-subtile mt at this wave's
-  // j-th k-block.
-  auto xfrag = [&](const F& f, int mt, int h, int s, int64_t j) -> u32x4 {
-    if constexpr (XP) {
-      return h == 0 ? f.xb[mt][s] : ror8(f.xb[mt][s]);
-    } else if constexpr (XL) {
-      const int64_t k = xk(kb_first + j * kb_stride, h, s);
-      const int m = mt * 16 + li;
-      if (!xok[mt] || k >= K) return u32x4{0, 0, 0, 0};
-      const uint16_t* p = xs + (int64_t)m * K + k;
-      if constexpr (ALIGNED) {
-        return *reinterpret_cast<const u32x4*>(p);
-      } else {
-        uint32_t h[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) h[e] = (k + e < K) ? (uint32_t)p[e] : 0u;
-        return u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16),
-                     h[6] | (h[7] << 16)};
-      }
-    } else {
-      return f.xb[mt][h * SV + s];
-    }
+  // B operand for line half h, sub-chunk s of m-subtile mt.
+  auto xfrag = [&](const F& f, int mt, int h, int s) -> u32x4 {
+    if constexpr (XP) return h == 0 ? f.xb[mt][s] : ror8(f.xb[mt][s]);
+    return f.xb[mt][h * SV + s];
   };
 
   f32x4 acc[NACC];
@@ -205,7 +165,7 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
   // accumulator of (line half h, matrix mat, m-subtile mt)
   auto A = [&](int h, int mat, int mt) -> f32x4& { return acc[(h * NM + mat) * MT + mt]; };
 
-  auto compute_block = [&](const F& f, int64_t j) {
+  auto compute_block = [&](const F& f) {
 #pragma unroll
     for (int mat = 0; mat < NM; ++mat) {
       const u32x4 w = mat == 0 ? f.a0 : f.a1;
@@ -218,14 +178,14 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int h = 0; h < 2; ++h) {
-            A(h, mat, mt) = mfma16(wlo, xfrag(f, mt, h, 0, j), A(h, mat, mt));
-            A(h, mat, mt) = mfma16(whi, xfrag(f, mt, h, 1, j), A(h, mat, mt));
+            A(h, mat, mt) = mfma16(wlo, xfrag(f, mt, h, 0), A(h, mat, mt));
+            A(h, mat, mt) = mfma16(whi, xfrag(f, mt, h, 1), A(h, mat, mt));
           }
       } else {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-          for (int h = 0; h < 2; ++h) A(h, mat, mt) = mfma16(w, xfrag(f, mt, h, 0, j), A(h, mat, mt));
+          for (int h = 0; h < 2; ++h) A(h, mat, mt) = mfma16(w, xfrag(f, mt, h, 0), A(h, mat, mt));
       }
     }
   };
@@ -239,46 +199,12 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
   auto compute_chunk = [&](const F* f, int64_t c) {
 #pragma unroll
     for (int j = 0; j < U; ++j)
-      if (c * U + j < nmine) compute_block(f[j], c * U + j);
+      if (c * U + j < nmine) compute_block(f[j]);
   };
 
   // Prologue: two chunks of weight loads in flight before anything waits.
-  auto prologue = [&]() {
-    if (nchunks > 0) load_chunk(fa, 0);
-    if (nchunks > 1) load_chunk(fb, 1);
-  };
-  if constexpr (XL) {
-    // Stage x[0:M, 0:K] in LDS: issue the global reads of x, then the first
-    // two chunks of weight loads, then write x to LDS (waits only for the x
-    // reads, which were issued first).
-    const int64_t total = a.M * K;
-    constexpr int NT = NW * kWave;
-    if constexpr (ALIGNED) {
-      const int64_t nvec = total / 8;
-      const int64_t per_row = K / 8;
-      constexpr int XR = 4;
-      for (int64_t base = 0; base < nvec; base += (int64_t)NT * XR) {
-        u32x4 t[XR];
-#pragma unroll
-        for (int r = 0; r < XR; ++r) {
-          const int64_t i = base + threadIdx.x + (int64_t)r * NT;
-          t[r] = i < nvec ? ld16(a.x + (i / per_row) * a.ldx + (i % per_row) * 8) : u32x4{0, 0, 0, 0};
-        }
-        if (base == 0) prologue();
-#pragma unroll
-        for (int r = 0; r < XR; ++r) {
-          const int64_t i = base + threadIdx.x + (int64_t)r * NT;
-          if (i < nvec) *reinterpret_cast<u32x4*>(xs + i * 8) = t[r];
-        }
-      }
-    } else {
-      prologue();
-      for (int64_t i = threadIdx.x; i < total; i += NT) xs[i] = a.x[(i / K) * a.ldx + (i % K)];
-    }
-    __syncthreads();
-  } else {
-    prologue();
-  }
+  if (nchunks > 0) load_chunk(fa, 0);
+  if (nchunks > 1) load_chunk(fb, 1);
   // Steady state: while one chunk is consumed the other is in flight; a
   // consumed buffer is refilled with the chunk two ahead.
   for (int64_t c = 0; c < nchunks; c += 2) {
@@ -306,7 +232,7 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
 #pragma unroll
         for (int v = 0; v < XV; ++v)
           f.xb[mt][v] = load_bf16x8<false>(xrow[mt], xk(nkb, XP ? xhalf : v / SV, XP ? v : v % SV), K);
-      compute_block(f, 0);
+      compute_block(f);
     }
   }
 
@@ -368,18 +294,14 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
   }
 }
 
-// Dynamic LDS bytes an XL launch needs for x (M rows of K bf16).
-inline size_t xl_bytes(const StreamArgs& a) { return (size_t)a.M * (size_t)a.K * 2; }
-
-template <int NW, int MT, int U, int SPLIT, bool GATEUP, bool W8, bool XL, bool XP = false>
+template <int NW, int MT, int U, bool GATEUP, bool W8, bool XP = false>
 int launch_stream_cfg(const StreamArgs& a, bool aligned, hipStream_t s) {
   const dim3 grid((unsigned)((a.N + 7) / 8));
   const dim3 block(NW * kWave);
-  const size_t shm = XL ? xl_bytes(a) : 0;
   if (aligned)
-    hipLaunchKernelGGL((stream_kernel<NW, MT, U, SPLIT, GATEUP, W8, true, XL, XP>), grid, block, shm, s, a);
+    hipLaunchKernelGGL((stream_kernel<NW, MT, U, GATEUP, W8, true, XP>), grid, block, 0, s, a);
   else
-    hipLaunchKernelGGL((stream_kernel<NW, MT, U, SPLIT, GATEUP, W8, false, XL, XP>), grid, block, shm, s, a);
+    hipLaunchKernelGGL((stream_kernel<NW, MT, U, GATEUP, W8, false, XP>), grid, block, 0, s, a);
   return (int)hipGetLastError();
 }
 
@@ -434,9 +356,9 @@ int launch_stream(const StreamArgs& a, bool aligned, hipStream_t s) {
     return launch_tiled<GATEUP, W8>(a, aligned, s);
   // (int8 dequantisation needs registers of its own: 2 k-blocks per buffer)
   constexpr int U8 = (GATEUP && !W8) ? 4 : 2;
-  if (a.M <= 8) return launch_stream_cfg<4, 1, U8, 0, GATEUP, W8, false, true>(a, aligned, s);
-  if (a.M <= 16) return launch_stream_cfg<4, 1, 2, 0, GATEUP, W8, false>(a, aligned, s);
-  return launch_stream_cfg<4, 2, 2, 0, GATEUP, W8, false>(a, aligned, s);
+  if (a.M <= 8) return launch_stream_cfg<4, 1, U8, GATEUP, W8, true>(a, aligned, s);
+  if (a.M <= 16) return launch_stream_cfg<4, 1, 2, GATEUP, W8>(a, aligned, s);
+  return launch_stream_cfg<4, 2, 2, GATEUP, W8>(a, aligned, s);
 }
 
 template int launch_stream<false, false>(const StreamArgs&, bool, hipStream_t);
