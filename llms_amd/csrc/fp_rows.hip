@@ -595,15 +595,15 @@ int launch_rows_m(const StreamArgs& a, hipStream_t s) {
 }
 
 // Calls that rows_narrow_kernel takes from rows_kernel: where the latter's
-// workgroups of eight rows leave three eighths or more of their rounds idle (at N
-// = 3000, a quarter idle, K = 2560: 4.79 against 5.00; at N = 4096, two full
-// rounds, 8B o 7.44 against 7.72, two rows 7.94 against 11.27), K long enough to give the eight waves work (0.6B o, K
-// = 2048: 2.99 against 3.12; int8, half the bytes, 0.6B down, K = 3072: 3.30
-// against 3.35) and within their chunks, byte offsets below 2^31.
+// workgroups of eight rows leave three eighths or more of their last round idle
+// (up to 1280 outputs, and 2049 to 2560. At N = 3000, a quarter idle, K = 2560: 4.79
+// against 5.00; at N = 4096, two full rounds, 8B o 7.44 against 7.72, two rows
+// 7.94 against 11.27), K long enough to give the eight waves work (0.6B o, K =
+// 2048: 2.99 against 3.12; int8, half the bytes, 0.6B down, K = 3072: 3.30 against
+// 3.35) and within their chunks, byte offsets below 2^31.
 template <bool W8>
 bool narrow_rows(const StreamArgs& a) {
-  const int64_t wgs = (a.N + 7) / 8, rounds = (wgs + 255) / 256;
-  return !a.gamma && a.M <= 2 && a.N <= 3072 && 8 * wgs <= 5 * 256 * rounds &&
+  return !a.gamma && a.M <= 2 && (a.N <= 1280 || (a.N > 2048 && a.N <= 2560)) &&
          a.K >= (W8 ? 4096 : 2560) && a.K <= kNarrowChunks * 8 * 512 &&
          (a.N * a.ldw0 + a.K) * (W8 ? 1 : 2) < ((int64_t)1 << 31);
 }
@@ -620,8 +620,7 @@ int launch_narrow(const StreamArgs& a, hipStream_t s) {
   const int64_t need = (a.N + 511) / 512;
   if (need <= 2) return launch_narrow_cfg<2, MM, W8>(a, s);
   if (need <= 3) return launch_narrow_cfg<3, MM, W8>(a, s);
-  if (need <= 5) return launch_narrow_cfg<5, MM, W8>(a, s);
-  return launch_narrow_cfg<6, MM, W8>(a, s);
+  return launch_narrow_cfg<5, MM, W8>(a, s);
 }
 
 template <bool GATEUP, bool W8>

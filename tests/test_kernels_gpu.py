@@ -1130,11 +1130,10 @@ def test_tile_loops_few_ksteps(K):
            f"int8 gate-up M={M} K={K}")
 
 
-# (M, K, N): one and two x rows on whole rows split over eight waves (K of every
-# chunk count from 5 to 24, a last chunk partly past the row, the first K past
-# the limit; N below, at and past 2, 3, 5 and 6 rows per workgroup, a partial last
-# workgroup), and the 16- and 32-row split-K tiles at their row edges, one past one
-# round of the chip (2560 columns at 65-128 rows: 32-row tiles; 1024: 16-row)
+# (M, K, N): one and two x rows around the whole-row kernel's limits (N 2048 / 2049,
+# 2560 / 2561 and up to 1280; the first K past the limit; most of these run rows_kernel,
+# NARROW_PARTIAL the other), and the 16- and 32-row split-K tiles at their row edges, one
+# past one round of the chip (2560 columns at 65-128 rows: 32-row tiles; 1024: 16-row)
 NARROW = [(1, 2560, 2560), (2, 4104, 2555), (1, 9728, 2561), (2, 12288, 1300), (1, 12296, 1300),
           (1, 4096, 1000), (2, 8192, 1025), (1, 2568, 7), (2, 5000, 2657), (1, 4112, 1328),
           (3, 1024, 4096), (16, 2048, 2555), (17, 2112, 4095), (32, 4096, 1000), (33, 2560, 2560),
@@ -1163,9 +1162,10 @@ def test_narrow_outputs(M, K, N):
 # (M, K, N) on whole rows split over eight waves whose last workgroup is partial: 1-4
 # of five rows past N, 1-2 of three, 1 of two; the first, second and third K chunk of a
 # wave partly past the row, the largest K and the first past it (K a multiple of 16: the
-# int8 kernel takes the call too)
+# int8 kernel takes the call too); both sides of the widths it takes
 NARROW_PARTIAL = [(1, 2576, 2551), (2, 4112, 2552), (1, 8208, 2053), (2, 9744, 2559),
-                  (1, 12288, 2051), (1, 12304, 2051), (2, 4112, 1027), (1, 8208, 1028), (1, 5008, 513)]
+                  (1, 12288, 2051), (1, 12304, 2051), (2, 4112, 1027), (1, 8208, 1028), (1, 5008, 513),
+                  (1, 4096, 1280), (2, 4096, 1281), (1, 4096, 2048), (2, 4096, 2049), (1, 4096, 2560)]
 
 
 @pytest.mark.parametrize("M,K,N", NARROW_PARTIAL)
