@@ -1198,70 +1198,89 @@ int split_ref_tile(int64_t M, int64_t wrows) {
   return M <= 1536 ? kT128x128 : kT256x256;
 }
 
-// Cost model of an unsplit prefill grid, fitted to warm-clock measurements on
-// MI355X (Qwen3-0.6B/4B/8B QKV, gate-up, o and down, M = 256..8192; the
-// dispatch it yields is within 0.1% of the best of the candidates below on
-// average over those 120 shapes, 4% at worst). A grid's time is set by its busiest CU,
-// which runs k = ceil(tiles / 256) tiles; what a tile costs hardly depends on
-// how many other CUs are busy. 256 x 256, 192 x 256 and 320 x 256 tiles (one per CU)
-// cost k times (per-k-step + per-tile) units; tiles that fit two per CU run
-// in pairs: k / 2 pairs and k % 2 single tiles, each with its own per-k-step
-// cost (a pair costs ~1.1-1.3 times a single), plus a per-tile cost. Units
-// are relative (a common per-shape factor is divided out). 192 x 256 tiles
-// (3/4 of the work of 256 x 256) take ~0.92 of the time: they pay where their
-// count fills whole rounds (QKV 6144 x 2048: 256 tiles, 69.4 -> 63.0 us).
+// Cost model of an unsplit prefill grid, fitted to measurements on MI355X. A
+// grid's time is set by its busiest CU, which runs k = ceil(tiles / 256) tiles;
+// what a tile costs hardly depends on how many other CUs are busy. Tiles of one
+// per CU cost k times (per-k-step + per-tile) units; tiles that fit two per CU run
+// in pairs: k / 2 pairs and k % 2 single tiles, each with its own per-k-step cost,
+// plus a per-tile cost. Units are relative (a common per-shape factor is divided
+// out), of int8 and bf16 separately.
 struct TileCost {
   double single, pair, tile;
 };
-constexpr TileCost kCost64x128{0.576, 0.598, 0.0};
-constexpr TileCost kCost128x128{0.616, 0.765, 1.085};
-constexpr TileCost kCost256x256{1.086, 0.0, 7.200};
-constexpr TileCost kCost192x256{0.948, 0.0, 4.843};
-constexpr TileCost kCost320x256{1.331, 0.0, 7.814};
-constexpr double kCostLaunch = 1.925;  // the tail plan's second launch
-// bf16: the four-wave tiles with three weight stages (one unit is about 1.36 us):
-// 256 x 256 4B QKV M = 2048 56.4 us, 8B down M = 4096 272, 192 x 256 4B QKV M =
-// 2048 52.2, 8B QKV M = 4096 154, 192 x 128 4096 -> 3072 at 2048 rows 44.4, 160 x
-// 128 4B o M = 2048 41.1.
-// The gate-up epilogue of 256 x 256 costs six units more (4B M = 2048 in two
-// rounds 137.5, 8B M = 4096 in six 574). With under 32 k-steps (0.6B) 256 x 256 and
-// 192 x 256 keep eight waves: 4096 x 1024 at 4096 rows 33.0 against 33.9.
-constexpr TileCost kCostW256x256{0.87, 0.0, 8.5};
-constexpr TileCost kCostW192x256{0.79, 0.0, 6.0};
-constexpr TileCost kCostW256x128{0.54, 0.0, 6.0};
-constexpr TileCost kCostW192x128{0.42, 0.0, 6.0};
-constexpr TileCost kCostW160x128{0.37, 0.0, 6.5};
+// int8: Qwen3-0.6B/4B/8B QKV, gate-up, o and down, M = 256..8192; within 0.1% of
+// the best candidate on average over those 120 shapes.
+constexpr TileCost kCost8_64x128{0.576, 0.598, 0.0};
+constexpr TileCost kCost8_128x128{0.616, 0.765, 1.085};
+constexpr TileCost kCost8_256x256{1.086, 0.0, 7.200};
+constexpr TileCost kCost8_192x256{0.948, 0.0, 4.843};
+constexpr double kCost8Launch = 1.925;  // the tail plan's second launch
+// bf16, in us (QKV-like outputs, then gate-up, whose epilogue is longer): every
+// tile forced over 1400 drawn and Qwen3 shapes, M = 200..9000, N = 512..13000, K =
+// 512..12288. 64 x 128 and 128 x 128 are gemm_kernel's, 320 x 256 eight waves,
+// the others four waves with three weight stages; under 32 k-steps 256 x 256 and
+// 192 x 256 run eight waves (launch_gemm_tile) and have a cost of their own. The
+// three small four-wave tiles carry 4% against the model's spread, so that they
+// replace another plan only where they clearly win. Against the plans without
+// four-wave tiles: 0.91 of the time on average over 1290 of those shapes, over 6%
+// slower on two. One set of costs from a few 4B and 8B shapes, used at every K,
+// was over 6% slower on 31 (us without four-wave tiles, with that set, now):
+// gate-up of 9248 outputs, K = 1024 at 1559 rows 62.6, 86.2, 63.3; 10688 at 513
+// rows 32.4, 44.1, 33.1; 10936, K = 5120 at 609 rows 140, 163, 137.
+constexpr TileCost kCost64x128[2] = {{0.69, 0.73, 2.6}, {0.67, 0.70, 5.0}};
+constexpr TileCost kCost128x128[2] = {{0.74, 0.99, 3.9}, {0.73, 0.97, 7.4}};
+constexpr TileCost kCost320x256[2] = {{1.48, 0.0, 10.9}, {1.39, 0.0, 19.8}};
+constexpr TileCost kCost256x256[2] = {{1.01, 0.0, 16.0}, {1.00, 0.0, 18.5}};
+constexpr TileCost kCost192x256[2] = {{0.81, 0.0, 13.1}, {0.81, 0.0, 15.6}};
+constexpr TileCost kCost256x256Short[2] = {{1.38, 0.0, 6.7}, {1.30, 0.0, 14.2}};
+constexpr TileCost kCost192x256Short[2] = {{1.22, 0.0, 5.3}, {1.14, 0.0, 11.9}};
+constexpr TileCost kCost256x128[2] = {{0.73, 0.0, 7.1}, {0.73, 0.0, 10.4}};
+constexpr TileCost kCost192x128[2] = {{0.62, 0.0, 5.2}, {0.61, 0.0, 8.1}};
+constexpr TileCost kCost160x128[2] = {{0.58, 0.0, 4.6}, {0.57, 0.0, 6.7}};
+constexpr double kCostLaunch = 2.6;
+constexpr int64_t kShortSteps = 32;  // k-steps from which the two largest run four waves
+
+const TileCost& tile_cost(int tile, int64_t nkt, bool gateup, bool bf16) {
+  if (!bf16)
+    return tile == kT64x128    ? kCost8_64x128
+           : tile == kT128x128 ? kCost8_128x128
+           : tile == kT192x256 ? kCost8_192x256
+                               : kCost8_256x256;
+  const bool few = nkt < kShortSteps;
+  switch (tile) {
+    case kT64x128: return kCost64x128[gateup];
+    case kT128x128: return kCost128x128[gateup];
+    case kT320x256: return kCost320x256[gateup];
+    case kT192x256: return few ? kCost192x256Short[gateup] : kCost192x256[gateup];
+    case kT256x128: return kCost256x128[gateup];
+    case kT192x128: return kCost192x128[gateup];
+    case kT160x128: return kCost160x128[gateup];
+    default: return few ? kCost256x256Short[gateup] : kCost256x256[gateup];
+  }
+}
 
 double grid_cost(int tile, int64_t M, int64_t N, int64_t nkt, bool gateup, bool bf16) {
   const int64_t n = tile_count(tile, M, N, gateup);
   if (n == 0) return 0.0;
   const int64_t k = (n + kCUs - 1) / kCUs;
-  const TileCost& c = tile == kT64x128    ? kCost64x128
-                      : tile == kT128x128 ? kCost128x128
-                      : tile == kT192x256 ? (bf16 ? kCostW192x256 : kCost192x256)
-                      : tile == kT320x256 ? kCost320x256
-                      : tile == kT256x128 ? kCostW256x128
-                      : tile == kT192x128 ? kCostW192x128
-                      : tile == kT160x128 ? kCostW160x128
-                                          : (bf16 ? kCostW256x256 : kCost256x256);
-  const double extra = bf16 && gateup && tile == kT256x256 ? 6.0 : 0.0;
-  if (kTiles[tile].per_cu == 1) return (double)k * ((double)nkt * c.single + c.tile + extra);
+  const TileCost& c = tile_cost(tile, nkt, gateup, bf16);
+  if (kTiles[tile].per_cu == 1) return (double)k * ((double)nkt * c.single + c.tile);
   const int64_t pairs = k / 2, singles = k % 2;
   return (double)nkt * ((double)pairs * c.pair + (double)singles * c.single) +
          (double)(pairs + singles) * c.tile;
 }
 
 // The unsplit plan: for bf16 weights a single round of k-step-128 tiles where
-// one fits (k128_tile); otherwise the cheapest of 64 x 128, 128 x 128,
-// 256 x 256, 192 x 256, 320 x 256 (bf16, at most two rounds: 11% more bytes
-// per k-step than 256 x 256 for 25% more work, which pays where it saves a
-// round: 4B gate-up M = 2048 195.6 -> 184.4 us, M = 1024 116.7 -> 99.5 us;
-// 4B QKV M = 3072 104.8 -> 83.8 us), and
-// "256 x 256 for whole rounds + a 128 x 128 tail" (nmain > 0: the first
-// nmain output columns as whole 256 x 256 rounds, the rest as 128 x 128 tiles
-// in a second launch). The tail form turns the last partial round of 256 x
-// 256 tiles into 128 x 128 tiles that spread over all CUs (measured 4B
-// gate-up M = 2048: 223.6 -> 203.4 us; 4B QKV M = 4096: 142.7 -> 125.9 us).
+// one fits (k128_tile) or of four-wave tiles; otherwise the cheapest of 64 x 128,
+// 128 x 128, 256 x 256, 192 x 256, for bf16 also 320 x 256 (11% more bytes per
+// k-step than 256 x 256 for 25% more work, which pays where it saves a round: 4B
+// gate-up M = 1024 116.7 -> 99.5 us, 4B QKV M = 3072 104.8 -> 83.8), 256 x 128, 192
+// x 128 and 160 x 128, and "256 x 256 for whole rounds + a tail" (nmain > 0: the
+// first nmain output columns as whole 256 x 256 rounds, the rest on the cheapest
+// tile for them, 128 x 128 for int8, in a second launch). The tail form turns the
+// last partial round of 256 x 256 tiles into tiles that spread over all CUs
+// (measured with 128 x 128: 4B gate-up M = 2048 223.6 -> 203.4 us; 4B QKV M = 4096
+// 142.7 -> 125.9).
 // Both tiles contract every output over the same k-steps in the same order,
 // so each plan's result is bit-identical to the others'. One correction to
 // the model: where 128 x 128 tiles would run one per CU and 64 x 128 tiles at
@@ -1412,7 +1431,8 @@ GemmPlan gemm_plan_unsplit(int64_t M, int64_t N, int64_t K, bool gateup, bool bf
     double ctail;
     int tail = cheapest(N - nmain, &ctail);
     if (!bf16) tail = kT128x128, ctail = grid_cost(tail, M, N - nmain, nkt, gateup, false);
-    const double c = grid_cost(kT256x256, M, nmain, nkt, gateup, bf16) + ctail + kCostLaunch;
+    const double c = grid_cost(kT256x256, M, nmain, nkt, gateup, bf16) + ctail +
+                     (bf16 ? kCostLaunch : kCost8Launch);
     if (c < cbest) best = GemmPlan{kT256x256, nmain, tail}, cbest = c;
   }
   const auto per_cu = [&](int t) { return (tile_count(t, M, N, gateup) + kCUs - 1) / kCUs; };
@@ -1475,10 +1495,10 @@ int launch_gemm_tile(const StreamArgs& a, int tile, hipStream_t s) {
       // cannot be split into whole gate/up pairs per wave column take one wave
       // column)
       case kT256x256:
-        if (a.K < 32 * kBK) return launch_tiles_cfg<256, 256, 4, 2, GATEUP>(a, s);
+        if (a.K < kShortSteps * kBK) return launch_tiles_cfg<256, 256, 4, 2, GATEUP>(a, s);
         return launch_w3_cfg<256, 256, 2, 2, GATEUP>(a, s);
       case kT192x256:
-        if (a.K < 32 * kBK) return launch_tiles_cfg<192, 256, 2, 4, GATEUP>(a, s);
+        if (a.K < kShortSteps * kBK) return launch_tiles_cfg<192, 256, 2, 4, GATEUP>(a, s);
         return launch_w3_cfg<192, 256, 2, 2, GATEUP>(a, s);
       case kT256x128: return launch_w3_cfg<256, 128, 4, 1, GATEUP>(a, s);
       case kT192x128: return launch_w3_cfg<192, 128, 2, 2, GATEUP>(a, s);

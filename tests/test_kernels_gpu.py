@@ -1246,8 +1246,7 @@ def test_quantise_rows_of_any_size_and_alignment(K):
 
 # (op, M, K, N) that run each four-wave tile with three weight stages: fewer k-steps
 # than stages would hold is not planned (32 at least for the two largest), odd and even
-# step counts, several tiles per workgroup, partial tiles both ways, the two-launch
-# form with its tail
+# step counts, several tiles per workgroup, partial tiles both ways
 W3_TILES = [
     ("linear", 4090, 2112, 4090),    # 256 x 256, odd step count, one round
     ("linear", 2040, 2560, 6140),    # 192 x 256
@@ -1259,12 +1258,24 @@ W3_TILES = [
     ("gate-up", 510, 2560, 4860),    # 160 x 128, one wave column
     ("gate-up", 500, 2560, 9700),    # 160 x 256, one wave column
     ("gate-up", 250, 4096, 12280),   # 192 x 128
-    ("gate-up", 1000, 4096, 8000),   # 256 x 256 or its tail form
-    ("linear", 4000, 2112, 6100),    # more than a round
+    ("gate-up", 1000, 4096, 8000),   # 256 x 256
+    ("linear", 4000, 2112, 6100),    # 192 x 256, more than a round
+    ("gate-up", 305, 2112, 8342),    # 256 x 128, one wave column per 64 weight rows
+    ("gate-up", 392, 2176, 5533),    # 192 x 128, odd output width
+]
+# ... and whole 256 x 256 rounds (from 32 k-steps four waves, below eight) followed by
+# each tail tile in a second launch
+TAIL_TILES = [
+    ("gate-up", 1545, 2048, 5795), ("linear", 2072, 2048, 9005),   # 160 x 128
+    ("gate-up", 1542, 2048, 6147), ("linear", 2097, 2048, 9620),   # 192 x 128
+    ("gate-up", 1566, 2048, 7245), ("linear", 2830, 2048, 8210),   # 192 x 256
+    ("gate-up", 1124, 2048, 9952), ("linear", 2581, 2048, 8833),   # 256 x 128
+    ("gate-up", 1570, 512, 7032), ("linear", 2632, 576, 8939),     # 128 x 128
+    ("gate-up", 1305, 512, 6736), ("linear", 2056, 512, 8962),     # 64 x 128
 ]
 
 
-@pytest.mark.parametrize("op,M,K,N", W3_TILES)
+@pytest.mark.parametrize("op,M,K,N", W3_TILES + TAIL_TILES)
 def test_three_weight_stage_tiles(op, M, K, N):
     """Against the oracle on rows at the tiles' edges, bit-identical on a second
     call, and bit-identical to the same rows computed as part of a smaller
