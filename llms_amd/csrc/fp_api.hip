@@ -163,23 +163,38 @@ int64_t w8_workspace_bytes(int64_t M, int64_t N, int64_t K, bool gateup) {
 }
 
 // Where the rows kernel, if it takes the call, also normalises. Every one of its
-// workgroups (N / 8 of them, several rounds for gate-up) repeats the norm of all
-// the rows behind two barriers, which costs more with each element of x, while a
-// launch of rmsnorm_kernel costs 2-3.5 us once and lets the plain dispatch choose
-// its kernel (int8 from 2 rows: fp_xpanel.hip). One box, 12 weight sets in a
-// graph, us, in the rows kernel / as its own launch: bf16 one row, 4B QKV 8.70 /
-// 9.17, gate-up 18.05 / 18.85, 8B 10.89 / 12.50, 32.19 / 34.13; two rows, 0.6B
-// (K = 1024) 5.14 / 5.97, 6.60 / 7.28, 4B 10.94 / 10.37, 22.32 / 20.35, 8B 13.95 /
-// 13.14, 38.39 / 34.59; int8 one row, 0.6B 4.33 / 5.27, 5.49 / 5.95, 4B 8.37 /
-// 8.54, 16.24 / 13.55, 8B 9.84 / 9.67, 23.96 / 22.12; two rows, 0.6B 4.87 / 5.88,
-// 6.97 / 7.16, 4B 10.21 / 9.46, 20.69 / 19.29; three and four rows, 0.6B 6.90-8.80 /
-// 6.35-7.28, 4B 14.3-14.8 / 9.4-9.6, 29.7-31.2 / 19.3-19.4. A tied head's thousands
-// of workgroups repeat it too often: 151936 x 2560 at one row 120 / 109.
+// workgroups (N / 8 of them) repeats the norm of all the rows behind two barriers,
+// which costs more with each element of x and each round of workgroups, while a
+// launch of rmsnorm_kernel costs 1-3.5 us once and lets the plain dispatch choose
+// its kernel (int8 from 2 rows: fp_xpanel.hip). Graph of 2-24 weight sets, us, in
+// the rows kernel / as its own launch:
+//   one bf16 row: 4B QKV 8.70 / 9.17, gate-up 18.05 / 18.85, 8B 10.89 / 12.50, 32.19
+//   / 34.13. A tied head's thousands of workgroups repeat it too often (151936 x
+//   2560 120 / 109; 43871 x 2048 33.2 / 31.8) but for the longest rows (96529 x 4096
+//   122.7 / 124.9).
+//   one round of workgroups (N <= 2048): two bf16 rows, 1596 x 2048 5.21 / 5.84,
+//   gate-up 711 x 2560 6.71 / 7.45, 1779 x 3072 6.49 / 7.12, but 270 x 3072 5.80
+//   / 5.39; int8 949 x 3072 4.58 / 5.59, two rows, gate-up 755 x 2048 7.40 / 8.22 (the
+//   kernel takes K in chunks of 1024: 1668 x 1536 7.67 / 7.40), four rows 885 x 1024
+//   5.02 / 5.38.
+//   more rounds: two bf16 rows 4B QKV 10.94 / 10.37, gate-up 22.32 / 20.35, 0.6B (K =
+//   1024) 5.14 / 5.97, 6.60 / 7.28, 3731 x 1536 6.39 / 6.93; one int8 row 0.6B 4.33 /
+//   5.27, 5.49 / 5.95, 3416 x 4096 7.38 / 7.77, 4B 8.37 / 8.54, gate-up 16.24 / 13.55,
+//   8B 9.84 / 9.67, 23.96 / 22.12; two 4B 10.21 / 9.46, 20.69 / 19.29; three and four
+//   14.3-14.8 / 9.4-9.6, 29.7-31.2 / 19.3-19.4.
 template <bool GATEUP, bool W8>
 bool norm_in_rows(int64_t M, int64_t N, int64_t K) {
-  if (N > 32768) return false;
-  if (W8) return M <= 2 && M * K <= (GATEUP ? 2048 : 2560);
-  return M == 1 || M * K <= 2048;
+  const int64_t x = M * K;
+  if (N > 32768) return !W8 && !GATEUP && M == 1 && K > 3072;
+  if (!W8) {
+    if (M == 1 || x <= 2048) return true;
+    if (N <= 2048) return GATEUP || x <= 5120 || N > 1024;
+    return !GATEUP && N <= 4096 && x <= 3072;
+  }
+  if (M <= 2 && x <= (GATEUP ? 2048 : 2560)) return true;
+  if constexpr (GATEUP) return N <= 2048 && M > 1 && K % 1024 == 0 && K <= (M == 2 ? 3072 : 2048);
+  if (M == 1) return N <= 4096;
+  return N <= 2048 && K <= (M == 2 ? 3072 : 1024);
 }
 
 // RMSNorm prologue + projection: one launch on the rows kernel (x normalised

@@ -272,6 +272,28 @@ def test_norm_in_rows_or_apart(M, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,K,N", [(2, 2560, 2048), (2, 2560, 2056), (2, 3072, 1024), (2, 3072, 1032),
+                                   (2, 1536, 4096), (2, 1536, 4104), (1, 4096, 4096), (1, 4096, 4104),
+                                   (3, 1024, 2048), (4, 2048, 2048), (1, 4096, 32800)])
+def test_norm_in_rows_or_apart_by_width(M, K, N):
+    """The same at the widths where the rule changes, bf16 and int8."""
+    kern = _kern()
+    check_norm_qkv(M, K, N - 32, 16, seed=90 + K + M)
+    if N <= 4104:
+        check_norm_gate_up(M, K, N // 2, seed=91 + K + M)
+    x, g = _x(92, M, K), _norm_weight(93, K)
+    _, w = qkv_inputs(94, 1, K, N, 0)
+    q, s = kern.quantize_w8_per_row(w.to(DEV))
+    wq = ref.dequant_w8(q.cpu().numpy(), s.cpu().numpy())
+    y = kern.fused_rmsnorm_qkv_w8(x.to(DEV), g.to(DEV), EPS, q, s, n_q=N, n_k=0)[0]
+    _check(y.cpu(), ref.ref_rmsnorm_qkv_full(bits(x), bits(g), EPS, wq, N, 0), f"int8 norm+qkv {M} {K} {N}")
+    h = N // 2
+    y = kern.fused_rmsnorm_gate_up_silu_w8(x.to(DEV), g.to(DEV), EPS, q[:h], s[:h], q[h:], s[h:])
+    _check(y.cpu(), ref.ref_rmsnorm_gate_up_silu_full(bits(x), bits(g), EPS, wq[:h], wq[h:]),
+           f"int8 norm+gate-up {M} {K} {h}")
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,K,V", [(1, 256, 40000), (2, 1024, 33000), (3, 2560, 8200), (8, 2560, 8201),
                                    (9, 4096, 8320), (16, 1024, 10000), (17, 256, 9000),
                                    (33, 256, 8300)])
