@@ -188,12 +188,12 @@ bool norm_in_rows(int64_t M, int64_t N, int64_t K) {
   if (N > 32768) return !W8 && !GATEUP && M == 1 && K > 3072;
   if (!W8) {
     if (M == 1 || x <= 2048) return true;
-    if (N <= 2048) return GATEUP || x <= 5120 || N > 1024;
+    if (N <= 2048) return x <= (GATEUP || N > 1024 ? 8192 : 5120);
     return !GATEUP && N <= 4096 && x <= 3072;
   }
   if (M <= 2 && x <= (GATEUP ? 2048 : 2560)) return true;
   if constexpr (GATEUP) return N <= 2048 && M > 1 && K % 1024 == 0 && K <= (M == 2 ? 3072 : 2048);
-  if (M == 1) return N <= 4096;
+  if (M == 1) return N <= 4096 && K <= 4096;
   return N <= 2048 && K <= (M == 2 ? 3072 : 1024);
 }
 
