@@ -412,14 +412,21 @@ int launch_splitk(const StreamArgs& a, hipStream_t s) {
     if (a.M <= 16 && a.N > 4096 && a.N <= 8192 && a.K >= 2048 && a.K <= 3072)
       return launch_splitk_cfg<32, 16, 8, 2, false, W8>(a, s);
     // Wide outputs (a tied head: thousands of tiles) up to 32 rows: each tile
-    // reads the x rows again, so more weight rows per tile, fewer of them with
-    // a long K at up to 8 rows. One box, us, against the 16-row (from 17 rows
-    // 32-row) tiles: 151936 x 2560 at 8, 16, 24 rows 128.5, 160.4, 188.4 ->
-    // 121.6, 133.7, 158.6; 32000 x 4096 at 16, 32 rows 48.2, 58.4 -> 45.2, 53.8;
-    // 151936 x 4096 at 8 rows stays (193 against 205).
-    if (a.N > 8192 && a.M <= 32) {
-      if (a.M > 16) return launch_splitk_cfg<64, 32, 4, 2, false, W8>(a, s);
-      if (a.K <= 3072 || a.M > 8) return launch_splitk_cfg<32, 16, 4, 3, false, W8>(a, s);
+    // reads the x rows again, so more weight rows per tile, where their rounds
+    // fill the chip. Over 400 drawn shapes, time against the 16-row (from 17 rows
+    // 32-row) tiles: from 17 rows 0.79-0.96 but for 257-384 tiles (a second round
+    // half empty or more: 1.01-1.06). Up to 16 rows 0.89-0.97 with 384-512 tiles (two
+    // per CU), 0.88-1.01 from 48000 outputs (28672 from 9 rows) with K from 1024
+    // (151936 x 2560 at 16 rows 160.4 -> 133.7 us), 1.00-1.14 for other widths, and
+    // 1.02-1.29 at any width for rows of a multiple of 8 KB (K = 4096, 8192).
+    if (a.N > 8192 && a.M > 16 && a.M <= 32) {
+      const int64_t tiles = (a.N + 63) / 64;
+      if (tiles <= 256 || tiles > 384) return launch_splitk_cfg<64, 32, 4, 2, false, W8>(a, s);
+    }
+    if (a.N > 8192 && a.M <= 16 && a.K % 4096 != 0) {
+      const int64_t tiles = (a.N + 31) / 32;
+      if ((tiles >= 384 && tiles <= 512) || (a.N >= (a.M > 8 ? 28672 : 48000) && a.K >= 1024))
+        return launch_splitk_cfg<32, 16, 4, 3, false, W8>(a, s);
     }
     if (a.M <= 16) return launch_splitk_cfg<16, 16, 4, 3, false, W8>(a, s);
     if (a.M <= 32) return launch_splitk_cfg<32, 32, 4, 3, false, W8>(a, s);

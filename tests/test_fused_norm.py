@@ -296,7 +296,8 @@ def test_norm_in_rows_or_apart_by_width(M, K, N):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,V", [(1, 256, 40000), (2, 1024, 33000), (3, 2560, 8200), (8, 2560, 8201),
                                    (9, 4096, 8320), (16, 1024, 10000), (17, 256, 9000),
-                                   (33, 256, 8300)])
+                                   (33, 256, 8300), (16, 1024, 12300), (5, 512, 16380), (9, 1024, 28680),
+                                   (12, 4096, 28680), (8, 1024, 48001), (20, 512, 16390), (32, 512, 24580)])
 def test_norm_and_wide_head(M, K, V):
     """The final norm and head of a model: wide outputs at the row counts where
     their tile changes, against the oracle; past 16 rows, with gradients or a
