@@ -120,6 +120,20 @@ def fused_rmsnorm_gate_up_silu_w8(x: torch.Tensor, norm_weight: torch.Tensor, ep
     return y.reshape(*lead, N)
 
 
+def _library_head(rows: int, W: torch.Tensor) -> bool:
+    """Whether ``F.linear`` with the norm before it beats the fused call on W at
+    2 to 16 rows: wide heads whose rows 16-byte loads do not divide (us, fused /
+    torch: 2 rows on 32000 x 2541 80 / 73, 16 on 89491 x 2541 438 / 210; 1000 x 2541 18 /
+    37), and 2 to 4 rows on wide heads of short rows (2 on 151936 x 64 40 / 25, on 32000
+    x 64 15 / 19, on 151936 x 256 43 / 42; 8 on 151936 x 64 23 / 28)."""
+    N, K = W.shape
+    if rows == 1 or N <= 16384:
+        return False
+    if K % 8 or W.stride(0) % 8 or W.data_ptr() % 16:
+        return True
+    return rows <= 4 and K < 256 and N > 32768
+
+
 def fused_rmsnorm_head(h: torch.Tensor, norm, W: torch.Tensor) -> torch.Tensor | None:
     """``F.linear(norm(h), W)``, the final norm and output head of a model, on
     the fused kernels at decode and verify row counts (up to 16 rows of h); None
@@ -127,13 +141,14 @@ def fused_rmsnorm_head(h: torch.Tensor, norm, W: torch.Tensor) -> torch.Tensor |
     types and devices, gradients, torch.func transforms, autocast, a norm that is
     not the plain ``RMSNorm`` or has another weight shape or eps than the kernels
     take, a head whose rows are not contiguous (its copy would cost more than the
-    call). One row of 4B, 151936 x 2560: 109 us against 240 for ``F.linear``
-    alone."""
+    call), a head where the library is faster (:func:`_library_head`). One row of
+    4B, 151936 x 2560: 109 us against 240 for ``F.linear`` alone."""
     if (not h.is_cuda or h.dtype != torch.bfloat16 or W.dtype != torch.bfloat16
             or not 1 <= h.numel() <= 16 * h.shape[-1] or not plain_norm(norm)
             or norm.weight.dtype != torch.bfloat16 or norm.weight.shape != h.shape[-1:]
             or not 0.0 <= norm.eps < float("inf") or W.device != h.device
             or W.dim() != 2 or W.shape[1] != h.shape[-1] or W.stride(1) != 1
-            or autocast() or transformed(h, W, norm.weight)):
+            or autocast() or transformed(h, W, norm.weight)
+            or _library_head(h.numel() // h.shape[-1], W)):
         return None
     return fused_rmsnorm_qkv(h, norm.weight, norm.eps, W, n_q=W.shape[0], n_k=0)[0]

@@ -340,3 +340,20 @@ def test_head_calls_left_to_torch():
                      (norm(K, EPS), w.T.contiguous().T), (norm(K, EPS), w[:, :-8]),
                      (norm(K, EPS), w[0])):
             assert fused_rmsnorm_head(h, n, t) is None
+
+
+def test_head_where_the_library_is_faster():
+    """Wide heads whose rows 16-byte loads do not divide (by length, stride or
+    address) from two rows of h, and very wide ones of short rows at two to four,
+    are left to torch."""
+    from llms_amd.kernels.fused_norm import _library_head
+
+    def left(rows, K, N=20000, off=0, pad=0):
+        w = torch.empty(N * (K + pad) + 64, dtype=torch.bfloat16)
+        off += -(w.data_ptr() // 2) % 8
+        return _library_head(rows, w[off:off + N * (K + pad)].view(N, K + pad)[:, :K])
+
+    assert left(2, 541) and left(16, 541) and not left(1, 541) and not left(2, 541, N=16384)
+    assert not left(2, 544) and left(2, 544, off=1) and left(2, 544, pad=4) and not left(2, 544, pad=8)
+    assert left(4, 64, N=40000) and not left(5, 64, N=40000) and not left(1, 64, N=40000)
+    assert not left(2, 256, N=40000) and not left(2, 64, N=32768)
