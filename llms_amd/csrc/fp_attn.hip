@@ -270,13 +270,13 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(AttnArgs a) {
 
   // q rows of this lane's columns (clamped: rows past the last are not stored)
   u32x4 qf[RT][DK];
-  int lim[RT];  // last visible key
+  int lim[RT];  // last visible key (none past the cache's end)
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
     int rr = row0 + rt * 16 + li;
     if (rr >= rows) rr = rows - 1;
     const int t = rr / G, h = kh * G + (rr - t * G);
-    lim[rt] = p0 + t;
+    lim[rt] = p0 + t < a.S ? p0 + t : a.S - 1;
     const uint16_t* qp = a.qn + (((int64_t)b * a.T + t) * a.Hq + h) * D + 8 * grp;
 #pragma unroll
     for (int i = 0; i < DK; ++i) qf[rt][i] = ld16(qp + 32 * i);
@@ -489,13 +489,14 @@ __global__ __launch_bounds__(256, 2) void attn_tiles_kernel(AttnArgs a, int n_rt
     int rr = row0 + rt * 16 + li;
     if (rr >= rows) rr = rows - 1;
     const int t = rr / G, h = kh * G + (rr - t * G);
-    lim[rt] = p0 + t;
+    lim[rt] = p0 + t < a.S ? p0 + t : a.S - 1;
     const uint16_t* qp = a.qn + (((int64_t)b * a.T + t) * a.Hq + h) * D + 8 * grp;
 #pragma unroll
     for (int i = 0; i < DK; ++i) qf[rt][i] = ld16(qp + 32 * i);
   }
   // the wave's first and last visible key over its rows (uniform)
-  const int lim_lo = p0 + (row0 < rows ? row0 : rows - 1) / G;
+  int lim_lo = p0 + (row0 < rows ? row0 : rows - 1) / G;
+  if (lim_lo >= a.S) lim_lo = a.S - 1;
   const int lim_hi = p0 + (row0 + 16 * RT - 1 < rows ? row0 + 16 * RT - 1 : rows - 1) / G;
 
   const uint16_t* kb = a.ck + b * a.ckb + kh * a.ckh;

@@ -4,10 +4,11 @@ form it stands in for (``kernels/_eager.py``).
 QK-norm, RoPE and the cache rows are the same bf16 roundings of the same
 values: the only freedom is the fp32 sum of squares, whose order may move the
 scale by an ulp of fp32 and so flip a bf16 rounding (an ulp, 2^-8 of the value)
-now and then. The attention output is rounded once from fp32, so against the
-fp64 softmax over the kernel's own cache rows it is within half a bf16 ulp plus
-fp32 evaluation error: |y - t| <= 2^-8 |t| + 1e-5 max|v|, the bound of
-``test_attend_cpu.py``.
+now and then; a flipped q moves a score, and so a row (``_check``). Where q is
+exact (the C entry point without norm weights, RoPE by 0) the output is rounded
+once from fp32, so against the fp64 softmax over the kernel's own cache rows it
+is within half a bf16 ulp plus fp32 evaluation error: |y - t| <= 2^-8 |t| + 1e-5
+max|v|, the bound of ``test_attend_cpu.py``.
 """
 
 from __future__ import annotations
@@ -289,3 +290,91 @@ def test_inference_cache_is_written_in_inference_mode_only():
         assert cache.k[0]._version > version
     with torch.inference_mode():
         assert torch.equal(run(inf), want)
+
+
+def _direct(q, k, v, ck, cv, pos, pos_dev=None, short=0):
+    """fp_attention_bf16 without norm weights and with cos = 1, sin = 0: its
+    status and y [B, T, Hq, D]. short: bytes the workspace lacks."""
+    import ctypes
+
+    from llms_amd import _lib
+    from tests.test_capi import _AttentionArgs
+
+    lib = _lib.capi()
+    (B, T, Hq, D), Hk, S = q.shape, k.shape[2], ck.shape[2]
+    cos, sin = torch.ones(T, D, device=DEV).bfloat16(), torch.zeros(T, D, device=DEV).bfloat16()
+    y = torch.zeros(B, T, Hq, D, device=DEV, dtype=torch.bfloat16)
+    need = lib.fp_attention_workspace_bytes(B, T, Hq, Hk, D, S if pos_dev is not None else pos + T)
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    P = lambda t: t.data_ptr()  # noqa: E731
+    a = _AttentionArgs(q=P(q), k=P(k), v=P(v), ldq=Hq * D, ldk=Hk * D, ldv=Hk * D, cos=P(cos),
+                       sin=P(sin), ld_cos=D, ld_sin=D, cache_k=P(ck), cache_v=P(cv),
+                       k_s_b=ck.stride(0), k_s_h=ck.stride(1), k_s_p=ck.stride(2), v_s_b=cv.stride(0),
+                       v_s_h=cv.stride(1), v_s_p=cv.stride(2), y=P(y), B=B, T=T, n_heads=Hq,
+                       n_kv_heads=Hk, head_dim=D, cache_len=S, pos=pos,
+                       pos_dev=None if pos_dev is None else P(pos_dev))
+    st = lib.fp_attention_bf16(ctypes.byref(a), P(ws), need - short,
+                               torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return st, y
+
+
+def _rows(B, T, Hq, Hk, D, S, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(B + T + D)
+    r = lambda *s: (torch.randn(*s, generator=g, device=DEV) * scale).bfloat16()  # noqa: E731
+    return r(B, T, Hq, D), r(B, T, Hk, D), r(B, T, Hk, D), r(B, Hk, S, D), r(B, Hk, S, D)
+
+
+def _fp64(q, ck, cv, pos):
+    """Causal softmax attention of q [B, T, Hq, D] at pos .. in 64 bits; rows
+    that see no key are NaN."""
+    B, T, Hq, D = q.shape
+    end = max(0, min(pos + T, ck.shape[2]))
+    fk, fv = (t[:, :, :end].double().repeat_interleave(Hq // ck.shape[1], dim=1) for t in (ck, cv))
+    s = torch.matmul(q.transpose(1, 2).double(), fk.transpose(-2, -1).contiguous()) * D ** -0.5
+    hide = torch.arange(end, device=DEV)[None] > torch.arange(pos, pos + T, device=DEV)[:, None]
+    return torch.matmul(torch.softmax(s.masked_fill(hide, float("-inf")), -1), fv).transpose(1, 2)
+
+
+@pytest.mark.parametrize("B,T,Hq,Hk,D,S,pos", [(1, 1, 32, 8, 128, 2048, 2000), (2, 4, 8, 2, 64, 600, 500),
+                                               (1, 200, 8, 2, 128, 500, 300), (1, 700, 16, 8, 64, 700, 0)])
+@pytest.mark.parametrize("scale", [0.25, 1.0, 2.0])
+def test_probabilities_keep_fp32_precision(B, T, Hq, Hk, D, S, pos, scale):
+    """q and the keys enter exactly, so nothing but fp32 evaluation and the one
+    rounding of the output is between y and 64 bits: p.V in fewer than 24 bits of
+    p would show (one bf16 part exceeds the bound: ``test_attend_cpu.py``). Flat to peaked
+    softmax; both kernels, with and without a key split."""
+    q, k, v, ck, cv = _rows(B, T, Hq, Hk, D, S, scale)
+    st, y = _direct(q, k, v, ck, cv, pos)
+    assert st == 0
+    for c, n in ((ck, k), (cv, v)):
+        assert torch.equal(c[:, :, pos:pos + T], n.transpose(1, 2))
+    t = _fp64(q, ck, cv, pos)
+    d = (y.double() - t).abs()
+    print(B, T, D, scale, "max excess", (d - 2.0 ** -8 * t.abs()).max().item())
+    assert bool((d <= 2.0 ** -8 * t.abs() + 1e-5 * cv.double().abs().max()).all())
+
+
+@pytest.mark.parametrize("T", [2, 100])
+def test_workspace_and_device_positions_outside_the_cache(T):
+    """A workspace one byte short is refused. Device positions outside the cache
+    are neither written nor attended; inside, the int position's values."""
+    B, Hq, Hk, D, S = 1, 8, 2, 64, 150
+    q, k, v, ck0, cv0 = _rows(B, T, Hq, Hk, D, S)
+    assert _direct(q, k, v, ck0.clone(), cv0.clone(), 5, short=1)[0] == 6
+    for pos in (40, S - 1, S + 3, -1, -T, 2 ** 40, -2 ** 40):
+        print(T, pos, flush=True)
+        ck, cv = ck0.clone(), cv0.clone()
+        st, y = _direct(q, k, v, ck, cv, 0, pos_dev=torch.tensor(pos, device=DEV))
+        assert st == 0
+        for c, c0, n in ((ck, ck0, k), (cv, cv0, v)):
+            want = c0.clone()
+            lo, hi = max(pos, 0), min(pos + T, S)
+            if lo < hi:
+                want[:, :, lo:hi] = n[:, lo - pos:hi - pos].transpose(1, 2)
+            assert torch.equal(c, want), pos
+        t = _fp64(q, ck, cv, max(min(pos, S + T), -2 * T))
+        seen = pos + torch.arange(T, device=DEV) >= 0
+        d = (y.double() - t).abs()[:, seen]
+        assert bool((d <= 2.0 ** -8 * t[:, seen].abs() + 1e-5 * cv.double().abs().max()).all()), pos
+        assert bool(y[:, ~seen].isnan().all()), pos
