@@ -161,3 +161,21 @@ def test_plain_norm_sees_what_is_attached():
     assert not plain_norm(m)
     del m.forward
     assert plain_norm(m) and not plain_norm(type("Sub", (RMSNorm,), {})(8))
+
+
+@pytest.mark.parametrize("parts,holds", [(1, False), (2, True), (3, True)])
+def test_bound_tells_the_parts_of_p_apart(parts, holds):
+    """The bound that the attention kernels' output is held to, |y - t| <= 2^-8 |t|
+    + 1e-5 max|v|, fails for probabilities rounded to one bf16 and holds for two
+    or three bf16 parts of them."""
+    g = torch.Generator().manual_seed(3)
+    s = torch.randn(64, 500, generator=g, dtype=torch.float64)
+    v = torch.randn(500, 128, generator=g).bfloat16().double()
+    p = torch.softmax(s, -1)
+    t = p @ v
+    left, approx = p.clone(), torch.zeros_like(p)
+    for _ in range(parts):
+        c = left.bfloat16().double()
+        approx, left = approx + c, left - c
+    y = (approx @ v).bfloat16().double()
+    assert bool(((y - t).abs() <= 2.0 ** -8 * t.abs() + 1e-5 * v.abs().max()).all()) == holds
