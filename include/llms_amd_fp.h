@@ -217,8 +217,9 @@ int fp_linear_w8_ws(const void* x, int64_t ldx,
  * and then the contract of the matching projection on xn. Decode-sized calls
  * (the row-streaming regime: bf16 M <= 2, int8 M <= 4, with room for x in
  * LDS) whose x, weights and gamma are 16-byte aligned with row strides that
- * are multiples of 8 (int8 weights: 16) run as one launch that normalises x
- * while staging it and need no workspace. Every other call needs a workspace
+ * are multiples of 8 (int8 weights: 16) need no workspace: they can run as one
+ * launch that normalises x while staging it (with a workspace the norm is a
+ * launch of its own where that is faster). Every other call needs a workspace
  * (the normalised rows, then any split-k partials) and returns
  * FP_ERR_WORKSPACE without one; fp_rmsnorm_workspace_bytes(M, N, K, gate_up,
  * int8) is enough for any pointers and strides of that shape. eps must be

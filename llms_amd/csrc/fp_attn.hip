@@ -450,7 +450,7 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(AttnArgs a) {
 // t, group head h at row t * G + h; wave w rows 16 RT w ..), and walks its
 // keys in tiles of 64 shared by the four waves: K by LDS DMA, V through
 // registers (checked for infinities and NaN on the way), both double-buffered,
-// one barrier per tile. Row tiles with the most keys start first.
+// one barrier per tile. Within a head, row tiles with the most keys start first.
 template <int D, int RT>
 __global__ __launch_bounds__(256, 2) void attn_tiles_kernel(AttnArgs a, int n_rt) {
   constexpr int NW = 4, KT = 64;

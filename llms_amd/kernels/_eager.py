@@ -2,9 +2,10 @@
 
 Plain torch restatements of the Qwen3 attention neighbours of the fused QKV
 projection — RMSNorm with fp32 statistics (``src/engine/attention.py:20-33``)
-and rotate-half RoPE (``src/engine/attention.py:36-76``). They are not on the
-fused path; ``TritonAttention`` applies them after the projection exactly as
-the reference's forward does.
+and rotate-half RoPE (``src/engine/attention.py:36-76``), the cache write and the
+attention itself. ``TritonAttention`` applies them after the projection, as the
+reference's forward does, wherever its HIP kernels (``fused_attention.py``) do
+not take the call.
 """
 
 from __future__ import annotations

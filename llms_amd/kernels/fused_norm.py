@@ -3,10 +3,10 @@
 The reference's decoder block normalises before each projection
 (``self.attn(self.norm1(x), ...)``, ``self.ffn(self.norm2(h))``,
 ``src/engine/model.py:57-66``; RMSNorm ``src/engine/attention.py:28-33``).
-Here the norm runs inside the projection call: for decode-sized calls (the
-row-streaming regime) in the same launch, with x normalised on its way into
-LDS; for larger M as a prologue kernel writing the normalised rows to a torch
-workspace, then the usual kernels. Rounding follows the reference: fp32
+Here the norm runs inside the projection call: at one row (and at two to four
+where few workgroups repeat it) in the projection's own launch, with x
+normalised on its way into LDS; else as a prologue kernel writing the
+normalised rows to a torch workspace, then the usual kernels. Rounding follows the reference: fp32
 statistics, ``bf16(x * rsqrt(mean(x^2) + eps))``, then the bf16 product with
 the norm weight.
 
