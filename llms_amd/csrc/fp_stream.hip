@@ -333,7 +333,7 @@ int launch_stream(const StreamArgs& a, bool aligned, hipStream_t s) {
   // bf16 outputs of more than 8192 columns from 33 rows: whole rounds of the
   // prefill tiles (one box, us, 64 rows, against the 32-row split-K tiles:
   // 151936 x 2560 247.8 -> 180.6, 32000 x 2560 55.0 -> 39.6; 190 drawn shapes of 33-64
-  // rows, 8193-40000 outputs, K = 512-4096: 0.79 of the time at the median, 1.05 at most)
+  // rows, 8193-40000 outputs, K = 512-4096: 0.79 of the time at the median, 1.04 at most)
   if (!W8 && !GATEUP && a.N > kSplitkSmallN && a.M > 32 && gemm_supported(a, aligned, false))
     return launch_gemm<GATEUP, false>(a, s);
   // bf16 from 3 rows, wide gate-up from 4 or 6: split-K tiles (fp_splitk.hip)

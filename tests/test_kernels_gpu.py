@@ -1223,7 +1223,7 @@ def test_rows_of_any_alignment(M, K, N):
            ref.ref_gate_up_silu_full(bits(x), dg, du), "int8 gate-up")
 
 
-@pytest.mark.parametrize("K", [1, 7, 8, 15, 16, 255, 2041, 2042, 4089, 4090, 6137, 6138, 10233, 10234,
+@pytest.mark.parametrize("K", [1, 7, 8, 15, 16, 255, 1023, 1024, 1025, 2041, 2042, 4089, 4090, 6137, 6138, 10233, 10234,
                                16377, 16378])
 def test_quantise_rows_of_any_size_and_alignment(K):
     """Row lengths on both sides of each chunk count per thread, the rows
