@@ -202,9 +202,14 @@ __global__ __launch_bounds__(NW * kWave) void stream_kernel(StreamArgs a) {
       if (c * U + j < nmine) compute_block(f[j]);
   };
 
-  // Prologue: two chunks of weight loads in flight before anything waits.
-  if (nchunks > 0) load_chunk(fa, 0);
-  if (nchunks > 1) load_chunk(fb, 1);
+  // Prologue: two chunks of weight loads in flight before anything waits. (A
+  // lambda: written out here the compiler orders the address arithmetic otherwise,
+  // and calls of 3-4 us take 8-11% longer.)
+  auto prologue = [&]() {
+    if (nchunks > 0) load_chunk(fa, 0);
+    if (nchunks > 1) load_chunk(fb, 1);
+  };
+  prologue();
   // Steady state: while one chunk is consumed the other is in flight; a
   // consumed buffer is refilled with the chunk two ahead.
   for (int64_t c = 0; c < nchunks; c += 2) {
