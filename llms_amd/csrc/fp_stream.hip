@@ -310,6 +310,13 @@ int launch_stream_cfg(const StreamArgs& a, bool aligned, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
+template <int NW, int MT, int U, bool GATEUP, bool W8>
+int launch_stream_aligned(const StreamArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((stream_kernel<NW, MT, U, GATEUP, W8, true>), dim3((unsigned)((a.N + 7) / 8)),
+                     dim3(NW * kWave), 0, s, a);
+  return (int)hipGetLastError();
+}
+
 }  // namespace
 
 // Configurations measured on MI355X (Qwen3-4B shapes, 36 cycled weight sets):
@@ -355,16 +362,25 @@ int launch_stream(const StreamArgs& a, bool aligned, hipStream_t s) {
   // above do not take): the general tiles from 33 rows, and from 9 for unaligned
   // gate-up over at least 8192 weight rows, whose 32-row tiles fill the chip. One
   // box, us, stream / 32 x 32 tiles: gate-up N = 9700, K = 2541 at 16 (int8), 20,
-  // 40 rows 55 / 44, 78 / 38, 121 / 51, N = 4800 at 4, 16 rows 32 / 38, 47 / 39; K =
-  // 2056 (aligned) at 16, 64 rows 27 / 29, 66 / 58; 6100 columns, K = 3001 at 16
-  // rows 36 / 37, 2541 columns at 20, 64 rows 30 / 37, 69 / 37.
-  if (a.M > 32 || (!aligned && GATEUP && a.M > 8 && wrows >= kSplitkSmallN))
+  // 40 rows 55 / 44, 78 / 38, 121 / 51, N = 4800 at 4, 16 rows 32 / 38, 47 / 39; 6100
+  // columns, K = 3001 at 16 rows 36 / 37, 2541 columns at 20, 64 rows 30 / 37, 69 / 37.
+  // Aligned rows of a long K with up to two workgroups of 8 rows per CU stream on to
+  // 64 rows (700 drawn shapes; stream / tiles: int8 171 x 3856 at 33 rows 14.6 / 37.4,
+  // 1030 x 2768 at 40 12.5 / 28.0, gate-up 1827 x 3808 at 45 20.4 / 46.5, bf16 173 x 3856
+  // at 35 14.5 / 27.1; a shorter K, bf16 gate-up 2282 x 976 at 63 rows 17.3 / 10.1).
+  const int64_t stream_k = GATEUP ? (a.N > 2048 ? 1300 : W8 ? 600 : 800)
+                                  : (a.N > 2048 ? 800 : W8 ? 320 : 600);
+  const bool stream_on = aligned && a.N <= 4096 && a.K >= stream_k;
+  if ((a.M > 32 && !stream_on) ||
+      (!aligned && GATEUP && a.M > 8 && wrows >= kSplitkSmallN))
     return launch_tiled<GATEUP, W8>(a, aligned, s);
   // (int8 dequantisation needs registers of its own: 2 k-blocks per buffer)
   constexpr int U8 = (GATEUP && !W8) ? 4 : 2;
   if (a.M <= 8) return launch_stream_cfg<4, 1, U8, GATEUP, W8, true>(a, aligned, s);
   if (a.M <= 16) return launch_stream_cfg<4, 1, 2, GATEUP, W8>(a, aligned, s);
-  return launch_stream_cfg<4, 2, 2, GATEUP, W8>(a, aligned, s);
+  if (a.M <= 32) return launch_stream_cfg<4, 2, 2, GATEUP, W8>(a, aligned, s);
+  if (a.M <= 48) return launch_stream_aligned<4, 3, 2, GATEUP, W8>(a, s);
+  return launch_stream_aligned<4, 4, 1, GATEUP, W8>(a, s);
 }
 
 template int launch_stream<false, false>(const StreamArgs&, bool, hipStream_t);

@@ -1223,6 +1223,32 @@ def test_rows_of_any_alignment(M, K, N):
            ref.ref_gate_up_silu_full(bits(x), dg, du), "int8 gate-up")
 
 
+# (M, K, N): aligned rows of whole 16-element chunks but no whole 64-wide step at 33-64
+# rows: on the streaming kernel (3 and 4 x tiles of 16; both sides of 48 rows, of the
+# shortest K and of 2048 and 4096 outputs) and on the general tiles
+ALIGNED_MID = [(33, 3856, 171), (48, 1040, 2050), (49, 2768, 130), (64, 624, 2048), (64, 816, 4096),
+               (40, 336, 500), (33, 1328, 4090), (63, 592, 70), (50, 1040, 4100), (64, 96, 33)]
+
+
+@pytest.mark.parametrize("M,K,N", ALIGNED_MID)
+def test_aligned_rows_at_33_to_64(M, K, N):
+    """bf16 and int8, linear and gate-up, against the oracle; x as a row-strided
+    view with NaN beside its rows."""
+    kern = _kernels()
+    x, wg, wu = ffn_inputs(1900 + M + K, M, K, N, w_std=0.05)
+    wide = torch.full((M, K + 16), float("nan"), dtype=torch.bfloat16, device=DEV)
+    wide[:, :K] = x.to(DEV)
+    xd, gd, ud = wide[:, :K], wg.to(DEV), wu.to(DEV)
+    _check(kern.fused_linear(xd, gd).cpu(), ref.ref_linear(bits(x), bits(wg)), "linear")
+    _check(kern.triton_fused_gate_up_silu(xd, gd, ud).cpu(),
+           ref.ref_gate_up_silu_full(bits(x), bits(wg), bits(wu)), "gate-up")
+    (qg, sg), (qu, su) = (kern.quantize_w8_per_row(w) for w in (gd, ud))
+    dg, du = (ref.dequant_w8(q.cpu().numpy(), s.cpu().numpy()) for q, s in ((qg, sg), (qu, su)))
+    _check(kern.fused_linear_w8(xd, qg, sg).cpu(), ref.ref_linear(bits(x), dg), "int8 linear")
+    _check(kern.fused_gate_up_silu_w8(xd, qg, sg, qu, su).cpu(),
+           ref.ref_gate_up_silu_full(bits(x), dg, du), "int8 gate-up")
+
+
 @pytest.mark.parametrize("K", [1, 7, 8, 15, 16, 255, 1023, 1024, 1025, 2041, 2042, 4089, 4090, 6137, 6138, 10233, 10234,
                                16377, 16378])
 def test_quantise_rows_of_any_size_and_alignment(K):
