@@ -265,15 +265,20 @@ int launch_tiled(const StreamArgs& a, bool aligned, hipStream_t s) {
   // int8 that reaches here either suits the in-register gemm or had no
   // workspace to dequantise into: gemm_kernel either way
   if (W8 && gemm_supported(a, aligned, true)) return launch_gemm<GATEUP, true>(a, s);
-  // The general tiles: 128 x 128 where they give a workgroup for every CU, then
-  // 64 x 64, then (few rows or narrow outputs) 32 x 32. One box, us, K = 2541 or
-  // 3001, 128 x 128 / 64 x 64 / 32 x 32: gate-up N = 9700 at 300 rows 75 / 121 /
-  // 199, at 100 68 / 62 / 97, at 20 - / 44 / 38; 2541 columns at 1000 rows 59 / 51 /
-  // 85, at 128 75 / 45 / 37; 6000 columns at 200 rows 46 / 31 / 34.
+  // The general tiles: 128 x 128 where they give a workgroup for every CU or the 64 x
+  // 64 tiles would be more than three per CU, then 64 x 64, then (few rows or narrow
+  // outputs) 32 x 32. One box, us, K = 2541 or 3001, 128 x 128 / 64 x 64 / 32 x 32:
+  // gate-up N = 9700 at 300 rows 75 / 121 / 199, at 100 68 / 62 / 97, at 20 - / 44 / 38;
+  // 2541 columns at 1000 rows 59 / 51 / 85, at 128 75 / 45 / 37; 6000 columns at 200
+  // rows 46 / 31 / 34. 600 drawn shapes of 150-270 tiles of 128 x 128, 128 x 128 against 64
+  // x 64: with 769 and more of the latter bf16 0.82-0.87 of the time (2190 rows, 1453
+  // columns, K = 3024 61 / 75 us), int8 gate-up 0.95, int8 linear 1.00-1.06; with fewer
+  // 1.05-1.22.
   const auto count = [&](int64_t t) { return ((wrows + t - 1) / t) * ((a.M + t - 1) / t); };
   if (a.M <= 32 || (count(128) < 256 && count(64) < 192))
     return launch_cfg<32, 32, 64, 1, 2, 4, GATEUP, W8>(a, aligned, s);
-  if (count(128) < 256) return launch_cfg<64, 64, 64, 2, 2, 4, GATEUP, W8>(a, aligned, s);
+  if (count(128) < 256 && (count(64) <= 768 || (W8 && !GATEUP)))
+    return launch_cfg<64, 64, 64, 2, 2, 4, GATEUP, W8>(a, aligned, s);
   return launch_cfg<128, 128, 64, 2, 2, 1, GATEUP, W8>(a, aligned, s);
 }
 
