@@ -243,12 +243,12 @@ int check_common(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldy) {
 }
 
 // B, T, heads and head size of an attention call: sizes that keep every grid
-// dimension and row index within 32 bits.
+// (in threads) and row index within 32 bits.
 int check_attention(int64_t B, int64_t T, int64_t Hq, int64_t Hk, int64_t D) {
   if (B < 1 || T < 1 || Hk < 1 || Hq < Hk || Hq % Hk != 0 || (D != 64 && D != 128))
     return FP_ERR_SHAPE;
   if (B > 65535 || Hq > 65535 || B * Hk > 65535 || T > (int64_t)1 << 24 ||
-      T * (Hq / Hk) > (int64_t)1 << 30 || B * T * (Hq + 2 * Hk) > (int64_t)1 << 31)
+      B * T > (int64_t)1 << 27 || B * T * (Hq + 2 * Hk) > (int64_t)1 << 27)
     return FP_ERR_SHAPE;
   return FP_OK;
 }

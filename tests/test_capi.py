@@ -238,6 +238,18 @@ def test_attention_refuses_overlapping_caches():
         assert _attention_status(**bad) == FP_ERR_STRIDE, bad
 
 
+def test_attention_sizes_beyond_a_grid_are_refused():
+    """Head rows whose launch would pass 2^32 threads (16 per row) get no
+    workspace and FP_ERR_SHAPE, so the module's torch form takes the call."""
+    from llms_amd import _lib
+
+    wb = _lib.capi().fp_attention_workspace_bytes
+    assert wb(1, 1 << 21, 32, 8, 128, 1 << 21) > 0      # 48 x 2^21 head rows
+    assert wb(1, 3 << 20, 32, 8, 128, 3 << 20) == 0     # 48 x 3 x 2^20
+    assert wb(64, 1 << 20, 1, 1, 64, 1 << 20) == 0
+    assert _attention_status(T=1 << 24, cache_len=1 << 25) == FP_ERR_SHAPE
+
+
 def test_python_wrappers_raise_reference_errors():
     """The wrappers' shape checks run before anything else, with the
     reference's messages (tests/test_kernels_fused_ffn.py:203-229,
